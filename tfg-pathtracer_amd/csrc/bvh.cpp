@@ -364,6 +364,17 @@ bool quantizeNode(const WideNode<W>& in, QNode<W>& out) {
 template bool quantizeNode<4>(const WideNode<4>&, QNode<4>&);
 template bool quantizeNode<8>(const WideNode<8>&, QNode<8>&);
 
+void packLaneNode(const QNode<4>& n, uint32_t out[16]) {
+    for (int j = 0; j < 4; j++) {
+        uint32_t* w = out + 4 * j;
+        w[0] = (uint32_t)n.child[j];
+        w[1] = n.plane(0, j) | n.plane(2, j) << 8 | (j < 3 ? ((n.exps >> (8 * j)) & 0xffu) << 23 : 0u);
+        w[2] = n.plane(4, j) | n.plane(1, j) << 8 | n.plane(3, j) << 16 | n.plane(5, j) << 24;
+        w[3] = 0;
+        if (j < 3) std::memcpy(&w[3], &n.p[j], 4);
+    }
+}
+
 WideBvh collapseWide(const Bvh2& b, const float* v, int n, int width) {
     if (width != 4 && width != 8) throw std::runtime_error("BVH width must be 4 or 8");
     WideBvh out;

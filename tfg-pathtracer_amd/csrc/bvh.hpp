@@ -101,6 +101,11 @@ Bvh2 buildBvh2(const float* vertices, int n, int threads = 0);
 // conservative with respect to the Moller-Trumbore acceptance region.
 WideBvh collapseWide(const Bvh2& b, const float* vertices, int n, int width);
 
+// A quantized BVH4 node as the device reads it: four 16-byte words, word j
+// with child j's code and planes and the origin and step of axis j (the word
+// layout is listed with the traversal, pt_device.hpp).
+void packLaneNode(const QNode<4>& n, uint32_t out[16]);
+
 // Quantizes one FP32 wide node (boxes already padded); returns false if a
 // child box is not finite.
 template <int W>

@@ -327,7 +327,19 @@ static int uploadBvh(el_ctx* c, int width) {
         return fail(c, EL_ERR_RANGE, ex.what());
     }
     c->width = width;
-    EL_HIP(c, upload(c->dNodes, c->wide.nodes.data(), c->wide.nodes.size(), c->stream));
+    std::vector<uint32_t> lanes;   // the BVH4 nodes as the quads read them
+    if (width == 4) {
+        lanes.resize(c->wide.nodeCount * 16);
+        parallelFor(c->wide.nodeCount, [&](size_t i0, size_t i1) {
+            for (size_t i = i0; i < i1; i++) {
+                QNode<4> n;
+                std::memcpy(&n, c->wide.nodes.data() + i * sizeof n, sizeof n);
+                packLaneNode(n, &lanes[i * 16]);
+            }
+        });
+    }
+    const void* nodes = width == 4 ? (const void*)lanes.data() : (const void*)c->wide.nodes.data();
+    EL_HIP(c, upload(c->dNodes, nodes, c->wide.nodes.size(), c->stream));
     EL_HIP(c, upload(c->dTris, c->wide.triStream.data(), c->wide.triStream.size() * sizeof(float), c->stream));
     c->gcap = std::max(1, c->wide.stackBound + 2 - dev::kShortStack);
     EL_HIP(c, c->dGstack.ensure((size_t)kSpillSets * c->gcap * c->maxThreads * sizeof(int)));
@@ -335,6 +347,7 @@ static int uploadBvh(el_ctx* c, int width) {
     c->ds.tris = c->dTris.as<float4>();
     c->ds.width = width;
     c->ds.gcap = c->gcap;
+    c->ds.quads = width == 4 && c->wide.stackBound + 2 <= dev::kQuadStack;
     c->stats.bvh_width = (uint32_t)width;
     c->stats.stack_bound = (uint32_t)c->wide.stackBound;
     c->stats.node_bytes = c->wide.nodes.size();
@@ -1454,8 +1467,11 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         b->width = width;
     }
     // scene records: shared spill capacity, per-scene key and accumulation
-    int gcap = 1;
-    for (auto* c : b->scenes) gcap = std::max(gcap, c->gcap);
+    int gcap = 1, quads = 1;
+    for (auto* c : b->scenes) {
+        gcap = std::max(gcap, c->gcap);
+        quads &= c->ds.quads;
+    }
     std::vector<DevScene> recs(S);
     std::vector<uint64_t> work(S), npadv(S);
     uint64_t total = 0;
@@ -1463,6 +1479,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         el_ctx* c = b->scenes[i];
         recs[i] = c->ds;
         recs[i].gcap = gcap;
+        recs[i].quads = quads;
         recs[i].seedLo = (uint32_t)b->seed[i];
         recs[i].seedHi = (uint32_t)(b->seed[i] >> 32);
         recs[i].accum = c->dAccum.as<float4>();

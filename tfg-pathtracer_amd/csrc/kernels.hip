@@ -28,6 +28,7 @@ namespace eleven {
 namespace dev {
 
 constexpr int kMaxWaves = kMaxBlock / 64;
+static_assert(kQuadStack * 16 == kShortStack * 64, "both stacks take the same LDS per wave");
 
 // Minimum waves per SIMD the register allocator must leave room for, per
 // kernel family (1 = no constraint).  Traversal is latency-bound and gains
@@ -77,24 +78,57 @@ __device__ __forceinline__ void blockFlush(unsigned long long* counters, const i
     }
 }
 
-// Chunked work of a traversal launch over n queue items (counter set `kind`):
-// chunks of kChunkRays, smaller (down to 64) when the queue would not give
-// every wave of the grid eight of them.
-template <bool WIDE>
-__device__ __forceinline__ WorkSource chunkSource(uint32_t* qcounters, int kind, uint32_t n) {
-    WorkSource ws;
-    ws.begin = ws.end = 0;
-    ws.ctr = qcounters + kQChunk + kind * kChunkShares * kChunkStride;
+// Whether a launch over n rays of a BVH4 gives each ray to a quad of lanes
+// (traceQuadRange) instead of a lane (traceWaveRange).  A launch that does
+// not fill the GPU lasts as long as one ray's chain of node visits, which is
+// shorter by quads (a visit is ~70 VALU instructions after one 16-byte load
+// instead of ~146 after four; 16 rays share a wave's leaf rounds instead of
+// 64), while one that does is bound by instruction issue, where a lane per
+// ray needs fewer in all.  Whole calls, lanes against quads: 16,384 rays of
+// the 64-sphere field 92 -> 57 us, 262,144 119 -> 86, 2^20 178 -> 198
+// (occlusion on a 131,072-triangle terrain 249 -> 209), 2^21 294 -> 357; the
+// 256 x 256 frame of 16 samples, whose first launch holds 2^20 rays, 1479 ->
+// 1351 us, a 1920 x 1080 one of one sample (2^21) 2.6 -> 3.1 ms.
+constexpr uint32_t kQuadRays = 1u << 20;
+template <int W>
+__device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n) {
+    return W == 4 && s.quads && n <= kQuadRays;
+}
+
+// Chunks of a traversal launch over n items: kChunkRays, smaller (down to the
+// G rays a wave holds at once: one per lane, or one per quad) when n items
+// would not give every wave of the grid eight of them.
+__device__ __forceinline__ WorkSource splitWork(uint32_t n, bool quads) {
+    const uint32_t G = quads ? 16 : 64;
+    WorkSource ws{};
     ws.n = n;
-    const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
-    const uint32_t fit = (uint32_t)(((uint64_t)n / ((uint64_t)waves * 8)) & ~63ull);
-    ws.chunk = fit < 64 ? 64u : (fit > kChunkRays ? kChunkRays : fit);
-    ws.stride = kChunkStride;
+    ws.waves = (gridDim.x * blockDim.x) >> 6;
+    const uint32_t fit = (uint32_t)((uint64_t)n / ((uint64_t)ws.waves * 8)) & ~(G - 1);
+    ws.chunk = fit < G ? G : (fit > kChunkRays ? kChunkRays : fit);
     ws.chunks = (uint32_t)(((uint64_t)n + ws.chunk - 1) / ws.chunk);
+    return ws;
+}
+// Chunks of a wave up to which a launch's waves take theirs in turn (wave w
+// the chunks w, w + waves, ...) instead of drawing them from counters.  8,192
+// waves drawing small chunks from 8 counters wait for each other's atomics;
+// a wave that gets many chunks all over the queue is loaded like the others
+// anyway.  Against drawing every chunk past a wave's first (render time): 1080p
+// terrain of 1 sample 3.18 -> 2.59 ms, of 4 samples 9.4 -> 8.2 (8 chunks: 9.4),
+// 512 x 512 field 3.48 -> 2.70 ms.  All chunks in turn cost the 64-sample
+// frame 92.8 -> 105 ms: its 63 chunks a wave are drawn.
+constexpr uint32_t kStaticChunks = 32;
+
+// The work of a queue of n items, drawn from the counters of `kind` where it
+// has more than kStaticChunks chunks for a wave.
+template <bool WIDE>
+__device__ __forceinline__ WorkSource chunkSource(uint32_t* qcounters, int kind, uint32_t n, bool quads) {
+    WorkSource ws = splitWork(n, quads);
+    if (ws.chunks > (uint64_t)ws.waves * kStaticChunks) ws.waves = 0;
+    ws.ctr = qcounters + kQChunk + kind * kChunkShares * kChunkStride;
+    ws.stride = kChunkStride;
     static_assert(kChunkShares == (int)kWorkShares, "one chunk share per lane");
     ws.parts = WIDE ? kChunkShares : kXcds;
     ws.home = blockIdx.x % ws.parts;
-    ws.fixed = ws.chunks <= waves;
     return ws;
 }
 // Zeroes the chunk counters of `kind` (threads 0..kChunkShares-1 of block 0).
@@ -178,31 +212,31 @@ __device__ __forceinline__ TravStack makeStack(const DevScene& s, int* gstack, u
     return st;
 }
 
-// ------------------------------------------------------------------ trace --
-// Items [begin, end) of the calling wave: n items split evenly over the
-// grid's waves (block sizes are multiples of 64).
-// Items [begin, end) of the calling wave: n items in chunks of a multiple of
-// 64 over the grid's waves (block sizes are multiples of 64), so a small
-// batch fills few waves completely rather than many waves with one lane.
-__device__ __forceinline__ void waveRange(uint32_t n, uint32_t& begin, uint32_t& end) {
-    const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
-    const uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint64_t chunk = (((uint64_t)n + waves - 1) / waves + 63) & ~63ull;
-    const uint64_t b = chunk * w, e = b + chunk;
-    begin = (uint32_t)(b < n ? b : n);
-    end = (uint32_t)(e < n ? e : n);
+// Traces n rays, by quads or by lanes (useQuads).  overflow: a lane's stack was too small.
+template <int W, bool ANY, bool COUNT, bool PER_RAY_BVH, class Load, class Store>
+__device__ __forceinline__ void traceQueue(const DevScene& s, int* gstack, uint32_t gthreads, const WorkSource& ws,
+                                           uint32_t n, uint32_t refill, Load&& load, Store&& store,
+                                           TraceCounters& cnt, uint32_t& traced, uint32_t& overflow) {
+    if (useQuads<W>(s, n)) {
+        extern __shared__ int lds[];
+        QuadStack st{lds + (threadIdx.x >> 6) * (kQuadStack * 16) + ((threadIdx.x >> 2) & 15u), 0};
+        traceQuadRange<ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, traced);
+    } else {
+        TravStack st = makeStack(s, gstack, gthreads);
+        traceWaveRange<W, ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, traced);
+        overflow = st.overflow;
+    }
 }
 
+// ------------------------------------------------------------------ trace --
 template <int W, bool ANY, bool COUNT>
 EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, const float* __restrict__ tmax,
                                     uint32_t n, int32_t* __restrict__ outTri, float* __restrict__ outT,
                                     float* __restrict__ outUV, uint8_t* __restrict__ outOcc, int* gstack,
                                     uint32_t gthreads, uint32_t refill, unsigned long long* counters) {
-    TravStack st = makeStack(s, gstack, gthreads);
     TraceCounters cnt{0, 0};
-    uint32_t traced = 0;
-    WorkSource ws{};
-    waveRange(n, ws.begin, ws.end);
+    uint32_t traced = 0, overflow = 0;
+    const WorkSource ws = splitWork(n, useQuads<W>(s, n));
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr&) {
         const float* r = rays + (uint64_t)i * 6;
@@ -227,9 +261,9 @@ EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, 
             }
         }
     };
-    traceWaveRange<W, ANY, COUNT>(s, st, ws, refill, load, store, cnt, traced);
+    traceQueue<W, ANY, COUNT, false>(s, gstack, gthreads, ws, n, refill, load, store, cnt, traced, overflow);
     const int slots[3] = {kStatNodes, kStatTris, kStatOverflow};
-    const uint32_t vals[3] = {cnt.nodes, cnt.tris, (uint32_t)st.overflow};
+    const uint32_t vals[3] = {cnt.nodes, cnt.tris, overflow};
     blockFlush<3>(counters, slots, vals);
 }
 
@@ -805,7 +839,6 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restric
                                         const uint32_t* countIn, uint32_t* resetNext, uint32_t refill,
                                         unsigned long long* counters) {
     const DevScene& s0 = sc.any();
-    TravStack st = makeStack(s0, q.gstack, q.gthreads);
     TraceCounters cnt{0, 0};
     QueueMap qm;
     qm.load(countIn);
@@ -820,8 +853,8 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restric
     }
     resetChunks(q.counters, chunkShadow(q.parity, 0));
     resetChunks(q.counters, chunkShadow(q.parity, 1));
-    uint32_t rays = 0;
-    const WorkSource ws = chunkSource<P::kMany>(q.counters, kChunkExt, n);
+    uint32_t rays = 0, overflow = 0;
+    const WorkSource ws = chunkSource<P::kMany>(q.counters, kChunkExt, n, useQuads<W>(s0, n));
     const uint32_t segSize = q.segSize;
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr& bvh) {
@@ -843,9 +876,9 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restric
     auto store = [&](uint32_t i, const TraceResult& h, bool) {
         q.hits[qm.entry(i, segSize)] = make_float4(__int_as_float(h.tri), h.t, h.u, h.v);
     };
-    traceWaveRange<W, false, COUNT, P::kMany>(s0, st, ws, refill, load, store, cnt, rays);
+    traceQueue<W, false, COUNT, P::kMany>(s0, q.gstack, q.gthreads, ws, n, refill, load, store, cnt, rays, overflow);
     const int slots[5] = {kStatRays, kStatOverflow, kStatNodes, kStatTris, kStatExtRays};
-    const uint32_t vals[5] = {rays, (uint32_t)st.overflow, cnt.nodes, cnt.tris, rays};
+    const uint32_t vals[5] = {rays, overflow, cnt.nodes, cnt.tris, rays};
     blockFlush<5>(counters, slots, vals);
 }
 
@@ -1054,13 +1087,13 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_shadow(P sc, WfState q, const float4* __restric
                                         const uint32_t* countIn, uint32_t refill,
                                         unsigned long long* counters) {
     const DevScene& s0 = sc.any();
-    TravStack st = makeStack(s0, q.gstack, q.gthreads);
     TraceCounters cnt{0, 0};
     QueueMap qm;
     qm.load(countIn);
     const uint32_t n = qm.total();
-    uint32_t traced = 0;
-    const WorkSource ws = chunkSource<P::kMany>(q.counters, chunkShadow(q.parity, sh == q.shadowH ? 0 : 1), n);
+    uint32_t traced = 0, overflow = 0;
+    const WorkSource ws =
+        chunkSource<P::kMany>(q.counters, chunkShadow(q.parity, sh == q.shadowH ? 0 : 1), n, useQuads<W>(s0, n));
     const uint32_t segSize = q.segSize;
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr& bvh) {
@@ -1099,9 +1132,9 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_shadow(P sc, WfState q, const float4* __restric
         const float4 L = q.pathL[slot];
         q.pathL[slot] = make_float4(L.x + C.x, L.y + C.y, L.z + C.z, L.w);
     };
-    traceWaveRange<W, true, false, P::kMany>(s0, st, ws, refill, load, store, cnt, traced);
+    traceQueue<W, true, false, P::kMany>(s0, q.gstack, q.gthreads, ws, n, refill, load, store, cnt, traced, overflow);
     const int slots[1] = {kStatOverflow};
-    const uint32_t vals[1] = {(uint32_t)st.overflow};
+    const uint32_t vals[1] = {overflow};
     blockFlush<1>(counters, slots, vals);
 }
 
@@ -1287,10 +1320,15 @@ static uint32_t gridFor(uint64_t n, uint32_t block, uint32_t maxBlocks) {
     return (uint32_t)(g < maxBlocks ? g : maxBlocks);
 }
 
+// Grid of a queue traversal over at most n rays of a tree of this width.
+static uint32_t queueGrid(const LaunchCfg& c, int width, uint64_t n) {
+    return gridFor(n * (width == 4 ? 4 : 1), c.block, c.maxThreads / c.block);
+}
+
 hipError_t launchTrace(const LaunchCfg& c, const DevScene& s, const float* rays, const float* tmax, uint32_t n,
                        int32_t* tri, float* t, float* uv, uint8_t* occ, bool any, bool count,
                        unsigned long long* counters) {
-    uint32_t grid = gridFor(n, c.block, c.maxThreads / c.block);
+    uint32_t grid = queueGrid(c, s.width, n);
     size_t lds = sizeof(int) * kShortStack * c.block;
 #define EL_TRACE(WW, A, C)                                                                                   \
     hipLaunchKernelGGL((k_trace<WW, A, C>), dim3(grid), dim3(c.block), lds, c.stream, s, rays, tmax, n, tri, t, \
@@ -1368,7 +1406,7 @@ hipError_t launchWfCamera(const LaunchCfg& c, const DevScene& s, const RenderArg
 hipError_t launchWfExtend(const LaunchCfg& c, const DevScene& s, const WfState& q, const float4* rayIn,
                           const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount, bool countTraversal,
                           unsigned long long* counters) {
-    uint32_t grid = gridFor(maxCount, c.block, c.maxThreads / c.block);
+    uint32_t grid = queueGrid(c, s.width, maxCount);
     size_t lds = sizeof(int) * kShortStack * c.block;
 #define EL_EXT(WW, C)                                                                                       \
     hipLaunchKernelGGL((k_wf_extend<WW, C, OneScene>), dim3(grid), dim3(c.block), lds, c.stream, OneScene{s}, q, \
@@ -1399,7 +1437,7 @@ hipError_t launchWfShade(const LaunchCfg& c, const DevScene& s, const RenderArgs
 
 hipError_t launchWfShadow(const LaunchCfg& c, const DevScene& s, const WfState& q, const float4* shadow,
                           const uint32_t* countIn, uint32_t maxCount, unsigned long long* counters) {
-    uint32_t grid = gridFor(maxCount, c.block, c.maxThreads / c.block);
+    uint32_t grid = queueGrid(c, s.width, maxCount);
     size_t lds = sizeof(int) * kShortStack * c.block;
     const bool rec = q.visBit != 0;
     if (s.width == 4 && rec)
@@ -1438,7 +1476,7 @@ hipError_t launchBtCamera(const LaunchCfg& c, const DevScene* scenes, const Batc
 hipError_t launchBtExtend(const LaunchCfg& c, const DevScene* scenes, int width, const WfState& q,
                           const float4* rayIn, const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount,
                           unsigned long long* counters) {
-    uint32_t grid = gridFor(maxCount, c.block, c.maxThreads / c.block);
+    uint32_t grid = queueGrid(c, width, maxCount);
     size_t lds = sizeof(int) * kShortStack * c.block;
     if (width == 4)
         hipLaunchKernelGGL((k_wf_extend<4, false, ManyScenes>), dim3(grid), dim3(c.block), lds, c.stream,
@@ -1461,7 +1499,7 @@ hipError_t launchBtShade(const LaunchCfg& c, const DevScene* scenes, const Rende
 hipError_t launchBtShadow(const LaunchCfg& c, const DevScene* scenes, int width, const WfState& q,
                           const float4* shadow, const uint32_t* countIn, uint32_t maxCount,
                           unsigned long long* counters) {
-    uint32_t grid = gridFor(maxCount, c.block, c.maxThreads / c.block);
+    uint32_t grid = queueGrid(c, width, maxCount);
     size_t lds = sizeof(int) * kShortStack * c.block;
     if (width == 4)
         hipLaunchKernelGGL((k_wf_shadow<4, ManyScenes>), dim3(grid), dim3(c.block), lds, c.stream,

@@ -34,9 +34,6 @@ namespace dev {
 #ifndef EL_LEAF_PIPE   // leaf triangles: next record loaded before the current one is tested
 #define EL_LEAF_PIPE 1
 #endif
-#ifndef EL_SLAB_AB     // slab distances as A + q B per axis (2 VALU per plane) instead of (b - o) / d
-#define EL_SLAB_AB 1
-#endif
 #ifndef EL_PUSH_BULK   // one stack-room check per node visit instead of one per push
 #define EL_PUSH_BULK 1
 #endif
@@ -178,7 +175,8 @@ struct DevScene {
     int32_t nLights;
     int32_t nTris;
     int32_t width;                 // BVH width (4 or 8)
-    int32_t gcap;                  // global stack entries per thread
+    int32_t gcap;                  // global stack entries per thread (a stack per lane)
+    int32_t quads;                 // BVH4 within kQuadStack: short queues give a ray to a quad of lanes
     DevCamera cam;
     // batches only: the scene's RNG key and accumulation buffers
     uint32_t seedLo, seedHi;
@@ -746,9 +744,18 @@ struct TravStack {
     }
 };
 
-// Quantized wide node as stored (eleven::QNode<W>, bvh.hpp): 16-byte words
-// per node, W = 4: 4 (header, q0-3, q4-5 + child0-1, child2-3 + pad);
-// W = 8: 6 (header, q0-11 in three words, child0-7 in two).
+// Quantized wide node as uploaded, in 16-byte words.
+//   W = 8: eleven::QNode<8> as it is, 6 words (header, q0-11 in three words,
+//          child0-7 in two).
+//   W = 4: 4 words, one per child (packLaneNode, bvh.hpp): word j holds child
+//          j's code, its six plane bytes, and the grid origin and step of
+//          axis j (j < 3), so that the four lanes of a quad that share a ray
+//          read a node with one load, 16 bytes each, and each lane has its
+//          own child and its own axis:
+//            x  child code
+//            y  lo x | lo y << 8 | exponent of axis j << 23 (the step's FP32 bits)
+//            z  lo z | hi x << 8 | hi y << 16 | hi z << 24
+//            w  grid origin of axis j (FP32 bits)
 template <int W>
 struct QNodeWords {
     static constexpr int kWords = W == 4 ? 4 : 6;
@@ -763,24 +770,33 @@ struct TraceCounters {
     uint32_t nodes, tris;
 };
 
+// Byte selectors (v_perm_b32 over z : y of a BVH4 node word) that gather a
+// child's near and far plane bytes (x, y, z) for a ray direction's signs.
+struct PlaneSel {
+    uint32_t nearSel, farSel;
+};
+__device__ __forceinline__ PlaneSel planeSel(float ix, float iy, float iz) {
+    PlaneSel s;
+    // y bytes 0, 1: lo x, lo y (selectors 0, 1); z bytes 0..3: lo z, hi x, hi y, hi z (4..7); 0x0c: zero
+    s.nearSel = 0x0c000000u | (ix < 0 ? 5u : 0u) | (iy < 0 ? 6u << 8 : 1u << 8) | (iz < 0 ? 7u << 16 : 4u << 16);
+    s.farSel = 0x0c000000u | (ix < 0 ? 0u : 5u) | (iy < 0 ? 1u << 8 : 6u << 8) | (iz < 0 ? 4u << 16 : 7u << 16);
+    return s;
+}
+// Reciprocal of a direction component for the slab tests (finite).
+__device__ __forceinline__ float slabInv(float d) {
+    const float tiny = 1e-30f;
+    return 1.0f / (fabsf(d) > tiny ? d : copysignf(tiny, d));
+}
+// Widening of a slab distance A + q B: near planes use A - |A| kSlabEps, far planes A + |A| kSlabEps (see visitWords).
+constexpr float kSlabEps = 1.0f / 524288.0f, kFarEps = 1.0f / 1048576.0f;
+
 // A ray prepared for slab tests: origin, direction and safe reciprocal.
 struct TRay {
     float ox, oy, oz, dx, dy, dz, ix, iy, iz;
 };
 
 __device__ __forceinline__ TRay makeTRay(float ox, float oy, float oz, float dx, float dy, float dz) {
-    const float tiny = 1e-30f;
-    TRay r;
-    r.ox = ox;
-    r.oy = oy;
-    r.oz = oz;
-    r.dx = dx;
-    r.dy = dy;
-    r.dz = dz;
-    r.ix = 1.0f / (fabsf(dx) > tiny ? dx : copysignf(tiny, dx));
-    r.iy = 1.0f / (fabsf(dy) > tiny ? dy : copysignf(tiny, dy));
-    r.iz = 1.0f / (fabsf(dz) > tiny ? dz : copysignf(tiny, dz));
-    return r;
+    return TRay{ox, oy, oz, dx, dy, dz, slabInv(dx), slabInv(dy), slabInv(dz)};
 }
 
 // Visits inner node `cur`: slab-tests its W children against [0, tcull],
@@ -791,96 +807,80 @@ __device__ __forceinline__ TRay makeTRay(float ox, float oy, float oz, float dx,
 // >= 0 inner node, <= -2 leaf, -1 empty slot (its box is inverted, so it is
 // never hit).
 //
-// Planes decode exactly (p + q * step is an FP32 value by construction), so
-// the computed slab distances (b - o) * (1/d) carry only relative rounding
-// error (< 2^-21 with the reciprocal's); widening tfar by 2^-20 of its
-// magnitude makes the test conservative: no box the ray touches is culled.
+// Planes decode exactly (p + q * step is an FP32 value by construction).
 // visitWords tests a node whose words are already loaded (the root, kept in
 // scalar registers by the wavefront traversal); visitNode loads them.
+//
+// Plane b = p + q s, so (b - o) / d = A + q B per axis with A = (p - o) inv
+// and B = s inv (exact: s is a power of two), and fma(q, B, A) rounds once; A
+// carries two roundings, so a distance is off by at most 2^-23 |A| + 2^-24
+// |t|.  Near planes use A - E and far planes A + E with E = 2^-19 |A| of their
+// own axis (an axis whose direction is near zero has a huge A, but also huge
+// distances of its own), and the 2^-20 |tf| widening covers the |t| term: the
+// test stays conservative.  An empty slot (child -1) has an inverted box, 255
+// grid steps from near to far plane; where 255 steps are below the rounding
+// of A (a node smaller than ~4e-6 of its distance from the origin on every
+// axis) the box passes the widened test, so the slot's code is checked as
+// well: entering it would end the traversal (-1 is the empty stack's code).
 template <int W, bool UNSORTED = false>
 __device__ __forceinline__ int visitWords(const uint4* np, const TRay& ray, float tcull, TravStack& st) {
-    constexpr int D = W / 4;   // dwords of bytes per (axis, side)
-    const uint4 h = np[0];
-    uint32_t q[6 * D];
-    int32_t child[W];
-    if constexpr (W == 4) {
-        const uint4 a = np[1], b = np[2], c = np[3];
-        q[0] = a.x, q[1] = a.y, q[2] = a.z, q[3] = a.w, q[4] = b.x, q[5] = b.y;
-        child[0] = (int32_t)b.z, child[1] = (int32_t)b.w, child[2] = (int32_t)c.x, child[3] = (int32_t)c.y;
-    } else {
-        const uint4 a = np[1], b = np[2], c = np[3], d = np[4], e = np[5];
-        q[0] = a.x, q[1] = a.y, q[2] = a.z, q[3] = a.w, q[4] = b.x, q[5] = b.y;
-        q[6] = b.z, q[7] = b.w, q[8] = c.x, q[9] = c.y, q[10] = c.z, q[11] = c.w;
-        child[0] = (int32_t)d.x, child[1] = (int32_t)d.y, child[2] = (int32_t)d.z, child[3] = (int32_t)d.w;
-        child[4] = (int32_t)e.x, child[5] = (int32_t)e.y, child[6] = (int32_t)e.z, child[7] = (int32_t)e.w;
-    }
-    const float px = __uint_as_float(h.x), py = __uint_as_float(h.y), pz = __uint_as_float(h.z);
-    const float sx = __uint_as_float((h.w & 0xffu) << 23);
-    const float sy = __uint_as_float(((h.w >> 8) & 0xffu) << 23);
-    const float sz = __uint_as_float(((h.w >> 16) & 0xffu) << 23);
-    // near / far plane bytes per axis by the direction's sign (q index: axis*2*D + side*D + dword)
-    const bool nx = ray.ix < 0, ny = ray.iy < 0, nz = ray.iz < 0;
-    uint32_t nearX[D], farX[D], nearY[D], farY[D], nearZ[D], farZ[D];
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-        nearX[d] = nx ? q[1 * D + d] : q[0 * D + d];
-        farX[d] = nx ? q[0 * D + d] : q[1 * D + d];
-        nearY[d] = ny ? q[3 * D + d] : q[2 * D + d];
-        farY[d] = ny ? q[2 * D + d] : q[3 * D + d];
-        nearZ[d] = nz ? q[5 * D + d] : q[4 * D + d];
-        farZ[d] = nz ? q[4 * D + d] : q[5 * D + d];
-    }
     uint32_t keys[W];
-#if EL_SLAB_AB
-    // Plane b = p + q s, so (b - o) / d = A + q B per axis with
-    // A = (p - o) inv and B = s inv (exact: s is a power of two), and
-    // fma(q, B, A) rounds once; A carries two roundings, so a distance is off
-    // by at most 2^-23 |A| + 2^-24 |t|.  Near planes use A - E and far planes
-    // A + E with E = 2^-19 |A| of their own axis (an axis whose direction is
-    // near zero has a huge A, but also huge distances of its own), and the
-    // 2^-20 |tf| widening below covers the |t| term: the test stays
-    // conservative.  An empty slot (child -1) has an inverted box, 255 grid
-    // steps from near to far plane; where 255 steps are below the rounding
-    // of A (a node smaller than ~4e-6 of its distance from the origin on
-    // every axis) the box passes the widened test, so the slot's code is
-    // checked as well: entering it would end the traversal (-1 is the empty
-    // stack's code).
+    int32_t child[W];
+    float px, py, pz, sx, sy, sz;
+    if constexpr (W == 4) {
+        px = __uint_as_float(np[0].w), py = __uint_as_float(np[1].w), pz = __uint_as_float(np[2].w);
+        sx = __uint_as_float(np[0].y & 0x7f800000u), sy = __uint_as_float(np[1].y & 0x7f800000u);
+        sz = __uint_as_float(np[2].y & 0x7f800000u);
+    } else {
+        const uint4 h = np[0];
+        px = __uint_as_float(h.x), py = __uint_as_float(h.y), pz = __uint_as_float(h.z);
+        sx = __uint_as_float((h.w & 0xffu) << 23);
+        sy = __uint_as_float(((h.w >> 8) & 0xffu) << 23);
+        sz = __uint_as_float(((h.w >> 16) & 0xffu) << 23);
+    }
     const float Ax = (px - ray.ox) * ray.ix, Ay = (py - ray.oy) * ray.iy, Az = (pz - ray.oz) * ray.iz;
     const float Bx = sx * ray.ix, By = sy * ray.iy, Bz = sz * ray.iz;
-    const float Ex = fabsf(Ax) * (1.0f / 524288.0f), Ey = fabsf(Ay) * (1.0f / 524288.0f),
-                Ez = fabsf(Az) * (1.0f / 524288.0f);
+    const float Ex = fabsf(Ax) * kSlabEps, Ey = fabsf(Ay) * kSlabEps, Ez = fabsf(Az) * kSlabEps;
     const float Anx = Ax - Ex, Afx = Ax + Ex, Any = Ay - Ey, Afy = Ay + Ey, Anz = Az - Ez, Afz = Az + Ez;
-#pragma unroll
-    for (int i = 0; i < W; i++) {
-        const int d = i >> 2, sh = 8 * (i & 3);
-        const float tx0 = fmaf((float)((nearX[d] >> sh) & 0xffu), Bx, Anx);
-        const float tx1 = fmaf((float)((farX[d] >> sh) & 0xffu), Bx, Afx);
-        const float ty0 = fmaf((float)((nearY[d] >> sh) & 0xffu), By, Any);
-        const float ty1 = fmaf((float)((farY[d] >> sh) & 0xffu), By, Afy);
-        const float tz0 = fmaf((float)((nearZ[d] >> sh) & 0xffu), Bz, Anz);
-        const float tz1 = fmaf((float)((farZ[d] >> sh) & 0xffu), Bz, Afz);
+    auto key = [&](int i, uint32_t qnx, uint32_t qny, uint32_t qnz, uint32_t qfx, uint32_t qfy, uint32_t qfz) {
+        const float tx0 = fmaf((float)qnx, Bx, Anx), tx1 = fmaf((float)qfx, Bx, Afx);
+        const float ty0 = fmaf((float)qny, By, Any), ty1 = fmaf((float)qfy, By, Afy);
+        const float tz0 = fmaf((float)qnz, Bz, Anz), tz1 = fmaf((float)qfz, Bz, Afz);
         const float tn = fmaxf(fmaxf(tx0, ty0), fmaxf(tz0, 0.0f));
         float tf = fminf(fminf(tx1, ty1), fminf(tz1, tcull));
-        tf = fmaf(fabsf(tf), 1.0f / 1048576.0f, tf);
+        tf = fmaf(fabsf(tf), kFarEps, tf);
         keys[i] = (tn <= tf && child[i] != -1) ? ((__float_as_uint(tn) & ~7u) | (uint32_t)i) : 0xFFFFFFFFu;
-    }
-#else
+    };
+    if constexpr (W == 4) {
+        const PlaneSel sel = planeSel(ray.ix, ray.iy, ray.iz);
 #pragma unroll
-    for (int i = 0; i < W; i++) {
-        const int d = i >> 2, sh = 8 * (i & 3);
-        const float bx0 = fmaf((float)((nearX[d] >> sh) & 0xffu), sx, px);
-        const float bx1 = fmaf((float)((farX[d] >> sh) & 0xffu), sx, px);
-        const float by0 = fmaf((float)((nearY[d] >> sh) & 0xffu), sy, py);
-        const float by1 = fmaf((float)((farY[d] >> sh) & 0xffu), sy, py);
-        const float bz0 = fmaf((float)((nearZ[d] >> sh) & 0xffu), sz, pz);
-        const float bz1 = fmaf((float)((farZ[d] >> sh) & 0xffu), sz, pz);
-        const float tn = fmaxf(fmaxf((bx0 - ray.ox) * ray.ix, (by0 - ray.oy) * ray.iy),
-                               fmaxf((bz0 - ray.oz) * ray.iz, 0.0f));
-        float tf = fminf(fminf((bx1 - ray.ox) * ray.ix, (by1 - ray.oy) * ray.iy), fminf((bz1 - ray.oz) * ray.iz, tcull));
-        tf = fmaf(fabsf(tf), 1.0f / 1048576.0f, tf);
-        keys[i] = (tn <= tf && child[i] != -1) ? ((__float_as_uint(tn) & ~7u) | (uint32_t)i) : 0xFFFFFFFFu;
+        for (int i = 0; i < 4; i++) {
+            const uint4 w = np[i];
+            child[i] = (int32_t)w.x;
+            const uint32_t n = __builtin_amdgcn_perm(w.z, w.y, sel.nearSel), f = __builtin_amdgcn_perm(w.z, w.y, sel.farSel);
+            key(i, n & 0xffu, (n >> 8) & 0xffu, (n >> 16) & 0xffu, f & 0xffu, (f >> 8) & 0xffu, (f >> 16) & 0xffu);
+        }
+    } else {
+        const uint4 a = np[1], b = np[2], c = np[3], d = np[4], e = np[5];
+        const uint32_t q[12] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w};
+        child[0] = (int32_t)d.x, child[1] = (int32_t)d.y, child[2] = (int32_t)d.z, child[3] = (int32_t)d.w;
+        child[W - 4] = (int32_t)e.x, child[W - 3] = (int32_t)e.y, child[W - 2] = (int32_t)e.z, child[W - 1] = (int32_t)e.w;
+        // near / far plane bytes per axis by the direction's sign (q index: axis * 4 + side * 2 + dword)
+        const bool nx = ray.ix < 0, ny = ray.iy < 0, nz = ray.iz < 0;
+        uint32_t nf[6][2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            nf[0][k] = nx ? q[2 + k] : q[k], nf[3][k] = nx ? q[k] : q[2 + k];
+            nf[1][k] = ny ? q[6 + k] : q[4 + k], nf[4][k] = ny ? q[4 + k] : q[6 + k];
+            nf[2][k] = nz ? q[10 + k] : q[8 + k], nf[5][k] = nz ? q[8 + k] : q[10 + k];
+        }
+#pragma unroll
+        for (int i = 0; i < W; i++) {
+            const int k = i >> 2, sh = 8 * (i & 3);
+            key(i, (nf[0][k] >> sh) & 0xffu, (nf[1][k] >> sh) & 0xffu, (nf[2][k] >> sh) & 0xffu,
+                (nf[3][k] >> sh) & 0xffu, (nf[4][k] >> sh) & 0xffu, (nf[5][k] >> sh) & 0xffu);
+        }
     }
-#endif
     if constexpr (UNSORTED) {
         int next = -2;   // the lowest hit slot is visited next, the others are pushed
 #if EL_PUSH_BULK
@@ -949,8 +949,8 @@ __device__ __forceinline__ int visitNode(const uint4* __restrict__ nodes, int cu
 // Tests one triangle record and updates the closest hit: smaller t wins,
 // equal t goes to the lower original index.  For ANY the first hit below
 // r.t is taken and true is returned (the query ends).
-template <bool ANY>
-__device__ __forceinline__ bool hitTriangle(const float4& A, const float4& B, const float4& C, const TRay& ray,
+template <bool ANY, class Ray>
+__device__ __forceinline__ bool hitTriangle(const float4& A, const float4& B, const float4& C, const Ray& ray,
                                             TraceResult& r) {
     float t, u, v;
     if (mtHit(A, B, C, ray.ox, ray.oy, ray.oz, ray.dx, ray.dy, ray.dz, t, u, v)) {
@@ -1063,27 +1063,83 @@ struct BvhPtr {
     const float4* tris;
 };
 
-// The items a wave traces: a fixed range [begin, end), or (ctr set) chunks
-// of `chunk` items handed out at run time.  Chunk c belongs to share
-// c % parts; share x is counted by ctr[x * stride].  A wave draws from its
-// home share first, then from the others, so waves that meet cheap rays take
-// more chunks and a launch ends when the work does, not when its slowest
-// fixed range does.  One scene uses 8 shares (one per XCD: the waves of an
-// XCD draw neighbouring chunks, which keeps their rays coherent in its L2),
-// a batch 64 (measured faster there).  Every counter starts the launch at 0.  A share is skipped without an atomic once a coherent read shows it
-// drawn out (a read never runs ahead of the counter, so no chunk is lost).
-// A queue with no more chunks than the grid has waves (the late bounces, small
-// frames) is handed out without counters: wave w takes chunk w -- the chunk
-// the dynamic scheme's share order would also give its XCD -- and waves past
-// the last chunk return at once.  Thousands of waves contending for eight
-// counters cost such a launch ~100 us whatever its size.
+// The items a wave traces: chunks of `chunk` items, either in turn (wave w of
+// `waves` takes the chunks w, w + waves, ...; without counters) or, with
+// waves == 0, handed out at run time.  Then chunk c belongs to share c % parts;
+// share x is counted by ctr[x * stride].  A wave draws from its home share
+// first, then from the others, so waves that meet cheap rays take more chunks
+// and a launch ends when the work does, not when its slowest wave's share
+// does.  One scene uses 8 shares (one per XCD: the waves of an XCD draw
+// neighbouring chunks, which keeps their rays coherent in its L2), a batch 64
+// (measured faster there).  Every counter starts the launch at 0.  A share is
+// skipped without an atomic once a coherent read shows it drawn out (a read
+// never runs ahead of the counter, so no chunk is lost).
 constexpr uint32_t kWorkShares = 64;   // shares of a wide WorkSource (one per lane of a wave)
 struct WorkSource {
-    uint32_t begin, end;
     uint32_t* ctr;
     uint32_t n, chunk, stride, parts, home;
     uint32_t chunks;   // ceil(n / chunk)
-    bool fixed;        // chunks <= waves of the grid: wave w takes chunk w, no counter atomics
+    uint32_t waves;    // 0: drawn from the counters
+};
+
+// A wave's place in its items (wave-uniform).
+struct WorkCursor {
+    uint32_t cursor, end, waveId;
+    uint32_t tried = 0;      // narrow source: shares found drawn out
+    __device__ __forceinline__ WorkCursor(const WorkSource& ws, uint32_t wave)
+        : cursor(0), end(0), waveId(wave) {}
+    // The next chunk after [cursor, end) is used up; false: no items left.
+    // The whole wave must call.
+    template <bool WIDE>
+    __device__ __forceinline__ bool draw(const WorkSource& ws) {
+        if (ws.waves) {   // chunks waveId, waveId + waves, ...
+            const uint32_t c = waveId;
+            waveId += ws.waves;
+            return take(ws, c);
+        }
+        const uint32_t lane = __lane_id();
+        // Wide sources (batches, parts == 64): lane l looks at share
+        // (home + l) % 64 at once (one load per lane instead of 64
+        // dependent loads), and the wave draws from the first share with
+        // chunks left.  Share x holds the chunks x, x + 64, ...:
+        // (chunks - x + 63) / 64 of them.
+        while (WIDE) {
+            const uint32_t x = (ws.home + lane) & (kWorkShares - 1);
+            const uint32_t seen =
+                __hip_atomic_load(ws.ctr + x * ws.stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const bool left = x < ws.chunks && seen < ((ws.chunks - x + kWorkShares - 1) >> 6);
+            const unsigned long long have = __ballot(left);
+            if (!have) return false;
+            const uint32_t pick = (ws.home + (uint32_t)(__ffsll((long long)have) - 1)) & (kWorkShares - 1);
+            uint32_t k = 0;
+            if (lane == 0) k = atomicAdd(ws.ctr + pick * ws.stride, 1u);
+            k = __builtin_amdgcn_readfirstlane(k);
+            if (take(ws, (uint64_t)pick + (uint64_t)kWorkShares * k)) return true;
+        }
+        // Narrow sources (one scene, parts == 8): one share at a time, from
+        // the wave's home share on; a share found drawn out is not looked at
+        // again.
+        while (!WIDE && tried < ws.parts) {
+            const uint32_t x = (ws.home + tried) % ws.parts;
+            uint32_t* const c = ws.ctr + x * ws.stride;
+            const uint32_t seen = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (((uint64_t)x + (uint64_t)ws.parts * seen) * ws.chunk < ws.n) {
+                uint32_t k = 0;
+                if (lane == (uint32_t)(__ffsll((long long)__ballot(true)) - 1)) k = atomicAdd(c, 1u);
+                k = __builtin_amdgcn_readfirstlane(k);
+                if (take(ws, (uint64_t)x + (uint64_t)ws.parts * k)) return true;
+            }
+            tried++;
+        }
+        return false;
+    }
+    __device__ __forceinline__ bool take(const WorkSource& ws, uint64_t chunk) {
+        const uint64_t first = chunk * ws.chunk;
+        if (first >= ws.n) return false;
+        cursor = __builtin_amdgcn_readfirstlane((uint32_t)first);
+        end = __builtin_amdgcn_readfirstlane((uint32_t)(first + ws.chunk < ws.n ? first + ws.chunk : ws.n));
+        return true;
+    }
 };
 
 template <int W, bool ANY, bool COUNT, bool PER_RAY_BVH = false, class Load, class Store>
@@ -1091,8 +1147,7 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
                                                uint32_t refill, Load&& load, Store&& store, TraceCounters& cnt,
                                                uint32_t& traced) {
     const uint32_t waveId = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (ws.ctr && ws.fixed && waveId >= ws.chunks) return;   // no chunk for this wave
-    bool fixedDrawn = false;
+    if (ws.waves && waveId >= ws.chunks) return;   // no chunk for this wave
     BvhPtr bvh{(const uint4*)s.nodes, s.tris};
     // One BVH for the whole wave: its root node (visited first by every ray)
     // is read once into scalar registers, and a new ray is tested against it
@@ -1110,9 +1165,8 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
     }
     const uint32_t lane = __lane_id();
     const unsigned long long ltMask = lane ? (~0ull >> (64 - lane)) : 0ull;
-    uint32_t cursor = ws.begin, end = ws.end;   // wave-uniform
-    uint32_t tried = 0;                         // narrow source: shares found drawn out
-    bool more = true;                           // wave-uniform: items may remain
+    WorkCursor wc(ws, waveId);
+    bool more = true;   // wave-uniform: items may remain
     bool live = false;
     uint32_t item = 0;
     TRay ray{};
@@ -1123,68 +1177,11 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
         const unsigned long long idle = __ballot(!live);
         const uint32_t nIdle = (uint32_t)__popcll(idle);
         const bool want = nIdle >= refill || nIdle == 64;
-        if (want && cursor >= end) {
-            more = false;
-            if (ws.ctr && ws.fixed) {   // the wave's one chunk
-                if (!fixedDrawn) {
-                    fixedDrawn = true;
-                    cursor = waveId * ws.chunk;
-                    end = cursor + ws.chunk < ws.n ? cursor + ws.chunk : ws.n;
-                    more = cursor < end;
-                }
-            }
-            // Wide sources (batches, parts == 64): lane l looks at share
-            // (home + l) % 64 at once (one load per lane instead of 64
-            // dependent loads; the whole wave runs here), and the wave draws
-            // from the first share with chunks left.  Share x holds the
-            // chunks x, x + 64, ...: (chunks - x + 63) / 64 of them.
-            while (PER_RAY_BVH && ws.ctr && !ws.fixed) {
-                const uint32_t x = (ws.home + lane) & (kWorkShares - 1);
-                const uint32_t seen =
-                    __hip_atomic_load(ws.ctr + x * ws.stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const bool left = x < ws.chunks && seen < ((ws.chunks - x + kWorkShares - 1) >> 6);
-                const unsigned long long have = __ballot(left);
-                if (!have) break;
-                const uint32_t pick = (ws.home + (uint32_t)(__ffsll((long long)have) - 1)) & (kWorkShares - 1);
-                uint32_t k = 0;
-                if (lane == 0) k = atomicAdd(ws.ctr + pick * ws.stride, 1u);
-                k = __builtin_amdgcn_readfirstlane(k);
-                const uint64_t first = ((uint64_t)pick + (uint64_t)kWorkShares * k) * ws.chunk;
-                if (first < ws.n) {
-                    cursor = (uint32_t)first;
-                    end = (uint32_t)(first + ws.chunk < ws.n ? first + ws.chunk : ws.n);
-                    more = true;
-                    break;
-                }
-            }
-            // Narrow sources (one scene, parts == 8): one share at a time,
-            // from the wave's home share on; a share found drawn out is not
-            // looked at again.
-            while (!PER_RAY_BVH && ws.ctr && !ws.fixed && tried < ws.parts) {
-                const uint32_t x = (ws.home + tried) % ws.parts;
-                uint32_t* const c = ws.ctr + x * ws.stride;
-                const uint32_t seen = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (((uint64_t)x + (uint64_t)ws.parts * seen) * ws.chunk >= ws.n) {
-                    tried++;
-                    continue;
-                }
-                uint32_t k = 0;
-                if (lane == (uint32_t)(__ffsll((long long)__ballot(true)) - 1)) k = atomicAdd(c, 1u);
-                k = __builtin_amdgcn_readfirstlane(k);
-                const uint64_t first = ((uint64_t)x + (uint64_t)ws.parts * k) * ws.chunk;
-                if (first < ws.n) {
-                    cursor = (uint32_t)first;
-                    end = (uint32_t)(first + ws.chunk < ws.n ? first + ws.chunk : ws.n);
-                    more = true;
-                    break;
-                }
-                tried++;
-            }
-        }
+        if (want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
         if (want && more) {
             if (!live) {
-                uint32_t i = cursor + (uint32_t)__popcll(idle & ltMask);
-                if (i < end) {
+                uint32_t i = wc.cursor + (uint32_t)__popcll(idle & ltMask);
+                if (i < wc.end) {
                     float ox, oy, oz, dx, dy, dz, tmax;
                     BvhPtr rb = bvh;
                     if (load(i, ox, oy, oz, dx, dy, dz, tmax, rb)) {
@@ -1214,7 +1211,7 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
                     }
                 }
             }
-            cursor += nIdle;
+            wc.cursor += nIdle;
         } else if (nIdle == 64 && !more) {
             break;   // no items left and every lane finished
         }
@@ -1268,6 +1265,260 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
         if (live && cur == -1 && leaf == -1 && leaf2 == -1) {
             store(item, r, true);
             traced++;
+            live = false;
+        }
+    }
+}
+
+// --------------------------------------------------------- quad traversal --
+// Short BVH4 launches give a ray to a quad (4 neighbouring lanes of a wave, 16
+// rays per wave): lane j tests child j of the ray's node and triangle j of its
+// leaf.  What such a launch waits for is one ray's chain of visits, each a
+// load and then the instructions that lead to the next node's address; with
+// a child per lane a visit is one coalesced 64-byte load and ~70 instructions,
+// and the quad's exchanges are DPP moves, which cost no LDS round trip.  A
+// launch over 3,072 rays takes 12-27 us instead of 35-53.
+constexpr int kQuadStack = 64;        // LDS entries per ray: 4 KB per wave, as kShortStack per lane
+constexpr uint32_t kQuadEntry = 64;   // bytes from a ray's stack entry to its next (16 rays interleaved)
+
+// Value of lane J (0..3) of the caller's quad, and of the lane whose index in
+// the quad differs by the bits of X.  The lanes of a quad always run together.
+template <int J>
+__device__ __forceinline__ uint32_t quadLane(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, J * 0x55, 0xf, 0xf, true);
+}
+template <int J>
+__device__ __forceinline__ float quadLane(float v) {
+    return __uint_as_float(quadLane<J>(__float_as_uint(v)));
+}
+template <int X>
+__device__ __forceinline__ uint32_t quadXor(uint32_t v) {
+    constexpr int ctrl = (0 ^ X) | (1 ^ X) << 2 | (2 ^ X) << 4 | (3 ^ X) << 6;
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, ctrl, 0xf, 0xf, true);
+}
+template <int X>
+__device__ __forceinline__ float quadXor(float v) {
+    return __uint_as_float(quadXor<X>(__float_as_uint(v)));
+}
+__device__ __forceinline__ float quadMin(float v) {
+    v = fminf(v, quadXor<1>(v));
+    return fminf(v, quadXor<2>(v));
+}
+__device__ __forceinline__ uint32_t quadOr(uint32_t v) {
+    v |= quadXor<1>(v);
+    return v | quadXor<2>(v);
+}
+__device__ __forceinline__ unsigned long long waveMask(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
+// A quad's stack: entry i at lds[16 i], the code -1 of an empty stack at entry
+// 0 (popped at most once per ray).  Trees whose worst case is deeper than
+// kQuadStack - 2 are traversed with a stack per lane, which can spill.
+// Entries written by one lane are read by all four: the wave barrier keeps
+// the compiler from moving reads over writes.
+struct QuadStack {
+    int* lds;
+    uint32_t sp;   // kQuadEntry x entries
+    __device__ __forceinline__ int& at(uint32_t off) { return *(int*)((char*)lds + off); }
+    __device__ __forceinline__ void reset() {
+        at(0) = -1;
+        sp = kQuadEntry;
+    }
+    __device__ __forceinline__ int pop() {
+        sp -= kQuadEntry;
+        return at(sp);
+    }
+};
+
+struct QuadRay {
+    float ox, oy, oz, dx, dy, dz;
+    float oa, ia;   // origin and slabInv of this lane's axis (lanes 0..2)
+    PlaneSel sel;
+};
+__device__ __forceinline__ QuadRay makeQuadRay(float ox, float oy, float oz, float dx, float dy, float dz,
+                                               uint32_t j) {
+    QuadRay r{ox, oy, oz, dx, dy, dz};
+    r.oa = j == 0 ? ox : j == 1 ? oy : oz;
+    r.ia = slabInv(j == 0 ? dx : j == 1 ? dy : dz);
+    r.sel = planeSel(quadLane<0>(r.ia), quadLane<1>(r.ia), quadLane<2>(r.ia));
+    return r;
+}
+
+// visitWords of a BVH4 node by the four lanes of a quad: pushes the hit
+// children far to near (ANY: in slot order).
+template <bool ANY>
+__device__ __forceinline__ void visitQuad(const uint4* __restrict__ nodes, int cur, const QuadRay& ray, float tcull,
+                                          uint32_t j, QuadStack& st) {
+    const uint4 w = nodes[(uint32_t)cur * 4u + j];
+    const float A = (__uint_as_float(w.w) - ray.oa) * ray.ia;
+    const float B = __uint_as_float(w.y & 0x7f800000u) * ray.ia;
+    const float An = fmaf(-fabsf(A), kSlabEps, A), Af = fmaf(fabsf(A), kSlabEps, A);
+    const uint32_t n = __builtin_amdgcn_perm(w.z, w.y, ray.sel.nearSel), f = __builtin_amdgcn_perm(w.z, w.y, ray.sel.farSel);
+    const float Bx = quadLane<0>(B), By = quadLane<1>(B), Bz = quadLane<2>(B);
+    const float tx0 = fmaf((float)(n & 0xffu), Bx, quadLane<0>(An)), tx1 = fmaf((float)(f & 0xffu), Bx, quadLane<0>(Af));
+    const float ty0 = fmaf((float)((n >> 8) & 0xffu), By, quadLane<1>(An));
+    const float ty1 = fmaf((float)((f >> 8) & 0xffu), By, quadLane<1>(Af));
+    const float tz0 = fmaf((float)((n >> 16) & 0xffu), Bz, quadLane<2>(An));
+    const float tz1 = fmaf((float)((f >> 16) & 0xffu), Bz, quadLane<2>(Af));
+    const float tn = fmaxf(fmaxf(tx0, ty0), fmaxf(tz0, 0.0f));
+    float tf = fminf(fminf(tx1, ty1), fminf(tz1, tcull));
+    tf = fmaf(fabsf(tf), kFarEps, tf);
+    const bool hit = tn <= tf && (int)w.x != -1;
+    uint32_t at = st.sp, top;
+    if constexpr (ANY) {
+        const uint32_t nib = quadOr(hit ? 1u << j : 0u);
+        top = (uint32_t)__popc(nib) * kQuadEntry;
+        at += (uint32_t)__popc(nib >> (j + 1)) * kQuadEntry;   // below the children taken after it
+    } else {
+        // distances as non-negative integers, so that a difference's sign bit is the comparison
+        const int key = hit ? (int)((__float_as_uint(tn) & ~3u) | j) : 0x7fffffff;
+        const uint32_t nearer = ((uint32_t)((int)quadXor<1>((uint32_t)key) - key) >> 31) +
+                                ((uint32_t)((int)quadXor<2>((uint32_t)key) - key) >> 31) +
+                                ((uint32_t)((int)quadXor<3>((uint32_t)key) - key) >> 31);
+        uint32_t c = hit ? kQuadEntry : 0u;
+        c += quadXor<1>(c);
+        top = c + quadXor<2>(c);
+        at += top - kQuadEntry - nearer * kQuadEntry;
+    }
+    if (hit) st.at(at) = (int)w.x;
+    st.sp += top;
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Tests the triangles of leaf `code`, lane j every fourth from the j-th on, as
+// hitTriangle into the lane's own best r.  ANY: true in every lane of the
+// quad if one of them hit.
+template <bool ANY, bool COUNT>
+__device__ __forceinline__ bool testLeafQuad(const float4* __restrict__ tris, int code, const QuadRay& ray, uint32_t j,
+                                             TraceResult& r, TraceCounters& cnt) {
+    const uint32_t k = (uint32_t)(-code - 2), first = k >> 4, count = (k & 15u) + 1;
+    bool found = false;
+    for (uint32_t i = j; i < count; i += 4) {
+        const float4* p = tris + 3 * (uint64_t)(first + i);
+        const float4 A = p[0], B = p[1], C = p[2];
+        if (COUNT) cnt.tris++;
+        found |= hitTriangle<ANY>(A, B, C, ray, r);
+    }
+    return ANY && quadOr(found ? 1u : 0u) != 0u;
+}
+
+// The ray's closest hit from the best hits of its four lanes: smaller t, then
+// lower index (a lane without a hit has t = tmax, tri -1).
+__device__ __forceinline__ void quadClosest(TraceResult& r) {
+    auto take = [&](float t, uint32_t id, float u, float v) {
+        if (t < r.t || (t == r.t && id < (uint32_t)r.tri)) {
+            r.t = t;
+            r.tri = (int32_t)id;
+            r.u = u;
+            r.v = v;
+        }
+    };
+    {
+        const float t = quadXor<1>(r.t), u = quadXor<1>(r.u), v = quadXor<1>(r.v);
+        const uint32_t id = quadXor<1>((uint32_t)r.tri);
+        take(t, id, u, v);
+    }
+    const float t = quadXor<2>(r.t), u = quadXor<2>(r.u), v = quadXor<2>(r.v);
+    const uint32_t id = quadXor<2>((uint32_t)r.tri);
+    take(t, id, u, v);
+}
+
+// traceWaveRange for BVH4 with a quad per ray.  A quad without a ray has cur,
+// leaf and leaf2 -1.
+template <bool ANY, bool COUNT, bool PER_RAY_BVH = false, class Load, class Store>
+__device__ __forceinline__ void traceQuadRange(const DevScene& s, QuadStack& st, const WorkSource& ws,
+                                               uint32_t refill, Load&& load, Store&& store, TraceCounters& cnt,
+                                               uint32_t& traced) {
+    const uint32_t waveId = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (ws.waves && waveId >= ws.chunks) return;   // no chunk for this wave
+    BvhPtr bvh{(const uint4*)s.nodes, s.tris};
+    const uint32_t lane = __lane_id(), j = lane & 3u;
+    const unsigned long long ltMask = (lane >> 2) ? (~0ull >> (64 - (lane & ~3u))) : 0ull;   // lanes of earlier quads
+    WorkCursor wc(ws, waveId);
+    bool more = true;   // wave-uniform: items may remain
+    bool live = false;
+    uint32_t item = 0;
+    QuadRay ray{};
+    TraceResult r{};
+    float tq = 0.f;   // the quad's culling distance
+    int cur = -1, leaf = -1, leaf2 = -1;
+    while (true) {
+        // ---- refill idle quads from the wave's range or the next chunk
+        const unsigned long long idle = waveMask(!live);
+        const uint32_t nIdle = (uint32_t)__popcll(idle);
+        const bool want = nIdle >= refill || nIdle == 64;
+        if (want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
+        if (want && more) {
+            if (!live) {
+                const uint32_t i = wc.cursor + ((uint32_t)__popcll(idle & ltMask) >> 2);
+                if (i < wc.end) {
+                    float ox, oy, oz, dx, dy, dz, tmax;
+                    BvhPtr rb = bvh;
+                    if (load(i, ox, oy, oz, dx, dy, dz, tmax, rb)) {
+                        if (PER_RAY_BVH) bvh = rb;
+                        ray = makeQuadRay(ox, oy, oz, dx, dy, dz, j);
+                        r.tri = -1;
+                        r.t = tmax;
+                        r.u = r.v = 0.f;
+                        tq = cullT<ANY>(tmax);
+                        st.reset();
+                        cur = 0;
+                        item = i;
+                        live = true;
+                    } else if (j == 0) {
+                        TraceResult dead;
+                        dead.tri = -2;
+                        dead.t = dead.u = dead.v = 0.f;
+                        store(i, dead, false);
+                    }
+                }
+            }
+            wc.cursor += nIdle >> 2;
+        } else if (nIdle == 64 && !more) {
+            break;   // no items left and every quad finished
+        }
+        // ---- inner nodes: descend until every live quad holds a leaf
+        while (waveMask(cur >= 0 && leaf == -1)) {
+            if (cur >= 0) {
+                if (COUNT) cnt.nodes += j == 0;
+                visitQuad<ANY>(PER_RAY_BVH ? bvh.nodes : (const uint4*)s.nodes, cur, ray, tq, j, st);
+                cur = st.pop();
+                if (cur <= -2 && (PER_RAY_BVH ? leaf : leaf2) == -1) {   // postponed: leaf2 is the older one
+                    leaf2 = leaf;
+                    leaf = cur;
+                    cur = st.pop();
+                }
+            }
+        }
+        // ---- leaves: the postponed ones, then any that follow on the stack
+        while (true) {
+            const bool has = leaf != -1 || cur <= -2;
+            if (!waveMask(has)) break;
+            if (has) {
+                int code;
+                if (leaf2 != -1) {
+                    code = leaf2;
+                    leaf2 = -1;
+                } else if (leaf != -1) {
+                    code = leaf;
+                    leaf = -1;
+                } else {
+                    code = cur;
+                    cur = st.pop();
+                }
+                if (testLeafQuad<ANY, COUNT>(PER_RAY_BVH ? bvh.tris : s.tris, code, ray, j, r, cnt)) {
+                    cur = -1;   // any-hit: done
+                    leaf = leaf2 = -1;
+                }
+                if (!ANY) tq = quadMin(cullT<ANY>(r.t));
+            }
+        }
+        // ---- finished rays
+        if (live && cur == -1) {
+            quadClosest(r);
+            if (j == 0) {
+                store(item, r, true);
+                traced++;
+            }
             live = false;
         }
     }
