@@ -6,9 +6,8 @@
  * (EL_OK == 0, negative on error) unless stated otherwise; the message of the
  * last error on a context is returned by el_last_error().
  *
- * Threading: one el_ctx per host thread; a context owns three HIP streams
- * on one device (its launches and the two shadow launches that may run
- * beside them).  No host thread it starts outlives a call: el_upload_scene
+ * Threading: one el_ctx per host thread; a context owns one HIP stream on
+ * one device.  No host thread it starts outlives a call: el_upload_scene
  * builds on up to the hardware's thread count, capped by OMP_NUM_THREADS
  * when that is set.  Calls are synchronous on return unless stated
  * otherwise.
@@ -66,23 +65,22 @@ extern "C" {
                                    device memory): el_adjoint then traces no
                                    ray.  The image is the same either way.   */
 
-#define EL_FLAG_SERIAL_SHADOWS 16u /* wavefront: run every shadow launch after
-                                     the bounce's shade on the one stream.  By
-                                     default the two shadow launches of a
-                                     bounce run on two more streams, beside
-                                     each other and the next bounce's
-                                     closest-hit launch, when the launches are
-                                     small (generations under 16 M paths, or
-                                     from the third bounce on); the image is
-                                     the same either way                       */
+#define EL_FLAG_SERIAL_SHADOWS 16u /* wavefront: every closest-hit and shadow
+                                     queue in a launch of its own, one after
+                                     the other.  By default a bounce's two
+                                     shadow queues and the next bounce's
+                                     closest hits are one launch where they
+                                     are small (generations under 16 M paths,
+                                     or from the third bounce on); the image
+                                     is the same either way                    */
 
 #define EL_FLAG_KERNEL_TIMES 32u /* wavefront: time every closest-hit, shade
-                                     and shadow launch with events on its
+                                     and shadow launch with events on the
                                      stream (el_stats extend_ms, shade_ms,
                                      shadow_ms; 0 without the flag).  The
-                                     events add a few microseconds between
-                                     launches: a 128x128 x 32 spp render takes
-                                     ~10 % longer with them                   */
+                                     launches are those of
+                                     EL_FLAG_SERIAL_SHADOWS, so a small render
+                                     takes longer with the flag                */
 
 /* Passes, same numbering as the reference's `enum Passes` (kernel.h:7). */
 #define EL_PASS_BEAUTY     0
@@ -170,11 +168,7 @@ typedef struct {
     double   extend_ms;        /* summed closest-hit kernel time (wavefront,
                                   EL_FLAG_KERNEL_TIMES; shadow_ms, shade_ms
                                   likewise)                                  */
-    double   shadow_ms;        /* summed shadow kernel time (wavefront); el_render
-                                  runs a bounce's two shadow launches on two
-                                  more streams while the next bounce's
-                                  closest-hit launch runs, so the times
-                                  overlap and their sum exceeds render_ms    */
+    double   shadow_ms;        /* summed shadow kernel time (wavefront)      */
     double   shade_ms;         /* summed shading kernel time (wavefront)     */
     uint64_t extend_launches;  /* number of closest-hit launches timed       */
     uint64_t extend_rays;      /* rays processed by those launches           */
@@ -357,11 +351,7 @@ typedef struct el_batch el_batch;
 #define EL_BATCH_GRAPH 1u   /* capture the launch sequence in a hipGraph once,
                                replay it on later renders with equal plans  */
 #define EL_BATCH_NO_CULL 4u /* as EL_FLAG_NO_CULL                            */
-#define EL_BATCH_SERIAL_SHADOWS 8u /* as EL_FLAG_SERIAL_SHADOWS (batches overlap
-                                      a bounce's shadow launches with the next
-                                      extension from the third bounce on, or
-                                      always for generations under 16 M paths,
-                                      also inside a captured graph)           */
+#define EL_BATCH_SERIAL_SHADOWS 8u /* as EL_FLAG_SERIAL_SHADOWS               */
 
 typedef struct {
     uint32_t max_depth;    /* 0 -> 5                                        */

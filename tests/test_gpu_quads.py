@@ -80,3 +80,21 @@ def test_tree_deeper_than_the_quads_stack(gpu_ctx):
     tb, tt, _, _ = orc.closest_brute(v, rays)
     assert np.array_equal(tri, tb) and np.array_equal(t[tb >= 0], tt[tb >= 0]) and (tb >= 0).any()
     assert gpu_ctx.render(2, depth=3, seed=1).paths == 2 * 32 * 32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("side,spp,width", [(8, 1, 4), (9, 3, 4), (40, 5, 8), (200, 9, 4), (512, 6, 4), (512, 2, 8)])
+def test_queues_in_one_launch_equal_launches_of_their_own(gpu_ctx, side, spp, width):
+    """A bounce's shadow queues and the next closest hits in one launch, its waves divided among them (a wave a chunk,
+    or in proportion to the rays), against a launch for each."""
+    print(f"[quads] {side}x{side} {spp} spp width {width}", flush=True)
+    gpu_ctx.upload(scenegen.sphere_field_arrays(n_spheres=20, res=(side, side), seed=2))
+    out = []
+    for flags in (0, eleven.FLAG_SERIAL_SHADOWS, 0):
+        gpu_ctx.clear()
+        st = gpu_ctx.render(spp, depth=5, seed=4, bvh_width=width, flags=flags)
+        img, cnt, rays, verts = gpu_ctx.read()
+        out.append((img.view(np.uint32), cnt, rays, verts, st.extend_rays))
+    gpu_ctx.render(1, depth=1, bvh_width=4)   # the context is shared: back to the default tree
+    for o in out[1:]:
+        assert all(np.array_equal(x, y) for x, y in zip(out[0], o))

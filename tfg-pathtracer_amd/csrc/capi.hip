@@ -150,12 +150,6 @@ struct el_ctx {
     bool aovOn = false;
 
     std::vector<hipEvent_t> evPool;
-    // Wavefront renders: the shadow launches of bounce b run on `shadowStream`
-    // (HDRI) and `shadowStreamP` (point lights) while the extension launch of
-    // bounce b + 1 runs on `stream`; syncPool holds the events that order
-    // them (no timing).
-    hipStream_t shadowStream = nullptr, shadowStreamP = nullptr;
-    std::vector<hipEvent_t> syncPool;
 };
 
 static int fail(el_ctx* c, int code, const std::string& what) {
@@ -216,8 +210,6 @@ int el_create(el_ctx** out, int device) {
     // resident-thread capacity: 32 waves of 64 lanes per CU
     c->maxThreads = (uint32_t)c->cus * 2048u;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
-    if (hipStreamCreateWithFlags(&c->shadowStream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
-    if (hipStreamCreateWithFlags(&c->shadowStreamP, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (c->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
     if (scratchAddress(device, &c->scratch) != hipSuccess) return EL_ERR_HIP;
     *out = c.release();
@@ -228,13 +220,8 @@ void el_destroy(el_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    if (c->shadowStream) (void)hipStreamSynchronize(c->shadowStream);
-    if (c->shadowStreamP) (void)hipStreamSynchronize(c->shadowStreamP);
     for (auto e : c->evPool) (void)hipEventDestroy(e);
-    for (auto e : c->syncPool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
-    if (c->shadowStream) (void)hipStreamDestroy(c->shadowStream);
-    if (c->shadowStreamP) (void)hipStreamDestroy(c->shadowStreamP);
     delete c;
 }
 
@@ -342,7 +329,7 @@ static int uploadBvh(el_ctx* c, int width) {
     EL_HIP(c, upload(c->dNodes, nodes, c->wide.nodes.size(), c->stream));
     EL_HIP(c, upload(c->dTris, c->wide.triStream.data(), c->wide.triStream.size() * sizeof(float), c->stream));
     c->gcap = std::max(1, c->wide.stackBound + 2 - dev::kShortStack);
-    EL_HIP(c, c->dGstack.ensure((size_t)kSpillSets * c->gcap * c->maxThreads * sizeof(int)));
+    EL_HIP(c, c->dGstack.ensure((size_t)c->gcap * c->maxThreads * sizeof(int)));
     c->ds.nodes = c->dNodes.p;
     c->ds.tris = c->dTris.as<float4>();
     c->ds.width = width;
@@ -574,18 +561,15 @@ int el_clear(el_ctx* c) {
 
 }  // extern "C"
 
-// Generations with fewer paths overlap every bounce's shadow launches with
-// the next extension; larger ones from the third bounce on.
-constexpr uint32_t kOverlapPaths = 16u << 20;
+// Generations with fewer paths trace every bounce's shadows in one launch with
+// the next extension; larger ones from the third bounce on (bounceTogether).
+constexpr uint32_t kTogetherPaths = 16u << 20;
 
-static hipEvent_t syncEvent(el_ctx* c, size_t i) {
-    while (c->syncPool.size() <= i) {
-        hipEvent_t e;
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return nullptr;
-        c->syncPool.push_back(e);
-    }
-    return c->syncPool[i];
-}
+// Large launches keep the GPU busy on their own, and rays of different queues
+// side by side cost cache hits (the extension's L2 hit rate fell from 0.70 to
+// 0.62 next to the first bounce's shadows); small ones last one ray's chain
+// of dependent fetches, which the three queues then spend at once.
+static bool bounceTogether(uint32_t paths, uint32_t bounce) { return paths < kTogetherPaths || bounce >= 2; }
 
 static hipEvent_t poolEvent(el_ctx* c, size_t i) {
     while (c->evPool.size() <= i) {
@@ -768,9 +752,6 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
         if (recordHits) {
             EL_HIP(c, c->wVis.ensure(Q * sizeof(uint32_t)));
             q.pathVis = c->wVis.as<uint32_t>();
-            // the shadow launches set visibility bits of one word per path:
-            // they stay in order, and the point-light terms are added at once
-            q.pendP = nullptr;
         }
         a.npad = (uint32_t)npad;
         size_t ev = 2;
@@ -780,99 +761,48 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
             a.genSample = (uint32_t)(start / npad);
             a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
             EL_HIP(c, launchWfCamera(lc, c->ds, a, q));
-            // Per bounce b: extend (stream) -> shade (stream) -> both shadow
-            // launches (shadowStream, shadowStreamP).  The shadows of bounce
-            // b need only what shade b wrote and update nothing the extension
-            // of bounce b + 1 reads (their counters are set b & 1, the
-            // extension clears set (b + 1) & 1), so the three overlap; shade
-            // b + 1 and finalize wait for them (they add to the path
-            // radiance).  The point-light launch writes its terms to pendP,
-            // which shade b + 1 or finalize adds after the HDRI term, so it
-            // also runs beside the HDRI launch (a recording render keeps the
-            // two in order on one stream).
-            LaunchCfg lcs = lc, lcp = lc;
-            lcs.stream = c->shadowStream;
-            lcp.stream = c->shadowStreamP;
-            const size_t spillSet = (size_t)c->gcap * lc.maxThreads;
-            hipEvent_t doneH = nullptr, doneP = nullptr;
-            // Large launches keep the GPU busy on their own, and overlapping
-            // two of them costs cache hits (the extension's L2 hit rate fell
-            // from 0.70 to 0.62 next to the first bounce's shadows); small
-            // ones last one ray's chain of dependent fetches, which the
-            // overlap hides.
-            const bool serial = (p->flags & EL_FLAG_SERIAL_SHADOWS) != 0;
+            // Per bounce b: extend -> shade -> both shadow queues.  Where the
+            // launches are small, the shadows of bounce b and the extension
+            // of bounce b + 1 are one launch (launchWfTrace).
+            const bool apart = (p->flags & (EL_FLAG_SERIAL_SHADOWS | EL_FLAG_KERNEL_TIMES | EL_FLAG_COUNT_TRAVERSAL)) != 0;
             const bool kernelTimes = (p->flags & EL_FLAG_KERNEL_TIMES) != 0;
+            auto launch = [&](int kind, auto&& f) -> hipError_t {   // one launch, timed if asked
+                if (!kernelTimes) return f();
+                hipEvent_t x0 = poolEvent(c, ev), x1 = poolEvent(c, ev + 1);
+                if (!x0 || !x1) return hipErrorOutOfMemory;
+                hipError_t e = hipEventRecord(x0, c->stream);
+                if (e == hipSuccess) e = f();
+                if (e == hipSuccess) e = hipEventRecord(x1, c->stream);
+                timed.push_back({ev, kind});
+                ev += 2;
+                return e;
+            };
+            bool extended = false;   // bounce b's closest hits were traced with the previous bounce's shadows
             for (uint32_t b = 0; b < depth; b++) {
-                const bool overlap = !serial && (a.genCount < kOverlapPaths || b >= 2);
+                const bool together = !apart && bounceTogether(a.genCount, b), more = b + 1 < depth;
                 a.bounce = b;
                 q.parity = b & 1u;
-                // point-light terms deferred where the two shadow launches run
-                // at once (elsewhere the P launch adds them itself)
-                q.deferP = overlap && q.pendP != nullptr ? 1u : 0u;
+                q.deferP = together ? 1u : 0u;
+                q.visBit = recordHits ? 1u << (2 * b) : 0u;
                 const int cur = b & 1, nxt = cur ^ 1;
                 uint32_t* cntCur = q.counters + (cur ? kQRay1 : kQRay0);
                 uint32_t* cntNxt = q.counters + (nxt ? kQRay1 : kQRay0);
-                hipEvent_t x0 = poolEvent(c, ev), x1 = poolEvent(c, ev + 1);
-                if (kernelTimes) EL_HIP(c, hipEventRecord(x0, c->stream));
-                EL_HIP(c, launchWfExtend(lc, c->ds, q, q.ray[cur], cntCur, cntNxt, a.genCount, countTrav, ctr));
-                if (kernelTimes) EL_HIP(c, hipEventRecord(x1, c->stream));
-                if (kernelTimes) timed.push_back({ev, 0});
-                ev += 2;
-                if (doneH) EL_HIP(c, hipStreamWaitEvent(c->stream, doneH, 0));
-                if (doneP) EL_HIP(c, hipStreamWaitEvent(c->stream, doneP, 0));
-                hipEvent_t y0 = poolEvent(c, ev), y1 = poolEvent(c, ev + 1);
-                if (kernelTimes) EL_HIP(c, hipEventRecord(y0, c->stream));
-                EL_HIP(c, launchWfShade(lc, c->ds, a, q, q.ray[cur], cntCur, q.ray[nxt], cntNxt, a.genCount, ctr));
-                if (kernelTimes) EL_HIP(c, hipEventRecord(y1, c->stream));
-                if (kernelTimes) timed.push_back({ev, 1});
-                ev += 2;
-                // beside the extension, each shadow launch spills to its own area
-                const bool split = q.deferP != 0u;   // H and P on their own streams
-                const LaunchCfg& lsH = overlap ? lcs : lc;
-                const LaunchCfg& lsP = split ? lcp : lsH;
-                WfState qh = q, qp = q;
-                if (overlap) qh.gstack = q.gstack + spillSet;
-                qp.gstack = split ? q.gstack + 2 * spillSet : qh.gstack;
-                if (recordHits) {
-                    qh.visBit = 1u << (2 * b);
-                    qp.visBit = 1u << (2 * b + 1);
+                if (!extended)
+                    EL_HIP(c, launch(0, [&] {
+                        return launchWfExtend(lc, c->ds, q, q.ray[cur], cntCur, cntNxt, a.genCount, countTrav, ctr);
+                    }));
+                EL_HIP(c, launch(1, [&] {
+                    return launchWfShade(lc, c->ds, a, q, q.ray[cur], cntCur, q.ray[nxt], cntNxt, a.genCount, ctr);
+                }));
+                if (together) {
+                    EL_HIP(c, launchWfTrace(lc, c->ds, q, more ? q.ray[nxt] : nullptr, cntNxt, cntCur, a.genCount, ctr));
+                } else {
+                    for (int light = 0; light < 2; light++)
+                        EL_HIP(c, launch(2, [&] { return launchWfShadow(lc, c->ds, q, light, a.genCount, ctr); }));
                 }
-                if (overlap) {
-                    hipEvent_t shaded = syncEvent(c, 3 * b);
-                    if (!shaded) return fail(c, EL_ERR_HIP, "event creation failed");
-                    EL_HIP(c, hipEventRecord(shaded, c->stream));
-                    EL_HIP(c, hipStreamWaitEvent(c->shadowStream, shaded, 0));
-                    if (split) EL_HIP(c, hipStreamWaitEvent(c->shadowStreamP, shaded, 0));
-                }
-                hipEvent_t z0 = poolEvent(c, ev), z1 = poolEvent(c, ev + 1);
-                if (kernelTimes) EL_HIP(c, hipEventRecord(z0, lsH.stream));
-                EL_HIP(c, launchWfShadow(lsH, c->ds, qh, q.shadowH, q.counters + qShadow(q.parity, 0), a.genCount,
-                                         ctr));
-                if (kernelTimes) EL_HIP(c, hipEventRecord(z1, lsH.stream));
-                if (kernelTimes) timed.push_back({ev, 2});
-                ev += 2;
-                hipEvent_t w0 = poolEvent(c, ev), w1 = poolEvent(c, ev + 1);
-                if (kernelTimes) EL_HIP(c, hipEventRecord(w0, lsP.stream));
-                EL_HIP(c, launchWfShadow(lsP, c->ds, qp, q.shadowP, q.counters + qShadow(q.parity, 1), a.genCount,
-                                         ctr));
-                if (kernelTimes) EL_HIP(c, hipEventRecord(w1, lsP.stream));
-                if (kernelTimes) timed.push_back({ev, 2});
-                ev += 2;
-                doneH = doneP = nullptr;
-                if (overlap) {
-                    doneH = syncEvent(c, 3 * b + 1);
-                    if (!doneH) return fail(c, EL_ERR_HIP, "event creation failed");
-                    EL_HIP(c, hipEventRecord(doneH, c->shadowStream));
-                }
-                if (split) {
-                    doneP = syncEvent(c, 3 * b + 2);
-                    if (!doneP) return fail(c, EL_ERR_HIP, "event creation failed");
-                    EL_HIP(c, hipEventRecord(doneP, c->shadowStreamP));
-                }
+                extended = together && more;
                 extendLaunches++;
             }
-            if (doneH) EL_HIP(c, hipStreamWaitEvent(c->stream, doneH, 0));
-            if (doneP) EL_HIP(c, hipStreamWaitEvent(c->stream, doneP, 0));
             EL_HIP(c, launchWfFinalize(lc, c->ds, a, q, c->dAccum.as<float4>(), c->dCounts.as<uint32_t>(), aovBuf,
                                        ctr));
         }
@@ -1305,24 +1235,13 @@ struct el_batch {
     std::vector<uint64_t> seed;
     int width = 4;
     DevBuf dScenes, dSegs, dGstack, dCounters;
-    DevBuf wRay0, wRay1, wHits, wShH, wShP, wT, wL, wPix, wSample, wQuiet, wCounters;
+    DevBuf wRay0, wRay1, wHits, wShH, wShP, wT, wL, wPix, wSample, wQuiet, wPend, wCounters;
     size_t wfCap = 0, wfQcap = 0;
     hipGraphExec_t graph = nullptr;
     std::string graphKey;
     el_stats stats{};
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    hipStream_t shadowStream = nullptr;   // shadow launches of small bounces (as el_render)
-    std::vector<hipEvent_t> syncPool;
 };
-
-static hipEvent_t batchSyncEvent(el_batch* b, size_t i) {
-    while (b->syncPool.size() <= i) {
-        hipEvent_t e;
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return nullptr;
-        b->syncPool.push_back(e);
-    }
-    return b->syncPool[i];
-}
 
 static int bfail(el_batch* b, int code, const std::string& what) {
     if (b) b->err = what;
@@ -1355,7 +1274,6 @@ int el_batch_create(el_batch** out, int device) {
     if (hipGetDeviceProperties(&prop, device) != hipSuccess) return EL_ERR_HIP;
     b->maxThreads = (uint32_t)prop.multiProcessorCount * 2048u;
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
-    if (hipStreamCreateWithFlags(&b->shadowStream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (hipEventCreate(&b->e0) != hipSuccess || hipEventCreate(&b->e1) != hipSuccess) return EL_ERR_HIP;
     if (b->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
     *out = b.release();
@@ -1370,10 +1288,7 @@ void el_batch_destroy(el_batch* b) {
     for (auto* c : b->scenes) el_destroy(c);
     if (b->e0) (void)hipEventDestroy(b->e0);
     if (b->e1) (void)hipEventDestroy(b->e1);
-    if (b->shadowStream) (void)hipStreamSynchronize(b->shadowStream);
-    for (auto e : b->syncPool) (void)hipEventDestroy(e);
     if (b->stream) (void)hipStreamDestroy(b->stream);
-    if (b->shadowStream) (void)hipStreamDestroy(b->shadowStream);
     delete b;
 }
 
@@ -1440,6 +1355,7 @@ static int batchEnsureWf(el_batch* b, size_t cap, size_t qcap) {
     EL_BHIP(b, b->wPix.ensure(cap * 4));
     EL_BHIP(b, b->wSample.ensure(cap * 4));
     EL_BHIP(b, b->wQuiet.ensure(cap * 8));
+    EL_BHIP(b, b->wPend.ensure(cap * 16));
     EL_BHIP(b, b->wCounters.ensure(kQCounters * sizeof(uint32_t)));
     b->wfCap = std::max(b->wfCap, cap);
     b->wfQcap = std::max(b->wfQcap, qcap);
@@ -1491,13 +1407,13 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         total += work[i];
     }
     EL_BHIP(b, upload(b->dScenes, recs.data(), S * sizeof(DevScene), b->stream));
-    EL_BHIP(b, b->dGstack.ensure((size_t)kSpillSets * gcap * b->maxThreads * sizeof(int)));
+    EL_BHIP(b, b->dGstack.ensure((size_t)gcap * b->maxThreads * sizeof(int)));
     // generation plan
     uint64_t Q = p->queue_cap;
     if (!Q) {
         size_t freeB = 0, totalB = 0;
         EL_BHIP(b, hipMemGetInfo(&freeB, &totalB));
-        Q = std::max<uint64_t>(1u << 20, freeB / 4 / (6 * 32 + 44));
+        Q = std::max<uint64_t>(1u << 20, freeB / 4 / (6 * 32 + 60));
     }
     Q = std::max<uint64_t>(64, (Q / 64) * 64);
     if (Q > total) Q = total;
@@ -1556,6 +1472,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
     q.pathSample = b->wSample.as<uint32_t>();
     q.pathQuiet = b->wQuiet.as<uint64_t>();
     q.pathAov = nullptr;
+    q.pendP = b->wPend.as<float4>();
     q.counters = b->wCounters.as<uint32_t>();
     q.segSize = (uint32_t)segSize;
     q.gstack = lc.gstack;
@@ -1570,22 +1487,17 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
     unsigned long long* ctr = b->dCounters.as<unsigned long long>();
     EL_BHIP(b, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, b->stream));
     const DevScene* dsc = b->dScenes.as<DevScene>();
-    // Shadow launches of small bounces overlap the next extension on a
-    // second stream, as in el_render (inside a captured graph the events
-    // become the graph's fork and join edges).
-    LaunchCfg lcs = lc;
-    lcs.stream = b->shadowStream;
-    const bool serialShadows = (p->flags & EL_BATCH_SERIAL_SHADOWS) != 0;
-    auto launchAll = [&]() -> hipError_t {
+    const bool apart = (p->flags & EL_BATCH_SERIAL_SHADOWS) != 0;
+    auto launchAll = [&]() -> hipError_t {   // the launches of el_render's loop
         hipError_t e;
-        size_t ev = 0;
         for (const BatchGen& g : gens) {
-            hipEvent_t shadowsDone = nullptr;
             const BatchSeg* gseg = b->dSegs.as<BatchSeg>() + g.segOffset;
             if ((e = launchBtCamera(lc, dsc, gseg, g.nseg, g.count, depth, !(p->flags & EL_BATCH_NO_CULL), q)) !=
                 hipSuccess)
                 return e;
+            bool extended = false;
             for (uint32_t bo = 0; bo < depth; bo++) {
+                const bool together = !apart && bounceTogether(g.count, bo), more = bo + 1 < depth;
                 RenderArgs a{};
                 a.maxDepth = depth;
                 a.bounce = bo;
@@ -1593,40 +1505,24 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
                 const int cur = bo & 1, nxt = cur ^ 1;
                 uint32_t* cntCur = q.counters + (cur ? kQRay1 : kQRay0);
                 uint32_t* cntNxt = q.counters + (nxt ? kQRay1 : kQRay0);
-                q.parity = bo & 1u;
-                const bool overlap = !serialShadows && (g.count < kOverlapPaths || bo >= 2);
-                if ((e = launchBtExtend(lc, dsc, width, q, q.ray[cur], cntCur, cntNxt, g.count, ctr)) != hipSuccess)
+                WfState qb = q;
+                qb.parity = bo & 1u;
+                qb.deferP = together ? 1u : 0u;
+                if (!extended &&
+                    (e = launchBtExtend(lc, dsc, width, qb, q.ray[cur], cntCur, cntNxt, g.count, ctr)) != hipSuccess)
                     return e;
-                if (shadowsDone && (e = hipStreamWaitEvent(b->stream, shadowsDone, 0)) != hipSuccess) return e;
-                if ((e = launchBtShade(lc, dsc, a, q, q.ray[cur], cntCur, q.ray[nxt], cntNxt, g.count, ctr)) !=
+                if ((e = launchBtShade(lc, dsc, a, qb, q.ray[cur], cntCur, q.ray[nxt], cntNxt, g.count, ctr)) !=
                     hipSuccess)
                     return e;
-                shadowsDone = nullptr;
-                if (overlap) {
-                    hipEvent_t shaded = batchSyncEvent(b, ev++), done = batchSyncEvent(b, ev++);
-                    if (!shaded || !done) return hipErrorOutOfMemory;
-                    if ((e = hipEventRecord(shaded, b->stream)) != hipSuccess) return e;
-                    if ((e = hipStreamWaitEvent(b->shadowStream, shaded, 0)) != hipSuccess) return e;
-                    WfState qs = q;   // the shadow stream's spill area
-                    qs.gstack = q.gstack + (size_t)gcap * lc.maxThreads;
-                    if ((e = launchBtShadow(lcs, dsc, width, qs, q.shadowH, q.counters + qShadow(q.parity, 0),
-                                            g.count, ctr)) != hipSuccess)
-                        return e;
-                    if ((e = launchBtShadow(lcs, dsc, width, qs, q.shadowP, q.counters + qShadow(q.parity, 1),
-                                            g.count, ctr)) != hipSuccess)
-                        return e;
-                    if ((e = hipEventRecord(done, b->shadowStream)) != hipSuccess) return e;
-                    shadowsDone = done;
+                if (together) {
+                    e = launchBtTrace(lc, dsc, width, qb, more ? q.ray[nxt] : nullptr, cntNxt, cntCur, g.count, ctr);
+                    if (e != hipSuccess) return e;
                 } else {
-                    if ((e = launchBtShadow(lc, dsc, width, q, q.shadowH, q.counters + qShadow(q.parity, 0), g.count,
-                                            ctr)) != hipSuccess)
-                        return e;
-                    if ((e = launchBtShadow(lc, dsc, width, q, q.shadowP, q.counters + qShadow(q.parity, 1), g.count,
-                                            ctr)) != hipSuccess)
-                        return e;
+                    for (int light = 0; light < 2; light++)
+                        if ((e = launchBtShadow(lc, dsc, width, qb, light, g.count, ctr)) != hipSuccess) return e;
                 }
+                extended = together && more;
             }
-            if (shadowsDone && (e = hipStreamWaitEvent(b->stream, shadowsDone, 0)) != hipSuccess) return e;
             if ((e = launchBtFinalize(lc, dsc, gseg, g.nseg, g.finTotal, q, ctr)) != hipSuccess) return e;
         }
         return hipSuccess;

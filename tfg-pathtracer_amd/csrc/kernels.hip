@@ -95,14 +95,19 @@ __device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n) {
     return W == 4 && s.quads && n <= kQuadRays;
 }
 
-// Chunks of a traversal launch over n items: kChunkRays, smaller (down to the
-// G rays a wave holds at once: one per lane, or one per quad) when n items
-// would not give every wave of the grid eight of them.
-__device__ __forceinline__ WorkSource splitWork(uint32_t n, bool quads) {
+// Waves of the grid and the calling one's index.
+__device__ __forceinline__ uint32_t gridWaves() { return (gridDim.x * blockDim.x) >> 6; }
+__device__ __forceinline__ uint32_t gridWave() { return (blockIdx.x * blockDim.x + threadIdx.x) >> 6; }
+
+// Chunks of n items for `waves` waves, the first-th of which calls: kChunkRays,
+// smaller (down to the G rays a wave holds at once: one per lane, or one per
+// quad) when n items would not give every wave eight of them.
+__device__ __forceinline__ WorkSource splitWork(uint32_t n, bool quads, uint32_t first, uint32_t waves) {
     const uint32_t G = quads ? 16 : 64;
     WorkSource ws{};
     ws.n = n;
-    ws.waves = (gridDim.x * blockDim.x) >> 6;
+    ws.first = first;
+    ws.waves = waves;
     const uint32_t fit = (uint32_t)((uint64_t)n / ((uint64_t)ws.waves * 8)) & ~(G - 1);
     ws.chunk = fit < G ? G : (fit > kChunkRays ? kChunkRays : fit);
     ws.chunks = (uint32_t)(((uint64_t)n + ws.chunk - 1) / ws.chunk);
@@ -121,15 +126,20 @@ constexpr uint32_t kStaticChunks = 32;
 // The work of a queue of n items, drawn from the counters of `kind` where it
 // has more than kStaticChunks chunks for a wave.
 template <bool WIDE>
-__device__ __forceinline__ WorkSource chunkSource(uint32_t* qcounters, int kind, uint32_t n, bool quads) {
-    WorkSource ws = splitWork(n, quads);
-    if (ws.chunks > (uint64_t)ws.waves * kStaticChunks) ws.waves = 0;
+__device__ __forceinline__ WorkSource chunkSource(uint32_t* qcounters, int kind, uint32_t n, bool quads,
+                                                  uint32_t first, uint32_t waves) {
+    WorkSource ws = splitWork(n, quads, first, waves);
+    if (ws.chunks > ws.waves * kStaticChunks) ws.waves = 0;
     ws.ctr = qcounters + kQChunk + kind * kChunkShares * kChunkStride;
     ws.stride = kChunkStride;
     static_assert(kChunkShares == (int)kWorkShares, "one chunk share per lane");
     ws.parts = WIDE ? kChunkShares : kXcds;
     ws.home = blockIdx.x % ws.parts;
     return ws;
+}
+template <bool WIDE>
+__device__ __forceinline__ WorkSource chunkSource(uint32_t* qcounters, int kind, uint32_t n, bool quads) {
+    return chunkSource<WIDE>(qcounters, kind, n, quads, gridWave(), gridWaves());
 }
 // Zeroes the chunk counters of `kind` (threads 0..kChunkShares-1 of block 0).
 __device__ __forceinline__ void resetChunks(uint32_t* qcounters, int kind) {
@@ -212,19 +222,19 @@ __device__ __forceinline__ TravStack makeStack(const DevScene& s, int* gstack, u
     return st;
 }
 
-// Traces n rays, by quads or by lanes (useQuads).  overflow: a lane's stack was too small.
+// Traces the items of ws, by quads or by lanes.  overflow is set if a lane's stack was too small.
 template <int W, bool ANY, bool COUNT, bool PER_RAY_BVH, class Load, class Store>
 __device__ __forceinline__ void traceQueue(const DevScene& s, int* gstack, uint32_t gthreads, const WorkSource& ws,
-                                           uint32_t n, uint32_t refill, Load&& load, Store&& store,
+                                           bool quads, uint32_t refill, Load&& load, Store&& store,
                                            TraceCounters& cnt, uint32_t& traced, uint32_t& overflow) {
-    if (useQuads<W>(s, n)) {
+    if (W == 4 && quads) {
         extern __shared__ int lds[];
         QuadStack st{lds + (threadIdx.x >> 6) * (kQuadStack * 16) + ((threadIdx.x >> 2) & 15u), 0};
         traceQuadRange<ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, traced);
     } else {
         TravStack st = makeStack(s, gstack, gthreads);
         traceWaveRange<W, ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, traced);
-        overflow = st.overflow;
+        overflow |= st.overflow;
     }
 }
 
@@ -236,7 +246,8 @@ EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, 
                                     uint32_t gthreads, uint32_t refill, unsigned long long* counters) {
     TraceCounters cnt{0, 0};
     uint32_t traced = 0, overflow = 0;
-    const WorkSource ws = splitWork(n, useQuads<W>(s, n));
+    const bool quads = useQuads<W>(s, n);
+    const WorkSource ws = splitWork(n, quads, gridWave(), gridWaves());
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr&) {
         const float* r = rays + (uint64_t)i * 6;
@@ -261,7 +272,7 @@ EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, 
             }
         }
     };
-    traceQueue<W, ANY, COUNT, false>(s, gstack, gthreads, ws, n, refill, load, store, cnt, traced, overflow);
+    traceQueue<W, ANY, COUNT, false>(s, gstack, gthreads, ws, quads, refill, load, store, cnt, traced, overflow);
     const int slots[3] = {kStatNodes, kStatTris, kStatOverflow};
     const uint32_t vals[3] = {cnt.nodes, cnt.tris, overflow};
     blockFlush<3>(counters, slots, vals);
@@ -832,29 +843,17 @@ struct ManyScenes {
     __device__ __forceinline__ const DevScene& any() const { return p[0]; }
 };
 
-// Also clears the counters the following shade kernel appends to: the next
-// ray queue and both shadow queues.
-template <int W, bool COUNT, class P>
-EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restrict__ rayIn,
-                                        const uint32_t* countIn, uint32_t* resetNext, uint32_t refill,
-                                        unsigned long long* counters) {
-    const DevScene& s0 = sc.any();
-    TraceCounters cnt{0, 0};
-    QueueMap qm;
-    qm.load(countIn);
-    const uint32_t n = qm.total();
-    // the counters the shade and shadow launches of this bounce use (set
-    // q.parity; the shadow launches of the previous bounce, which may still
-    // run, use the other set)
-    if (blockIdx.x == 0 && threadIdx.x < kXcds) {
-        resetNext[threadIdx.x] = 0;
-        q.counters[qShadow(q.parity, 0) + threadIdx.x] = 0;
-        q.counters[qShadow(q.parity, 1) + threadIdx.x] = 0;
-    }
-    resetChunks(q.counters, chunkShadow(q.parity, 0));
-    resetChunks(q.counters, chunkShadow(q.parity, 1));
+// Tallies of a launch's traversals.
+struct QueueTally {
     uint32_t rays = 0, overflow = 0;
-    const WorkSource ws = chunkSource<P::kMany>(q.counters, kChunkExt, n, useQuads<W>(s0, n));
+    TraceCounters cnt{0, 0};
+};
+
+// Closest hits of a ray queue's n entries.
+template <int W, bool COUNT, class P>
+__device__ __forceinline__ void extendQueue(const P& sc, const WfState& q, const float4* __restrict__ rayIn,
+                                            const QueueMap& qm, const WorkSource& ws, bool quads, uint32_t refill,
+                                            QueueTally& tl) {
     const uint32_t segSize = q.segSize;
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr& bvh) {
@@ -876,9 +875,35 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restric
     auto store = [&](uint32_t i, const TraceResult& h, bool) {
         q.hits[qm.entry(i, segSize)] = make_float4(__int_as_float(h.tri), h.t, h.u, h.v);
     };
-    traceQueue<W, false, COUNT, P::kMany>(s0, q.gstack, q.gthreads, ws, n, refill, load, store, cnt, rays, overflow);
+    traceQueue<W, false, COUNT, P::kMany>(sc.any(), q.gstack, q.gthreads, ws, quads, refill, load, store, tl.cnt,
+                                          tl.rays, tl.overflow);
+}
+
+// Clears the counters the next shade kernel appends to: the next ray queue
+// and both shadow queues of `parity`, with their chunk counters.
+__device__ __forceinline__ void resetForShade(const WfState& q, uint32_t* resetNext, uint32_t parity) {
+    if (blockIdx.x == 0 && threadIdx.x < kXcds) {
+        resetNext[threadIdx.x] = 0;
+        q.counters[qShadow(parity, 0) + threadIdx.x] = 0;
+        q.counters[qShadow(parity, 1) + threadIdx.x] = 0;
+    }
+    resetChunks(q.counters, chunkShadow(parity, 0));
+    resetChunks(q.counters, chunkShadow(parity, 1));
+}
+
+template <int W, bool COUNT, class P>
+EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restrict__ rayIn,
+                                        const uint32_t* countIn, uint32_t* resetNext, uint32_t refill,
+                                        unsigned long long* counters) {
+    QueueMap qm;
+    qm.load(countIn);
+    const uint32_t n = qm.total();
+    resetForShade(q, resetNext, q.parity);
+    const bool quads = useQuads<W>(sc.any(), n);
+    QueueTally tl;
+    extendQueue<W, COUNT>(sc, q, rayIn, qm, chunkSource<P::kMany>(q.counters, kChunkExt, n, quads), quads, refill, tl);
     const int slots[5] = {kStatRays, kStatOverflow, kStatNodes, kStatTris, kStatExtRays};
-    const uint32_t vals[5] = {rays, overflow, cnt.nodes, cnt.tris, rays};
+    const uint32_t vals[5] = {tl.rays, tl.overflow, tl.cnt.nodes, tl.cnt.tris, tl.rays};
     blockFlush<5>(counters, slots, vals);
 }
 
@@ -1078,22 +1103,17 @@ EL_KERNEL(EL_WPE_SHADE) void k_wf_shade(P sc, RenderArgs a, WfState q, const flo
 }
 
 // Any-hit test of a shadow queue; an unoccluded entry adds its contribution
-// to its path's radiance (each path has at most one entry per queue, and the
-// two shadow queues are separate launches, so the update needs no atomics).
-// REC: a recording render's launch; visible queries set q.visBit in the
-// path's visibility word, and queries traced only for the record add nothing.
-template <int W, class P, bool REC = false>
-EL_KERNEL(EL_WPE_TRAV) void k_wf_shadow(P sc, WfState q, const float4* __restrict__ sh,
-                                        const uint32_t* countIn, uint32_t refill,
-                                        unsigned long long* counters) {
-    const DevScene& s0 = sc.any();
-    TraceCounters cnt{0, 0};
-    QueueMap qm;
-    qm.load(countIn);
-    const uint32_t n = qm.total();
-    uint32_t traced = 0, overflow = 0;
-    const WorkSource ws =
-        chunkSource<P::kMany>(q.counters, chunkShadow(q.parity, sh == q.shadowH ? 0 : 1), n, useQuads<W>(s0, n));
+// to its path's radiance (each path has at most one entry per queue, and of
+// two queues that are traced at once the light's is deferred, so the update
+// needs no atomics).  defer: every query writes its term (zero if blocked) to
+// pendP for the next shade or finalize.  REC: a recording render; visible
+// queries set visBit in the path's visibility word (atomically: the path's
+// other query may be in flight), and queries traced only for the record add
+// nothing.
+template <int W, class P, bool REC>
+__device__ __forceinline__ void shadowQueue(const P& sc, const WfState& q, const float4* __restrict__ sh,
+                                            const QueueMap& qm, const WorkSource& ws, bool quads, bool defer,
+                                            uint32_t visBit, uint32_t refill, QueueTally& tl) {
     const uint32_t segSize = q.segSize;
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr& bvh) {
@@ -1112,30 +1132,107 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_shadow(P sc, WfState q, const float4* __restric
         }
         return true;
     };
-    // point-light queries of a render with deferred terms: every query
-    // writes its term (zero if blocked) for the next shade or finalize
-    const bool defer = !REC && !P::kMany && q.deferP != 0u && sh == q.shadowP;
     auto store = [&](uint32_t i, const TraceResult& h, bool) {
-        if (h.tri >= 0 && !defer) return;
+        const bool blocked = h.tri >= 0;
+        if (blocked && !defer) return;
         const uint64_t e = qm.entry(i, segSize);
         const uint32_t slot = __float_as_uint(sh[3 * e].w);
+        const float4 C = sh[3 * e + 2];
+        if (REC && !blocked) atomicOr(&q.pathVis[slot], visBit);
         if (defer) {
-            const float4 C = sh[3 * e + 2];
-            q.pendP[slot] = h.tri >= 0 ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(C.x, C.y, C.z, 0.f);
+            q.pendP[slot] = blocked ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(C.x, C.y, C.z, 0.f);
             return;
         }
-        const float4 C = sh[3 * e + 2];
-        if constexpr (REC) {
-            q.pathVis[slot] |= q.visBit;
-            if (C.x == 0.f && C.y == 0.f && C.z == 0.f) return;   // traced only for the record
-        }
+        if (REC && C.x == 0.f && C.y == 0.f && C.z == 0.f) return;   // traced only for the record
         const float4 L = q.pathL[slot];
         q.pathL[slot] = make_float4(L.x + C.x, L.y + C.y, L.z + C.z, L.w);
     };
-    traceQueue<W, true, false, P::kMany>(s0, q.gstack, q.gthreads, ws, n, refill, load, store, cnt, traced, overflow);
+    traceQueue<W, true, false, P::kMany>(sc.any(), q.gstack, q.gthreads, ws, quads, refill, load, store, tl.cnt,
+                                         tl.rays, tl.overflow);
+}
+
+// One shadow queue of bounce parity q.parity (light: 0 HDRI, 1 point light).
+template <int W, class P, bool REC = false>
+EL_KERNEL(EL_WPE_TRAV) void k_wf_shadow(P sc, WfState q, int light, uint32_t refill, unsigned long long* counters) {
+    QueueMap qm;
+    qm.load(q.counters + qShadow(q.parity, light));
+    const uint32_t n = qm.total();
+    const bool quads = useQuads<W>(sc.any(), n);
+    QueueTally tl;
+    shadowQueue<W, P, REC>(sc, q, light ? q.shadowP : q.shadowH, qm,
+                           chunkSource<P::kMany>(q.counters, chunkShadow(q.parity, light), n, quads), quads, false,
+                           q.visBit << light, refill, tl);
     const int slots[1] = {kStatOverflow};
-    const uint32_t vals[1] = {overflow};
+    const uint32_t vals[1] = {tl.overflow};
     blockFlush<1>(counters, slots, vals);
+}
+
+// What follows a shade in one launch: the next bounce's closest hits (rayIn
+// null: none, the last bounce) and this bounce's two shadow queues.  The
+// three read only what the shade wrote and update nothing of each other's (the
+// light terms are deferred; the counters that the next shade appends to are
+// the other parity's), so the launch's waves are divided among them.  In small launches, that last about one ray's chain of visits, the
+// three chains run side by side without the streams, events and waits
+// between them that three launches need (8 to 25 us a bounce): a 64 x 48 frame
+// of one sample renders in 245 instead of 348 us, 256 x 256 of 16 samples in
+// 1.02 instead of 1.11 ms; from 2^21 paths on it makes no difference.
+template <int W, class P, bool REC = false>
+EL_KERNEL(EL_WPE_TRAV) void k_wf_trace(P sc, WfState q, const float4* __restrict__ rayIn, const uint32_t* countIn,
+                                       uint32_t* resetNext, uint32_t refill, unsigned long long* counters) {
+    if (rayIn) resetForShade(q, resetNext, q.parity ^ 1u);
+    const uint32_t* const cntH = q.counters + qShadow(q.parity, 0);
+    const uint32_t* const cntP = q.counters + qShadow(q.parity, 1);
+    uint32_t nE = 0, nH = 0, nP = 0;
+#pragma unroll
+    for (int k = 0; k < kXcds; k++) {
+        nE += rayIn ? countIn[k] : 0u;
+        nH += cntH[k];
+        nP += cntP[k];
+    }
+    const bool quads = useQuads<W>(sc.any(), nE + nH + nP);
+    // Every wave works on one queue: a wave for each chunk if they suffice,
+    // else in proportion to the rays (at least one), a closest hit counted as
+    // 3/4 (of 0.6 to 2 the fastest: 960 x 540 terrain of 4 samples 2.61 ms, 2.69
+    // with 1, 2.83 with 2; every wave going through all three queues, 2.86).
+    const uint32_t waves = gridWaves(), G = quads ? 16 : 64;
+    uint32_t wE = (nE + G - 1) / G, wH = (nH + G - 1) / G;
+    if (wE + wH + (nP + G - 1) / G > waves) {
+        const float e = 0.75f * (float)nE, share = (float)(waves - 3) / (e + (float)nH + (float)nP);
+        wE = nE ? 1u + (uint32_t)(e * share) : 0u;
+        wH = nH ? 1u + (uint32_t)((float)nH * share) : 0u;
+    }
+    const uint32_t w = __builtin_amdgcn_readfirstlane(gridWave());
+    const int kind = w < wE ? 0 : w < wE + wH ? 1 : 2;
+    QueueTally tl;
+    QueueMap qm;
+    if (kind == 0) {
+        qm.load(countIn);
+        extendQueue<W, false>(sc, q, rayIn, qm, chunkSource<P::kMany>(q.counters, kChunkExt, nE, quads, w, wE), quads,
+                              refill, tl);
+    } else {
+        const int light = kind - 1;
+        qm.load(light ? cntP : cntH);
+        const WorkSource ws =
+            chunkSource<P::kMany>(q.counters, chunkShadow(q.parity, light), light ? nP : nH, quads,
+                                  light ? w - wE - wH : w - wE, light ? waves - wE - wH : wH);
+        shadowQueue<W, P, REC>(sc, q, light ? q.shadowP : q.shadowH, qm, ws, quads, light != 0, q.visBit << light,
+                               refill, tl);
+        tl.rays = 0;
+    }
+    const int slots[3] = {kStatRays, kStatOverflow, kStatExtRays};
+    const uint32_t vals[3] = {tl.rays, tl.overflow, tl.rays};
+    blockFlush<3>(counters, slots, vals);
+}
+
+// A path's radiance once every launch is done: the last bounce's deferred
+// point-light term is added last.
+__device__ __forceinline__ float4 finishedL(const WfState& q, uint32_t slot) {
+    float4 Lf = q.pathL[slot];
+    if (Lf.w == kPendEnd) {
+        const float4 Pp = q.pendP[slot];
+        if (!isZero4(Pp)) Lf = make_float4(Lf.x + Pp.x, Lf.y + Pp.y, Lf.z + Pp.z, Lf.w);
+    }
+    return Lf;
 }
 
 // One thread per distinct pixel of the generation; slots j, j+npad, ... hold
@@ -1158,11 +1255,7 @@ EL_KERNEL(1) void k_wf_finalize(DevScene s, RenderArgs a, WfState q, float4* __r
         if (aov)
             for (int k = 0; k < 3; k++) A[k] = aov[3 * (uint64_t)idx + k];
         for (uint32_t slot = j; slot < a.genCount; slot += a.npad, sample++) {
-            float4 Lf = q.pathL[slot];
-            if (Lf.w == kPendEnd) {   // the last bounce's deferred point-light term, added last
-                const float4 Pp = q.pendP[slot];
-                if (!isZero4(Pp)) Lf = make_float4(Lf.x + Pp.x, Lf.y + Pp.y, Lf.z + Pp.z, Lf.w);
-            }
+            const float4 Lf = finishedL(q, slot);
             paths++;
             if (a.rec) a.rec[(uint64_t)sample * s.cam.xRes * s.cam.yRes + idx] = make_float4(Lf.x, Lf.y, Lf.z, 1.f);
             if (a.recVis) a.recVis[(uint64_t)sample * s.cam.xRes * s.cam.yRes + idx] = q.pathVis[slot];
@@ -1253,7 +1346,7 @@ EL_KERNEL(1) void k_bt_finalize(ManyScenes sc, const BatchSeg* __restrict__ segs
         float4 acc = s.accum[idx];
         uint32_t n = s.counts[idx];
         for (uint32_t slot = first; slot < end; slot += g.npad) {
-            const float4 Lf = q.pathL[slot];
+            const float4 Lf = finishedL(q, slot);
             paths++;
             const v3 L = clamp3(mk(Lf.x, Lf.y, Lf.z));
             if (anyNan(L)) continue;
@@ -1435,23 +1528,35 @@ hipError_t launchWfShade(const LaunchCfg& c, const DevScene& s, const RenderArgs
     return hipGetLastError();
 }
 
-hipError_t launchWfShadow(const LaunchCfg& c, const DevScene& s, const WfState& q, const float4* shadow,
-                          const uint32_t* countIn, uint32_t maxCount, unsigned long long* counters) {
+// The four instantiations of a shadow or trace kernel over one scene.
+#define EL_QUEUE_KERNEL(K, ...)                                                                                   \
+    do {                                                                                                          \
+        if (s.width == 4 && rec)                                                                                  \
+            hipLaunchKernelGGL((K<4, OneScene, true>), dim3(grid), dim3(c.block), lds, c.stream, __VA_ARGS__);     \
+        else if (s.width == 4)                                                                                    \
+            hipLaunchKernelGGL((K<4, OneScene>), dim3(grid), dim3(c.block), lds, c.stream, __VA_ARGS__);          \
+        else if (rec)                                                                                             \
+            hipLaunchKernelGGL((K<8, OneScene, true>), dim3(grid), dim3(c.block), lds, c.stream, __VA_ARGS__);     \
+        else                                                                                                      \
+            hipLaunchKernelGGL((K<8, OneScene>), dim3(grid), dim3(c.block), lds, c.stream, __VA_ARGS__);          \
+    } while (0)
+
+hipError_t launchWfShadow(const LaunchCfg& c, const DevScene& s, const WfState& q, int light, uint32_t maxCount,
+                          unsigned long long* counters) {
     uint32_t grid = queueGrid(c, s.width, maxCount);
     size_t lds = sizeof(int) * kShortStack * c.block;
-    const bool rec = q.visBit != 0;
-    if (s.width == 4 && rec)
-        hipLaunchKernelGGL((k_wf_shadow<4, OneScene, true>), dim3(grid), dim3(c.block), lds, c.stream, OneScene{s},
-                           q, shadow, countIn, c.refill, counters);
-    else if (s.width == 4)
-        hipLaunchKernelGGL((k_wf_shadow<4, OneScene>), dim3(grid), dim3(c.block), lds, c.stream, OneScene{s}, q,
-                           shadow, countIn, c.refill, counters);
-    else if (rec)
-        hipLaunchKernelGGL((k_wf_shadow<8, OneScene, true>), dim3(grid), dim3(c.block), lds, c.stream, OneScene{s},
-                           q, shadow, countIn, c.refill, counters);
-    else
-        hipLaunchKernelGGL((k_wf_shadow<8, OneScene>), dim3(grid), dim3(c.block), lds, c.stream, OneScene{s}, q,
-                           shadow, countIn, c.refill, counters);
+    const bool rec = q.pathVis != nullptr;
+    EL_QUEUE_KERNEL(k_wf_shadow, OneScene{s}, q, light, c.refill, counters);
+    return hipGetLastError();
+}
+
+hipError_t launchWfTrace(const LaunchCfg& c, const DevScene& s, const WfState& q, const float4* rayIn,
+                         const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount,
+                         unsigned long long* counters) {
+    uint32_t grid = queueGrid(c, s.width, (uint64_t)maxCount * (rayIn ? 3 : 2));
+    size_t lds = sizeof(int) * kShortStack * c.block;
+    const bool rec = q.pathVis != nullptr;
+    EL_QUEUE_KERNEL(k_wf_trace, OneScene{s}, q, rayIn, countIn, resetNext, c.refill, counters);
     return hipGetLastError();
 }
 
@@ -1496,17 +1601,30 @@ hipError_t launchBtShade(const LaunchCfg& c, const DevScene* scenes, const Rende
     return hipGetLastError();
 }
 
-hipError_t launchBtShadow(const LaunchCfg& c, const DevScene* scenes, int width, const WfState& q,
-                          const float4* shadow, const uint32_t* countIn, uint32_t maxCount,
-                          unsigned long long* counters) {
+hipError_t launchBtShadow(const LaunchCfg& c, const DevScene* scenes, int width, const WfState& q, int light,
+                          uint32_t maxCount, unsigned long long* counters) {
     uint32_t grid = queueGrid(c, width, maxCount);
     size_t lds = sizeof(int) * kShortStack * c.block;
     if (width == 4)
         hipLaunchKernelGGL((k_wf_shadow<4, ManyScenes>), dim3(grid), dim3(c.block), lds, c.stream,
-                           ManyScenes{scenes}, q, shadow, countIn, c.refill, counters);
+                           ManyScenes{scenes}, q, light, c.refill, counters);
     else
         hipLaunchKernelGGL((k_wf_shadow<8, ManyScenes>), dim3(grid), dim3(c.block), lds, c.stream,
-                           ManyScenes{scenes}, q, shadow, countIn, c.refill, counters);
+                           ManyScenes{scenes}, q, light, c.refill, counters);
+    return hipGetLastError();
+}
+
+hipError_t launchBtTrace(const LaunchCfg& c, const DevScene* scenes, int width, const WfState& q,
+                         const float4* rayIn, const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount,
+                         unsigned long long* counters) {
+    uint32_t grid = queueGrid(c, width, (uint64_t)maxCount * (rayIn ? 3 : 2));
+    size_t lds = sizeof(int) * kShortStack * c.block;
+    if (width == 4)
+        hipLaunchKernelGGL((k_wf_trace<4, ManyScenes>), dim3(grid), dim3(c.block), lds, c.stream,
+                           ManyScenes{scenes}, q, rayIn, countIn, resetNext, c.refill, counters);
+    else
+        hipLaunchKernelGGL((k_wf_trace<8, ManyScenes>), dim3(grid), dim3(c.block), lds, c.stream,
+                           ManyScenes{scenes}, q, rayIn, countIn, resetNext, c.refill, counters);
     return hipGetLastError();
 }
 

@@ -31,9 +31,9 @@ constexpr int kStatRays = 0, kStatVerts = 1, kStatPaths = 2, kStatOverflow = 3, 
               kStatExtRays = 6;   // rays of the closest-hit (extension) launches
 
 // Queue counters: kXcds per queue.  The shadow queues' counts come in two
-// sets by bounce parity (bounce b uses set b & 1): the shadow launches of
-// bounce b may run while the extension launch of bounce b + 1, which clears
-// the set bounce b + 1 fills, is running.
+// sets by bounce parity (bounce b uses set b & 1): the shadows of bounce b may
+// be traced in one launch with the extension of bounce b + 1, which clears
+// the set bounce b + 1 fills.
 constexpr int kQRay0 = 0, kQRay1 = kXcds, kQShadow = 2 * kXcds;
 __host__ __device__ constexpr int qShadow(int parity, int light) { return kQShadow + (2 * parity + light) * kXcds; }
 // Work-chunk counters of the traversal launches (extend, and per parity the
@@ -80,11 +80,10 @@ struct WfState {
     uint64_t* pathQuiet;    // per path slot: bounces whose HDRI number is NaN-prone (bit b, b < 64)
     float4* pathAov;        // 3 per path slot (normal, tangent, bitangent) or null
     uint32_t* pathVis;      // recording renders: visibility bits per path slot (RenderArgs::recVis), else null
-    float4* pendP;          // per path slot: the point-light term of the last shadow P launch (0: blocked), or
-                            // null; with deferP the launch writes it here instead of adding it to pathL, so
-                            // it can run beside the HDRI shadow launch, and shade / finalize add it in order
-    uint32_t deferP;        // this bounce's point-light terms go to pendP (shade marks, shadow P writes)
-    uint32_t visBit;        // shadow launches of a recording render: the bit a visible query sets
+    float4* pendP;          // per path slot: the point-light term of the last k_wf_trace (0: blocked), which
+                            // traces both shadow queues at once; shade / finalize add it after the HDRI term
+    uint32_t deferP;        // this bounce's point-light terms go to pendP (shade marks them)
+    uint32_t visBit;        // recording renders: the bit a visible HDRI query of this bounce sets (light: the next)
     uint32_t parity;        // bounce & 1: the shadow counter set of this bounce's launches
     uint32_t* counters;     // kQCounters: per-XCD segment counts of the queues, work-chunk counters
     uint32_t segSize;       // entries per XCD segment of a compacted queue
@@ -101,13 +100,6 @@ struct BatchSeg {
     uint64_t wStart;
     uint32_t finStart, pad;
 };
-
-// Global traversal-stack spill areas per context (gcap x maxThreads ints
-// each): launches on the main stream use the first; the shadow launches
-// that run beside the next extension use the second (HDRI) and third (point
-// light).  A spill slot is addressed by the thread's grid index, which
-// kernels running at once share.
-constexpr int kSpillSets = 3;
 
 struct LaunchCfg {
     hipStream_t stream;
@@ -147,9 +139,11 @@ hipError_t launchBtExtend(const LaunchCfg& c, const dev::DevScene* scenes, int w
 hipError_t launchBtShade(const LaunchCfg& c, const dev::DevScene* scenes, const RenderArgs& a, const WfState& q,
                          const float4* rayIn, const uint32_t* countIn, float4* rayOut, uint32_t* countOut,
                          uint32_t maxCount, unsigned long long* counters);
-hipError_t launchBtShadow(const LaunchCfg& c, const dev::DevScene* scenes, int width, const WfState& q,
-                          const float4* shadow, const uint32_t* countIn, uint32_t maxCount,
-                          unsigned long long* counters);
+hipError_t launchBtShadow(const LaunchCfg& c, const dev::DevScene* scenes, int width, const WfState& q, int light,
+                          uint32_t maxCount, unsigned long long* counters);
+hipError_t launchBtTrace(const LaunchCfg& c, const dev::DevScene* scenes, int width, const WfState& q,
+                         const float4* rayIn, const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount,
+                         unsigned long long* counters);
 hipError_t launchBtFinalize(const LaunchCfg& c, const dev::DevScene* scenes, const BatchSeg* segs, uint32_t nseg,
                             uint32_t finTotal, const WfState& q, unsigned long long* counters);
 hipError_t launchWfCamera(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, const WfState& q);
@@ -159,8 +153,13 @@ hipError_t launchWfExtend(const LaunchCfg& c, const dev::DevScene& s, const WfSt
 hipError_t launchWfShade(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, const WfState& q,
                          const float4* rayIn, const uint32_t* countIn, float4* rayOut, uint32_t* countOut,
                          uint32_t maxCount, unsigned long long* counters);
-hipError_t launchWfShadow(const LaunchCfg& c, const dev::DevScene& s, const WfState& q, const float4* shadow,
-                          const uint32_t* countIn, uint32_t maxCount, unsigned long long* counters);
+// Shadow queue `light` (0 HDRI, 1 point light) of bounce parity q.parity; its terms are added to the paths' radiance.
+hipError_t launchWfShadow(const LaunchCfg& c, const dev::DevScene& s, const WfState& q, int light, uint32_t maxCount,
+                          unsigned long long* counters);
+// Both shadow queues of q.parity (the light's terms go to q.pendP) and, with rayIn, the next bounce's closest hits.
+hipError_t launchWfTrace(const LaunchCfg& c, const dev::DevScene& s, const WfState& q, const float4* rayIn,
+                         const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount,
+                         unsigned long long* counters);
 hipError_t launchWfFinalize(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, const WfState& q,
                             float4* accum, uint32_t* counts, float4* aov, unsigned long long* counters);
 

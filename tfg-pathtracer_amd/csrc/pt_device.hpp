@@ -1063,9 +1063,9 @@ struct BvhPtr {
     const float4* tris;
 };
 
-// The items a wave traces: chunks of `chunk` items, either in turn (wave w of
-// `waves` takes the chunks w, w + waves, ...; without counters) or, with
-// waves == 0, handed out at run time.  Then chunk c belongs to share c % parts;
+// The items a wave traces: chunks of `chunk` items, either in turn (the chunks
+// first, first + waves, ...; without counters) or, with waves == 0, handed out
+// at run time.  Then chunk c belongs to share c % parts;
 // share x is counted by ctr[x * stride].  A wave draws from its home share
 // first, then from the others, so waves that meet cheap rays take more chunks
 // and a launch ends when the work does, not when its slowest wave's share
@@ -1079,22 +1079,22 @@ struct WorkSource {
     uint32_t* ctr;
     uint32_t n, chunk, stride, parts, home;
     uint32_t chunks;   // ceil(n / chunk)
+    uint32_t first;    // this wave's first chunk (waves != 0)
     uint32_t waves;    // 0: drawn from the counters
 };
 
 // A wave's place in its items (wave-uniform).
 struct WorkCursor {
-    uint32_t cursor, end, waveId;
+    uint32_t cursor = 0, end = 0, next;
     uint32_t tried = 0;      // narrow source: shares found drawn out
-    __device__ __forceinline__ WorkCursor(const WorkSource& ws, uint32_t wave)
-        : cursor(0), end(0), waveId(wave) {}
+    __device__ __forceinline__ WorkCursor(const WorkSource& ws) : next(ws.first) {}
     // The next chunk after [cursor, end) is used up; false: no items left.
     // The whole wave must call.
     template <bool WIDE>
     __device__ __forceinline__ bool draw(const WorkSource& ws) {
-        if (ws.waves) {   // chunks waveId, waveId + waves, ...
-            const uint32_t c = waveId;
-            waveId += ws.waves;
+        if (ws.waves) {
+            const uint32_t c = next;
+            next += ws.waves;
             return take(ws, c);
         }
         const uint32_t lane = __lane_id();
@@ -1146,8 +1146,7 @@ template <int W, bool ANY, bool COUNT, bool PER_RAY_BVH = false, class Load, cla
 __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st, const WorkSource& ws,
                                                uint32_t refill, Load&& load, Store&& store, TraceCounters& cnt,
                                                uint32_t& traced) {
-    const uint32_t waveId = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (ws.waves && waveId >= ws.chunks) return;   // no chunk for this wave
+    if (ws.waves && ws.first >= ws.chunks) return;   // no chunk for this wave
     BvhPtr bvh{(const uint4*)s.nodes, s.tris};
     // One BVH for the whole wave: its root node (visited first by every ray)
     // is read once into scalar registers, and a new ray is tested against it
@@ -1165,7 +1164,7 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
     }
     const uint32_t lane = __lane_id();
     const unsigned long long ltMask = lane ? (~0ull >> (64 - lane)) : 0ull;
-    WorkCursor wc(ws, waveId);
+    WorkCursor wc(ws);
     bool more = true;   // wave-uniform: items may remain
     bool live = false;
     uint32_t item = 0;
@@ -1428,12 +1427,11 @@ template <bool ANY, bool COUNT, bool PER_RAY_BVH = false, class Load, class Stor
 __device__ __forceinline__ void traceQuadRange(const DevScene& s, QuadStack& st, const WorkSource& ws,
                                                uint32_t refill, Load&& load, Store&& store, TraceCounters& cnt,
                                                uint32_t& traced) {
-    const uint32_t waveId = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (ws.waves && waveId >= ws.chunks) return;   // no chunk for this wave
+    if (ws.waves && ws.first >= ws.chunks) return;   // no chunk for this wave
     BvhPtr bvh{(const uint4*)s.nodes, s.tris};
     const uint32_t lane = __lane_id(), j = lane & 3u;
     const unsigned long long ltMask = (lane >> 2) ? (~0ull >> (64 - (lane & ~3u))) : 0ull;   // lanes of earlier quads
-    WorkCursor wc(ws, waveId);
+    WorkCursor wc(ws);
     bool more = true;   // wave-uniform: items may remain
     bool live = false;
     uint32_t item = 0;
