@@ -280,7 +280,7 @@ def adjoint_bench(steps=5, with_cpu=True):
     (196,608 texels).  One gradient = forward render (wavefront) + adjoint
     (path replay) of an L2 loss against a target rendered with perturbed
     parameters; parameter and texture uploads included.  The headline is the
-    O(pixels) replay (nothing of a path kept between forward and adjoint);
+    bounded-memory replay (nothing of a path kept between forward and adjoint);
     `recorded` is the same step with EL_FLAG_RECORD_PATHS (every vertex of
     every path kept by the forward render), reported beside it."""
     import eleven
@@ -325,8 +325,8 @@ def adjoint_bench(steps=5, with_cpu=True):
     out = {"metric": "adjoint grads/s", "value": legs[False]["value"], "unit": "grads/s",
            "config": "sphere field 61,442 tris, 128x128, 32 spp, depth 4, gradient of 65 materials x 6 "
                      "parameters + 256x256 RGB albedo texture (L2 loss)",
-           "method": "path replay, O(pixels): the adjoint re-walks every path from its RNG counters (traced "
-                     "once, replayed from the thread's own vertex slots); nothing of a path kept after the forward",
+           "method": "path replay, bounded memory: the adjoint walks the paths again from their RNG counters (traced "
+                     "once, then replayed bounce by bounce); nothing of a path kept after the forward",
            **{k: v for k, v in legs[False].items() if k not in ("value", "unit", "record_mem_mb")},
            "recorded": {**legs[True], "method": "EL_FLAG_RECORD_PATHS: the forward keeps every path's radiance "
                                                 "and vertices (O(pixels x spp x depth)); the adjoint traces nothing"}}

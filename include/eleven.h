@@ -54,9 +54,7 @@ extern "C" {
 #define EL_FLAG_RECORD_PATHS 8u /* opt-in, O(pixels x spp x depth) memory:
                                    keep each path's radiance (16 B per path,
                                    when that fits half of the free device
-                                   memory) so that el_adjoint walks every
-                                   path once instead of twice; needs a cleared
-                                   accumulation (the record covers this one
+                                   memory); needs a cleared accumulation (the record covers this one
                                    render; el_clear and el_set_camera release
                                    it).  Wavefront renders with max_depth
                                    <= 16 also keep every vertex's hit and
@@ -181,13 +179,14 @@ typedef struct {
     uint32_t node_stride;      /* bytes per BVH node as stored (64 or 96)    */
     uint32_t tri_stride;       /* bytes per triangle record as stored (48)   */
     double   adjoint_ms;       /* device time of the last el_adjoint         */
-    uint64_t adjoint_rays;     /* BVH queries of the last el_adjoint (primal
-                                  walk + replay)                             */
+    uint64_t adjoint_rays;     /* BVH queries of the last el_adjoint (its walk
+                                  of the paths; 0 from recorded vertices)    */
     uint64_t texels_8bit;      /* texels read from the 8-bit copies (textures
                                   from 8-bit files, not since set_texture)   */
     uint64_t adjoint_bytes;    /* device memory the last el_adjoint used beyond
-                                  the scene and the accumulation: per-thread
-                                  vertex cache, adjoint image, gradients     */
+                                  the scene, the accumulation and the render's
+                                  queues: a generation's hits and shadow
+                                  answers, adjoint image, gradients          */
     uint64_t record_bytes;     /* device memory held by the last recording
                                   render (EL_FLAG_RECORD_PATHS), 0 if none   */
 } el_stats;
@@ -270,16 +269,14 @@ int  el_set_camera(el_ctx* ctx, const el_camera* camera);
  * generateHitData (kernel.cu:103-104) - written to d_materials[M][6], and to
  * the texels of texture params->grad_texture, written to d_texture[h][w][3]
  * (may be NULL if grad_texture < 0).  d_image is [H][W][3] in the layout of
- * el_read_passes.  Each path is replayed from its RNG counters, nothing of a
- * path outlives the thread that replays it; a material whose albedo comes
- * from a texture gets no albedo gradient (its texels do, if selected).
- * Without a recording render each path is walked twice: once traced, for its
- * radiance, keeping the closest hits of its vertices in the walking thread's
- * own slots (a buffer of resident threads x depth x 16 B, independent of the
- * pixel and sample counts), then replayed from those without tracing.  If
- * the render used EL_FLAG_RECORD_PATHS, each path is walked once (the
- * recorded radiance gives the radiance after each vertex), from its recorded
- * vertices when the render kept them.  With `device_ptrs` != 0 the three
+ * el_read_passes.  The paths are replayed from their RNG counters, a bounded
+ * number at a time; a material whose albedo comes from a texture gets no
+ * albedo gradient (its texels do, if selected).  Without a recording render
+ * the paths of a generation are traced again first, which needs at most
+ * 2 GiB whatever the pixel and sample counts; the vertices that a wavefront
+ * EL_FLAG_RECORD_PATHS render kept are replayed without tracing.  A context
+ * whose wavefront queues are larger already (they are shared) allocates only
+ * the rest.  With `device_ptrs` != 0 the three
  * arrays are device pointers.  d_materials and d_texture may be NULL:
  * nothing is copied out, and the sums stay in the context for following
  * EL_ADJ_ACCUMULATE calls. */

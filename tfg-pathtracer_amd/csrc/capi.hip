@@ -143,7 +143,7 @@ struct el_ctx {
     bool recValid = false;         // dRec covers the whole accumulation
     uint64_t totalRays = 0, totalVerts = 0, totalPaths = 0;
     DevBuf aImage, aMat, aTex;     // adjoint image, FP64 material and FP32 texel gradients
-    DevBuf aCache;                 // el_adjoint: each grid thread's vertices of the path it replays
+    DevBuf aHits, aVis, aQueue;    // el_adjoint: a generation's hits and shadow answers, the replay's queue counts
     DevBuf aTarget, aLoss;         // el_residual_l2: target image, FP64 loss
     size_t residualPx = 0;         // aImage holds el_residual_l2's residual for this many pixels (0: none)
     el_stats stats{};
@@ -658,6 +658,56 @@ static int wfPlan(el_ctx* c, const LaunchCfg& lc, uint64_t total, uint64_t npad,
     return EL_OK;
 }
 
+// Camera rays and every bounce of the generation a.genCount: extend -> shade ->
+// both shadow queues.  Where the launches are small, the shadows of bounce b
+// and the extension of bounce b + 1 are one launch (launchWfTrace).  With
+// EL_FLAG_KERNEL_TIMES in `flags` the launches are timed by evPool's events
+// from `ev` on (`timed`: event index, kind 0 extend, 1 shade, 2 shadow).
+static int wfWalk(el_ctx* c, const LaunchCfg& lc, RenderArgs a, WfState q, uint32_t flags,
+                  std::vector<std::pair<size_t, int>>& timed, size_t& ev, unsigned long long* ctr) {
+    const bool apart = (flags & (EL_FLAG_SERIAL_SHADOWS | EL_FLAG_KERNEL_TIMES | EL_FLAG_COUNT_TRAVERSAL)) != 0;
+    const bool kernelTimes = (flags & EL_FLAG_KERNEL_TIMES) != 0;
+    auto launch = [&](int kind, auto&& f) -> hipError_t {   // one launch, timed if asked
+        if (!kernelTimes) return f();
+        hipEvent_t x0 = poolEvent(c, ev), x1 = poolEvent(c, ev + 1);
+        if (!x0 || !x1) return hipErrorOutOfMemory;
+        hipError_t e = hipEventRecord(x0, c->stream);
+        if (e == hipSuccess) e = f();
+        if (e == hipSuccess) e = hipEventRecord(x1, c->stream);
+        timed.push_back({ev, kind});
+        ev += 2;
+        return e;
+    };
+    EL_HIP(c, launchWfCamera(lc, c->ds, a, q));
+    bool extended = false;   // bounce b's closest hits were traced with the previous bounce's shadows
+    for (uint32_t b = 0; b < a.maxDepth; b++) {
+        const bool together = !apart && bounceTogether(a.genCount, b), more = b + 1 < a.maxDepth;
+        a.bounce = b;
+        q.parity = b & 1u;
+        q.deferP = together ? 1u : 0u;
+        q.visBit = q.pathVis ? 1u << (2 * b) : 0u;
+        const int cur = b & 1, nxt = cur ^ 1;
+        uint32_t* cntCur = q.counters + (cur ? kQRay1 : kQRay0);
+        uint32_t* cntNxt = q.counters + (nxt ? kQRay1 : kQRay0);
+        if (!extended)
+            EL_HIP(c, launch(0, [&] {
+                return launchWfExtend(lc, c->ds, q, q.ray[cur], cntCur, cntNxt, a.genCount,
+                                      (flags & EL_FLAG_COUNT_TRAVERSAL) != 0, ctr);
+            }));
+        EL_HIP(c, launch(1, [&] {
+            return launchWfShade(lc, c->ds, a, q, q.ray[cur], cntCur, q.ray[nxt], cntNxt, a.genCount, ctr);
+        }));
+        if (together) {
+            EL_HIP(c, launchWfTrace(lc, c->ds, q, more ? q.ray[nxt] : nullptr, cntNxt, cntCur, a.genCount, ctr));
+        } else {
+            for (int light = 0; light < 2; light++)
+                EL_HIP(c, launch(2, [&] { return launchWfShadow(lc, c->ds, q, light, a.genCount, ctr); }));
+        }
+        extended = together && more;
+    }
+    return EL_OK;
+}
+
 extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     if (!c || !p) return fail(c, EL_ERR_ARG, "null argument");
     if (!c->hasScene) return fail(c, EL_ERR_STATE, "no scene uploaded");
@@ -732,7 +782,6 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     double extendMs = 0, shadeMs = 0, shadowMs = 0;
     uint64_t extendLaunches = 0;
     EL_HIP(c, hipEventRecord(e0, c->stream));
-    const bool countTrav = (p->flags & 2u) != 0;
     unsigned long long h[kCounterWords];   // the launches' tallies, read back with the last sync
 
     if (p->mode == EL_MODE_PLAIN) {
@@ -760,49 +809,9 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
             a.genPixel = (uint32_t)(start % npad);
             a.genSample = (uint32_t)(start / npad);
             a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
-            EL_HIP(c, launchWfCamera(lc, c->ds, a, q));
-            // Per bounce b: extend -> shade -> both shadow queues.  Where the
-            // launches are small, the shadows of bounce b and the extension
-            // of bounce b + 1 are one launch (launchWfTrace).
-            const bool apart = (p->flags & (EL_FLAG_SERIAL_SHADOWS | EL_FLAG_KERNEL_TIMES | EL_FLAG_COUNT_TRAVERSAL)) != 0;
-            const bool kernelTimes = (p->flags & EL_FLAG_KERNEL_TIMES) != 0;
-            auto launch = [&](int kind, auto&& f) -> hipError_t {   // one launch, timed if asked
-                if (!kernelTimes) return f();
-                hipEvent_t x0 = poolEvent(c, ev), x1 = poolEvent(c, ev + 1);
-                if (!x0 || !x1) return hipErrorOutOfMemory;
-                hipError_t e = hipEventRecord(x0, c->stream);
-                if (e == hipSuccess) e = f();
-                if (e == hipSuccess) e = hipEventRecord(x1, c->stream);
-                timed.push_back({ev, kind});
-                ev += 2;
-                return e;
-            };
-            bool extended = false;   // bounce b's closest hits were traced with the previous bounce's shadows
-            for (uint32_t b = 0; b < depth; b++) {
-                const bool together = !apart && bounceTogether(a.genCount, b), more = b + 1 < depth;
-                a.bounce = b;
-                q.parity = b & 1u;
-                q.deferP = together ? 1u : 0u;
-                q.visBit = recordHits ? 1u << (2 * b) : 0u;
-                const int cur = b & 1, nxt = cur ^ 1;
-                uint32_t* cntCur = q.counters + (cur ? kQRay1 : kQRay0);
-                uint32_t* cntNxt = q.counters + (nxt ? kQRay1 : kQRay0);
-                if (!extended)
-                    EL_HIP(c, launch(0, [&] {
-                        return launchWfExtend(lc, c->ds, q, q.ray[cur], cntCur, cntNxt, a.genCount, countTrav, ctr);
-                    }));
-                EL_HIP(c, launch(1, [&] {
-                    return launchWfShade(lc, c->ds, a, q, q.ray[cur], cntCur, q.ray[nxt], cntNxt, a.genCount, ctr);
-                }));
-                if (together) {
-                    EL_HIP(c, launchWfTrace(lc, c->ds, q, more ? q.ray[nxt] : nullptr, cntNxt, cntCur, a.genCount, ctr));
-                } else {
-                    for (int light = 0; light < 2; light++)
-                        EL_HIP(c, launch(2, [&] { return launchWfShadow(lc, c->ds, q, light, a.genCount, ctr); }));
-                }
-                extended = together && more;
-                extendLaunches++;
-            }
+            rc = wfWalk(c, lc, a, q, p->flags, timed, ev, ctr);
+            if (rc) return rc;
+            extendLaunches += depth;
             EL_HIP(c, launchWfFinalize(lc, c->ds, a, q, c->dAccum.as<float4>(), c->dCounts.as<uint32_t>(), aovBuf,
                                        ctr));
         }
@@ -872,6 +881,11 @@ extern "C" int el_residual_l2(el_ctx* c, const float* target, double* loss) {
     return EL_OK;
 }
 
+// el_adjoint: device memory for a generation of paths (queues, path state and
+// records), so that its memory does not grow with the pixels and samples:
+// 4.4 M paths at depth 6, enough to fill the GPU.
+constexpr uint64_t kAdjointBytes = 2ull << 30;
+
 extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* dimage, float* dmat, float* dtex,
                           int devp) {
     const bool accumulate = (p && (p->flags & EL_ADJ_ACCUMULATE) != 0);
@@ -913,31 +927,80 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     EL_HIP(c, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, c->stream));
     LaunchCfg lc = cfgOf(c);
     if (p->block) lc.block = p->block;
+    const uint32_t depth = c->accDepth;
     RenderArgs a{};
     a.k0 = (uint32_t)c->accSeed;
     a.k1 = (uint32_t)(c->accSeed >> 32);
     a.scene = c->accScene;
-    a.maxDepth = c->accDepth;
+    a.maxDepth = depth;
     a.sample = 0;
     a.cull = 1;   // exact: a zero-throughput path adds neither radiance nor gradient
-    if (c->recValid && c->recHits) {
-        // the recording stopped no later than this replay does (it culled
-        // alike or not at all), so every vertex the replay reads is recorded
+    AdjArgs g{};
+    g.dimage = c->aImage.as<float>();
+    g.counts = c->dCounts.as<uint32_t>();
+    g.gradTex = gtex;
+    g.dmat = c->aMat.as<double>();
+    g.dtex = ntex ? c->aTex.as<float>() : nullptr;
+    g.ldsMats = M <= kAdjLdsMats ? (uint32_t)M : 0u;
+    // The paths are replayed a generation at a time.  Recorded ones (a
+    // wavefront EL_FLAG_RECORD_PATHS render) are traced no more: the
+    // recording stopped no earlier than the replay does.  Others are walked
+    // again here, recording the generation's hits and shadow answers.
+    const bool recorded = c->recValid && c->recHits;
+    const uint64_t npad = (uint64_t)((c->cam.x_res + 7) / 8) * ((c->cam.y_res + 7) / 8) * 64;
+    const uint64_t total = (uint64_t)c->sampleBase * npad;
+    if (npad >= (1ull << 31)) return fail(c, EL_ERR_RANGE, "frame too large for the adjoint");
+    uint64_t Q = 0;
+    WfState q{};
+    const uint64_t perPath = 6 * 32 + 60 + (recorded ? 0 : 16 * depth + 4);
+    uint64_t budget = kAdjointBytes;
+    if (c->wfCap < std::min(total, budget / perPath)) {   // buffers will grow: by a quarter of what is free, as a render's
+        size_t freeB = 0, totalB = 0;
+        EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
+        budget = std::min<uint64_t>(budget, std::max<uint64_t>(freeB / 4, c->wfCap * perPath));
+    }
+    const uint64_t cap = std::max<uint64_t>(1u << 16, budget / perPath);
+    int rc = wfPlan(c, lc, total, npad, cap, false, q, Q);
+    if (rc) return rc;
+    if (recorded) {
         a.recHits = c->dRecHits.as<float4>();
         a.recVis = c->dRecVis.as<uint32_t>();
         a.recStride = (uint64_t)c->sampleBase * npx;
+        g.rec = c->dRec.as<float4>();
+    } else {
+        EL_HIP(c, c->aHits.ensure(Q * depth * sizeof(float4)));
+        EL_HIP(c, c->aVis.ensure(Q * sizeof(uint32_t)));
+        a.recHits = c->aHits.as<float4>();
+        a.recStride = Q;
+        a.recBySlot = 1;
+        q.pathVis = c->aVis.as<uint32_t>();
     }
-    float4* cache = nullptr;
-    if (!c->recValid) {   // the primal walk keeps its vertices for the replay, per grid thread
-        EL_HIP(c, c->aCache.ensure((size_t)lc.maxThreads * c->accDepth * sizeof(float4)));
-        cache = c->aCache.as<float4>();
-    }
+    const size_t countBytes = (depth + 1) * kXcds * sizeof(uint32_t);
+    EL_HIP(c, c->aQueue.ensure(countBytes));
+    g.queueCount = c->aQueue.as<uint32_t>();
+    a.npad = (uint32_t)npad;
     hipEvent_t e0 = poolEvent(c, 0), e1 = poolEvent(c, 1);
     if (!e0 || !e1) return fail(c, EL_ERR_HIP, "event creation failed");
     EL_HIP(c, hipEventRecord(e0, c->stream));
-    EL_HIP(c, launchAdjoint(lc, c->ds, a, c->sampleBase, c->aImage.as<float>(), c->dCounts.as<uint32_t>(),
-                            c->recValid ? c->dRec.as<float4>() : nullptr, cache, gtex, c->aMat.as<double>(),
-                            ntex ? c->aTex.as<float>() : nullptr, ctr));
+    for (uint64_t start = 0; start < total; start += Q) {
+        a.genPixel = (uint32_t)(start % npad);
+        a.genSample = (uint32_t)(start / npad);
+        a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
+        if (!recorded) {
+            std::vector<std::pair<size_t, int>> timed;
+            size_t ev = 2;
+            rc = wfWalk(c, lc, a, q, 0, timed, ev, ctr);
+            if (rc) return rc;
+        }
+        EL_HIP(c, hipMemsetAsync(c->aQueue.p, 0, countBytes, c->stream));
+        // the walk's ray and shadow queues are free: the replay's go there
+        float4* const state[2] = {q.shadowH, q.shadowP};
+        for (uint32_t b = 0; b < depth; b++) {
+            a.bounce = b;
+            const int cur = b & 1, nxt = cur ^ 1;
+            EL_HIP(c, launchAdjBounce(lc, c->ds, a, q, g, q.ray[cur], state[cur], q.ray[nxt], state[nxt], ctr));
+        }
+    }
     EL_HIP(c, hipEventRecord(e1, c->stream));
     std::vector<double> hm(M * 6);
     EL_HIP(c, hipMemcpyAsync(hm.data(), c->aMat.p, M * 6 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -962,7 +1025,7 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     c->adjSumTex = gtex;
     c->stats.adjoint_ms = ms;
     c->stats.adjoint_rays = tally(h, kStatRays);
-    c->stats.adjoint_bytes = c->aCache.n + c->aImage.n + c->aMat.n + c->aTex.n;
+    c->stats.adjoint_bytes = (recorded ? 0 : c->aHits.n + c->aVis.n) + c->aQueue.n + c->aImage.n + c->aMat.n + c->aTex.n;
     if (tally(h, kStatOverflow)) return fail(c, EL_ERR_RANGE, "traversal stack overflow (gradients incomplete)");
     return EL_OK;
 }

@@ -60,12 +60,15 @@ struct RenderArgs {
     float4* rec;            // per (sample, pixel): the path's radiance before the clamp, or null
     // Wavefront renders that record, and adjoints that replay, path vertices
     // (one scene; all null otherwise): the closest hit (tri, t, u, v; tri -1:
-    // escaped) of vertex b of path (sample, pixel) at recHits[b * recStride +
-    // sample * pixels + pixel], and per path the shadow queries that found
-    // the light visible: bit 2b HDRI, bit 2b + 1 point light of vertex b.
+    // escaped) of vertex b of a path at recHits[b * recStride + key], and per
+    // path the shadow queries that found the light visible, recVis[key]: bit
+    // 2b HDRI, bit 2b + 1 point light of vertex b.  key: sample * pixels +
+    // pixel, or with recBySlot the path's slot (el_adjoint's own walk of a
+    // generation, whose recVis is WfState::pathVis).
     float4* recHits;
     uint32_t* recVis;
     uint64_t recStride;
+    uint32_t recBySlot;
 };
 
 struct WfState {
@@ -89,6 +92,20 @@ struct WfState {
     uint32_t segSize;       // entries per XCD segment of a compacted queue
     int* gstack;
     uint32_t gthreads;
+};
+
+// Materials whose gradient sums k_adj_bounce keeps in LDS (24 KB of FP64: two blocks of it still fit a CU).
+constexpr uint32_t kAdjLdsMats = 512;
+
+struct AdjArgs {
+    const float* dimage;      // dLoss/dI, [pixel][3]
+    const uint32_t* counts;   // accepted samples per pixel
+    const float4* rec;        // the paths' radiance by record key, or null: WfState::pathL (pendP) by slot
+    int gradTex;
+    double* dmat;             // [materials][6], added to
+    float* dtex;              // texels of gradTex, added to
+    uint32_t ldsMats;         // materials summed in LDS (all), or 0
+    uint32_t* queueCount;     // kXcds per bounce 0..maxDepth, zero at the start
 };
 
 // One scene's share of a batch generation: path slots [slotStart,
@@ -122,13 +139,12 @@ hipError_t launchPlain(const LaunchCfg& c, const dev::DevScene& s, const RenderA
 // store); *loss += sum (mean image - target)^2 (the caller zeroes it).
 hipError_t launchResidualL2(hipStream_t stream, const float4* accum, const uint32_t* counts, const float* target,
                             uint32_t npx, float* r, double* loss);
-// rec: the forward render's per-path radiance (EL_FLAG_RECORD_PATHS) or null:
-// then every path is walked once for its radiance, keeping its vertices in
-// `cache` (c.maxThreads * a.maxDepth float4, vertex i of grid thread g at
-// i * c.maxThreads + g), and replayed from there for the gradient.
-hipError_t launchAdjoint(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, uint32_t spp,
-                         const float* dimage, const uint32_t* counts, const float4* rec, float4* cache, int gradTex,
-                         double* dmat, float* dtex, unsigned long long* counters);
+// One bounce (a.bounce) of the adjoint of a.genCount recorded paths; rayIn and
+// stateIn (T and radiance so far, 2 float4 per entry) hold the paths that reach
+// it (unused at bounce 0), rayOut and stateOut take those that go on.
+hipError_t launchAdjBounce(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, const WfState& q,
+                           const AdjArgs& g, const float4* rayIn, const float4* stateIn, float4* rayOut,
+                           float4* stateOut, unsigned long long* counters);
 // Batch (many scenes, scene id per queue entry): scenes = device array of
 // DevScene; segs = the generation's segment table (device).
 hipError_t launchBtCamera(const LaunchCfg& c, const dev::DevScene* scenes, const BatchSeg* segs, uint32_t nseg,

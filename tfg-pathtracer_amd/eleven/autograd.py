@@ -14,11 +14,12 @@ sample and bounce), so forward calls with the same seed use common random
 numbers: finite differences of the loss are differences of the same paths.
 
 Memory: by default nothing of a path is kept between the forward and the
-backward; the adjoint recomputes every path from its RNG counters (path
-replay), so the device memory of a gradient is O(pixels).  record=True keeps
-each path's radiance and, in wavefront mode, every vertex (16 B per path +
-16 B per vertex: O(pixels x spp x depth)), which lets the adjoint walk each
-path once without tracing.
+backward; the adjoint recomputes the paths from their RNG counters (path
+replay), a bounded number of them at a time, so the device memory of a
+gradient is O(pixels) plus at most 2 GiB.  record=True keeps each path's
+radiance and, in wavefront mode, every vertex (16 B per path + 16 B per
+vertex: O(pixels x spp x depth)), which lets the adjoint replay the paths
+without tracing.
 """
 from __future__ import annotations
 

@@ -19,7 +19,8 @@ numbers measures).  The parameters and texels are clamped to their valid
 ranges after every Adam update.
 
 Memory: by default the adjoint replays each path from its RNG counters
-(O(pixels) device memory per view); record=True keeps the replayed render's
+(O(pixels) device memory per view and at most 2 GiB for the paths in
+flight); record=True keeps the replayed render's
 paths instead (EL_FLAG_RECORD_PATHS: O(pixels x spp x depth)).
 """
 from __future__ import annotations
