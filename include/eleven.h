@@ -54,9 +54,11 @@ extern "C" {
 #define EL_FLAG_RECORD_PATHS 8u /* opt-in, O(pixels x spp x depth) memory:
                                    keep each path's radiance (16 B per path,
                                    when that fits half of the free device
-                                   memory); needs a cleared accumulation (the record covers this one
-                                   render; el_clear and el_set_camera release
-                                   it).  Wavefront renders with max_depth
+                                   memory); needs a cleared accumulation (the
+                                   record covers this one render and ends with
+                                   el_clear and el_set_camera; its buffers go
+                                   back at the next render that does not
+                                   record).  Wavefront renders with max_depth
                                    <= 16 also keep every vertex's hit and
                                    shadow answers (16 B per vertex + 4 B per
                                    path, when that fits a quarter of the free

@@ -61,6 +61,112 @@ struct DevBuf {
 
 constexpr int kCounterWords = kXcds * kStatSlots;   // per-XCD copies of the tallies (kernels.hpp)
 
+// Host memory that the GPU writes results to on their way to the caller's
+// arrays, which are pageable: two chunks in turn, one filled by the GPU while
+// the other is copied out.
+struct Stage {
+    static constexpr size_t kChunk = 4u << 20;
+    unsigned char* p = nullptr;
+    size_t n = 0;   // bytes of a chunk
+    bool two = false;
+    hipEvent_t filled[2] = {nullptr, nullptr};
+    unsigned long long* tallies = nullptr;   // kCounterWords
+    Stage() = default;
+    Stage(const Stage&) = delete;
+    Stage& operator=(const Stage&) = delete;
+    ~Stage() {
+        if (p) (void)hipHostFree(p);
+        if (tallies) (void)hipHostFree(tallies);
+        for (auto e : filled)
+            if (e) (void)hipEventDestroy(e);
+    }
+    hipError_t ensureTallies() {
+        if (tallies) return hipSuccess;
+        return hipHostMalloc((void**)&tallies, sizeof(unsigned long long) * kCounterWords, hipHostMallocDefault);
+    }
+    hipError_t ensure(size_t bytes) {
+        const size_t want = std::min(kChunk, std::max<size_t>(64u << 10, bytes));
+        const bool both = bytes > kChunk;
+        for (auto& e : filled)
+            if (!e)
+                if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming); r != hipSuccess) return r;
+        if (p && want <= n && both <= two) return hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+        const hipError_t r = hipHostMalloc((void**)&p, want * (both ? 2 : 1), hipHostMallocDefault);
+        if (r != hipSuccess) return r;
+        n = want;
+        two = both;
+        return hipSuccess;
+    }
+};
+
+// Takes `items` items of `itemBytes` through the stage: fill(first, n, chunk)
+// enqueues on `stream` what writes the items [first, first + n) to a chunk,
+// copy(first, n, chunk, i0, i1) copies the chunk's items [i0, i1) out, on up
+// to 8 host threads (a thread per MB: a frame's copy is bound by the page
+// faults of the caller's fresh arrays, which one thread takes one at a time).
+template <class Fill, class Copy>
+hipError_t stageOut(Stage& st, hipStream_t stream, size_t items, size_t itemBytes, Fill&& fill, Copy&& copy) {
+    if (!items) return hipSuccess;
+    hipError_t e = st.ensure(items * itemBytes);
+    if (e != hipSuccess) return e;
+    const size_t per = st.n / itemBytes, chunks = (items + per - 1) / per;
+    auto count = [&](size_t k) { return std::min(per, items - k * per); };
+    auto chunk = [&](size_t k) { return st.p + (k & 1) * st.n; };
+    auto issue = [&](size_t k) -> hipError_t {
+        hipError_t r = fill(k * per, count(k), chunk(k));
+        return r == hipSuccess ? hipEventRecord(st.filled[k & 1], stream) : r;
+    };
+    std::atomic<size_t> ready{0}, done{0};   // chunks filled; thread-chunks copied
+    std::atomic<bool> failed{false};         // no further chunk gets ready
+    std::atomic<size_t> team{0};             // threads that share a chunk, once known
+    auto part = [&](size_t k, size_t t) {
+        const size_t n = count(k), T = team.load(std::memory_order_relaxed);
+        copy(k * per, n, chunk(k), n * t / T, n * (t + 1) / T);
+    };
+    auto work = [&](size_t t) {
+        while (!team.load(std::memory_order_acquire)) std::this_thread::yield();
+        for (size_t k = 0; k < chunks; k++) {
+            while (ready.load(std::memory_order_acquire) <= k) {
+                if (failed.load(std::memory_order_acquire)) return;
+                std::this_thread::yield();
+            }
+            part(k, t);
+            done.fetch_add(1, std::memory_order_release);
+        }
+    };
+    const size_t wantThreads = std::min<size_t>({(size_t)hostThreads(), 8, items * itemBytes >> 20});
+    std::vector<std::thread> threads;
+    for (size_t k = 0; k < std::min<size_t>(chunks, 2) && e == hipSuccess; k++) e = issue(k);
+    if (e == hipSuccess) {
+        try {
+            threads.reserve(wantThreads);
+            for (size_t t = 1; t < wantThreads; t++) threads.emplace_back(work, t);
+        } catch (...) {   // fewer threads share the work
+        }
+    }
+    const size_t T = threads.size() + 1;
+    team.store(T, std::memory_order_release);
+    for (size_t k = 0; k < chunks && e == hipSuccess; k++) {
+        e = hipEventSynchronize(st.filled[k & 1]);
+        if (e != hipSuccess) break;
+        ready.store(k + 1, std::memory_order_release);
+        part(k, 0);
+        if (k + 2 < chunks) {   // the chunk is filled again once every thread has copied its share
+            while (done.load(std::memory_order_acquire) < (k + 1) * (T - 1)) std::this_thread::yield();
+            e = issue(k + 2);
+        }
+    }
+    if (e != hipSuccess) failed.store(true, std::memory_order_release);
+    for (auto& t : threads) t.join();
+    // an error leaves nothing in flight that writes the stage
+    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
+    return e;
+}
+
+
 // Sum of the per-XCD copies of tally `slot`.
 inline unsigned long long tally(const unsigned long long* h, int slot) {
     unsigned long long s = 0;
@@ -134,6 +240,7 @@ struct el_ctx {
     uint32_t sampleBase = 0;
     uint64_t accSeed = 0;          // seed / depth / RNG scene word of the renders in the accumulation
     uint32_t accDepth = 0, accScene = 0;
+    bool accPending = false;       // the accumulation is empty, but its buffers are not cleared
     bool accMixed = false;         // renders since el_clear used different seeds or depths
     DevBuf dRec;                   // per (sample, pixel) path radiance of a recorded render
     DevBuf dRecHits, dRecVis, wVis;  // its vertices (wavefront recordings: RenderArgs::recHits / recVis)
@@ -148,6 +255,7 @@ struct el_ctx {
     size_t residualPx = 0;         // aImage holds el_residual_l2's residual for this many pixels (0: none)
     el_stats stats{};
     bool aovOn = false;
+    std::shared_ptr<Stage> stage;   // one for all scenes of a batch
 
     std::vector<hipEvent_t> evPool;
 };
@@ -173,6 +281,13 @@ static hipError_t upload(DevBuf& b, const void* src, size_t bytes, hipStream_t s
     return e;
 }
 
+// The tallies to c->stage->tallies; waits for the stream.
+static hipError_t readTallies(el_ctx* c, const unsigned long long* ctr) {
+    const hipError_t e = hipMemcpyAsync(c->stage->tallies, ctr, sizeof(unsigned long long) * kCounterWords,
+                                        hipMemcpyDeviceToHost, c->stream);
+    return e == hipSuccess ? hipStreamSynchronize(c->stream) : e;
+}
+
 static LaunchCfg cfgOf(el_ctx* c) {
     LaunchCfg l;
     l.stream = c->stream;
@@ -184,18 +299,7 @@ static LaunchCfg cfgOf(el_ctx* c) {
     return l;
 }
 
-extern "C" {
-
-int el_device_count(int* out) {
-    if (!out) return EL_ERR_ARG;
-    int n = 0;
-    hipError_t e = hipGetDeviceCount(&n);
-    if (e != hipSuccess) n = 0;
-    *out = n;
-    return EL_OK;
-}
-
-int el_create(el_ctx** out, int device) {
+static int createContext(el_ctx** out, int device, std::shared_ptr<Stage> stage) {
     if (!out) return EL_ERR_ARG;
     *out = nullptr;
     std::unique_ptr<el_ctx> c(new el_ctx());
@@ -212,9 +316,24 @@ int el_create(el_ctx** out, int device) {
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (c->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
     if (scratchAddress(device, &c->scratch) != hipSuccess) return EL_ERR_HIP;
+    if (stage->ensureTallies() != hipSuccess) return EL_ERR_HIP;
+    c->stage = std::move(stage);
     *out = c.release();
     return EL_OK;
 }
+
+extern "C" {
+
+int el_device_count(int* out) {
+    if (!out) return EL_ERR_ARG;
+    int n = 0;
+    hipError_t e = hipGetDeviceCount(&n);
+    if (e != hipSuccess) n = 0;
+    *out = n;
+    return EL_OK;
+}
+
+int el_create(el_ctx** out, int device) { return createContext(out, device, std::make_shared<Stage>()); }
 
 void el_destroy(el_ctx* c) {
     if (!c) return;
@@ -345,28 +464,36 @@ static int uploadBvh(el_ctx* c, int width) {
     return EL_OK;
 }
 
-// Releases the buffers of a recording render (EL_FLAG_RECORD_PATHS), which
-// cover only the accumulation they were recorded into.
+// Gives back the buffers of a recording render (EL_FLAG_RECORD_PATHS), which
+// cover only the accumulation they were recorded into: at the next render that
+// does not record (recording steps in a row keep them) and with the scene.
 static void releaseRecord(el_ctx* c) {
     c->dRec.release();
     c->dRecHits.release();
     c->dRecVis.release();
     c->wVis.release();
-    c->recValid = false;
-    c->recHits = false;
 }
 
+// Empties the accumulation.  Its sums and counts are not written here: the next
+// wavefront render starts them from zero (RenderArgs::fresh), and whatever
+// else reads them first clears them (clearPending).
 static int clearAccum(el_ctx* c) {
-    size_t npx = (size_t)c->cam.x_res * c->cam.y_res;
-    EL_HIP(c, hipMemsetAsync(c->dAccum.p, 0, npx * sizeof(float4), c->stream));
-    EL_HIP(c, hipMemsetAsync(c->dCounts.p, 0, npx * sizeof(uint32_t), c->stream));
     if (c->dAov.p) EL_HIP(c, hipMemsetAsync(c->dAov.p, 0, c->dAov.n, c->stream));
+    c->accPending = true;
     c->sampleBase = 0;
     c->accMixed = false;
-    releaseRecord(c);
+    c->recValid = false;
+    c->recHits = false;
     c->totalRays = c->totalVerts = c->totalPaths = 0;
-    EL_HIP(c, hipStreamSynchronize(c->stream));
     return EL_OK;
+}
+static hipError_t clearPending(el_ctx* c) {
+    if (!c->accPending) return hipSuccess;
+    const size_t npx = (size_t)c->cam.x_res * c->cam.y_res;
+    hipError_t e = hipMemsetAsync(c->dAccum.p, 0, npx * sizeof(float4), c->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(c->dCounts.p, 0, npx * sizeof(uint32_t), c->stream);
+    if (e == hipSuccess) c->accPending = false;
+    return e;
 }
 
 extern "C" {
@@ -389,6 +516,7 @@ int el_upload_scene(el_ctx* c, const el_scene_view* v) {
     c->hasScene = false;
     c->adjSumValid = false;
     c->residualPx = 0;
+    releaseRecord(c);
     c->ntri = v->tri_count;
     c->cam = v->camera;
 
@@ -532,6 +660,7 @@ int el_upload_scene(el_ctx* c, const el_scene_view* v) {
     EL_HIP(c, launchEnvTable(c->stream, s, c->dEnvTab.as<float4>()));
     rc = clearAccum(c);
     if (rc) return rc;
+    EL_HIP(c, hipStreamSynchronize(c->stream));   // the uploads: a batch uses the scene on another stream
     c->hasScene = true;
     return EL_OK;
 }
@@ -615,6 +744,7 @@ static int wfPlan(el_ctx* c, const LaunchCfg& lc, uint64_t total, uint64_t npad,
     // memory holds (~216 B of queue and path state per path), so a
     // 1080p x 64 spp frame runs as a single generation.
     Q = queueCap;
+    if (!Q && total <= c->wfCap && (!aov || c->wAov.n >= total * 48)) Q = total;   // held already
     if (!Q) {
         size_t freeB = 0, totalB = 0;
         EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
@@ -678,7 +808,7 @@ static int wfWalk(el_ctx* c, const LaunchCfg& lc, RenderArgs a, WfState q, uint3
         ev += 2;
         return e;
     };
-    EL_HIP(c, launchWfCamera(lc, c->ds, a, q));
+    EL_HIP(c, launchWfCamera(lc, c->ds, a, q, ctr));
     bool extended = false;   // bounce b's closest hits were traced with the previous bounce's shadows
     for (uint32_t b = 0; b < a.maxDepth; b++) {
         const bool together = !apart && bounceTogether(a.genCount, b), more = b + 1 < a.maxDepth;
@@ -735,7 +865,10 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     c->aovOn = c->aovOn || aov;
     float4* aovBuf = aov ? c->dAov.as<float4>() : nullptr;
     unsigned long long* ctr = c->dCounters.as<unsigned long long>();
-    EL_HIP(c, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, c->stream));
+    if (p->mode == EL_MODE_PLAIN) {
+        EL_HIP(c, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, c->stream));
+        EL_HIP(c, clearPending(c));
+    }
     LaunchCfg lc = cfgOf(c);
     RenderArgs a{};
     a.k0 = (uint32_t)p->seed;
@@ -746,33 +879,37 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     a.cull = (p->flags & EL_FLAG_NO_CULL) ? 0u : 1u;
     bool record = (p->flags & EL_FLAG_RECORD_PATHS) != 0;
     bool recordHits = false;
+    if (!record && c->dRec.p) releaseRecord(c);
     if (record) {
         if (c->sampleBase != 0) return fail(c, EL_ERR_STATE, "EL_FLAG_RECORD_PATHS needs a cleared accumulation");
         // the radiance record (16 B per path) is kept only when it fits half
-        // of the free device memory; otherwise el_adjoint replays without it
-        size_t freeB = 0, totalB = 0;
-        EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
-        const size_t recBytes = (size_t)p->spp * npx * sizeof(float4);
-        record = recBytes <= c->dRec.n || recBytes <= freeB / 2;
-    }
-    if (record) {
-        EL_HIP(c, c->dRec.ensure((size_t)p->spp * npx * sizeof(float4)));
-        a.rec = c->dRec.as<float4>();
+        // of the free device memory; otherwise el_adjoint replays without it.
         // Wavefront renders also keep every vertex's hit and shadow answers
         // (16 B per vertex + 4 B per path) when they fit a quarter of the
         // free memory, so that el_adjoint replays without tracing.
-        if (p->mode != EL_MODE_PLAIN && depth <= (uint32_t)dev::kAdjMaxDepthHost) {
+        const size_t recBytes = (size_t)p->spp * npx * sizeof(float4), hitBytes = recBytes * depth;
+        const bool wantHits = p->mode != EL_MODE_PLAIN && depth <= (uint32_t)dev::kAdjMaxDepthHost;
+        auto holds = [](const DevBuf& b, size_t n) { return b.p && n <= b.n && n >= b.n / 4; };
+        // buffers of another size go back first: the rules are about the memory without them
+        if (!holds(c->dRec, recBytes) || (wantHits && !holds(c->dRecHits, hitBytes))) {
+            releaseRecord(c);
             size_t freeB = 0, totalB = 0;
             EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
-            const size_t hitBytes = (size_t)p->spp * npx * depth * sizeof(float4);
-            recordHits = hitBytes <= c->dRecHits.n || hitBytes <= freeB / 4;
-            if (recordHits) {
-                EL_HIP(c, c->dRecHits.ensure(hitBytes));
-                EL_HIP(c, c->dRecVis.ensure((size_t)p->spp * npx * sizeof(uint32_t)));
-                a.recHits = c->dRecHits.as<float4>();
-                a.recVis = c->dRecVis.as<uint32_t>();
-                a.recStride = (uint64_t)p->spp * npx;
-            }
+            record = recBytes <= freeB / 2;
+            recordHits = record && wantHits && hitBytes <= (freeB - recBytes) / 4;
+        } else {
+            recordHits = wantHits;
+        }
+        if (record) {
+            EL_HIP(c, c->dRec.ensure(recBytes));
+            a.rec = c->dRec.as<float4>();
+        }
+        if (recordHits) {
+            EL_HIP(c, c->dRecHits.ensure(hitBytes));
+            EL_HIP(c, c->dRecVis.ensure((size_t)p->spp * npx * sizeof(uint32_t)));
+            a.recHits = c->dRecHits.as<float4>();
+            a.recVis = c->dRecVis.as<uint32_t>();
+            a.recStride = (uint64_t)p->spp * npx;
         }
     }
     c->recValid = false;
@@ -782,7 +919,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     double extendMs = 0, shadeMs = 0, shadowMs = 0;
     uint64_t extendLaunches = 0;
     EL_HIP(c, hipEventRecord(e0, c->stream));
-    unsigned long long h[kCounterWords];   // the launches' tallies, read back with the last sync
+    unsigned long long* const h = c->stage->tallies;   // the launches' tallies, read back with the last sync
 
     if (p->mode == EL_MODE_PLAIN) {
         for (uint32_t s = 0; s < p->spp; s++) {
@@ -809,15 +946,17 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
             a.genPixel = (uint32_t)(start % npad);
             a.genSample = (uint32_t)(start / npad);
             a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
+            a.fresh = c->accPending ? 1u : 0u;
+            a.zeroTallies = start == 0 ? 1u : 0u;
             rc = wfWalk(c, lc, a, q, p->flags, timed, ev, ctr);
             if (rc) return rc;
             extendLaunches += depth;
             EL_HIP(c, launchWfFinalize(lc, c->ds, a, q, c->dAccum.as<float4>(), c->dCounts.as<uint32_t>(), aovBuf,
                                        ctr));
         }
+        c->accPending = false;
         EL_HIP(c, hipEventRecord(e1, c->stream));
-        EL_HIP(c, hipMemcpyAsync(h, ctr, sizeof h, hipMemcpyDeviceToHost, c->stream));
-        EL_HIP(c, hipStreamSynchronize(c->stream));   // the tallies and every event
+        EL_HIP(c, readTallies(c, ctr));   // the tallies and every event
         for (auto& t : timed) {
             float ms = 0;
             EL_HIP(c, hipEventElapsedTime(&ms, c->evPool[t.first], c->evPool[t.first + 1]));
@@ -826,8 +965,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     }
     if (p->mode == EL_MODE_PLAIN) {
         EL_HIP(c, hipEventRecord(e1, c->stream));
-        EL_HIP(c, hipMemcpyAsync(h, ctr, sizeof h, hipMemcpyDeviceToHost, c->stream));
-        EL_HIP(c, hipStreamSynchronize(c->stream));
+        EL_HIP(c, readTallies(c, ctr));
     }
     float totalMs = 0;
     EL_HIP(c, hipEventElapsedTime(&totalMs, e0, e1));
@@ -1004,13 +1142,20 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     EL_HIP(c, hipEventRecord(e1, c->stream));
     std::vector<double> hm(M * 6);
     EL_HIP(c, hipMemcpyAsync(hm.data(), c->aMat.p, M * 6 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    unsigned long long h[kCounterWords];
-    EL_HIP(c, hipMemcpyAsync(h, ctr, sizeof h, hipMemcpyDeviceToHost, c->stream));
-    // the texel gradients with the same sync
-    if (ntex && dtex)
-        EL_HIP(c, hipMemcpyAsync(dtex, c->aTex.p, ntex * sizeof(float),
-                                 devp ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, c->stream));
-    EL_HIP(c, hipStreamSynchronize(c->stream));
+    const unsigned long long* const h = c->stage->tallies;
+    if (ntex && dtex && devp)
+        EL_HIP(c, hipMemcpyAsync(dtex, c->aTex.p, ntex * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
+    if (ntex && dtex && !devp)
+        EL_HIP(c, stageOut(
+                      *c->stage, c->stream, ntex, sizeof(float),
+                      [&](size_t first, size_t n, unsigned char* chunk) {
+                          return hipMemcpyAsync(chunk, c->aTex.as<float>() + first, n * sizeof(float),
+                                                hipMemcpyDeviceToHost, c->stream);
+                      },
+                      [&](size_t first, size_t, const unsigned char* chunk, size_t i0, size_t i1) {
+                          std::memcpy(dtex + first + i0, (const float*)chunk + i0, (i1 - i0) * sizeof(float));
+                      }));
+    EL_HIP(c, readTallies(c, ctr));
     float ms = 0;
     EL_HIP(c, hipEventElapsedTime(&ms, e0, e1));
     std::vector<float> fm(M * 6);
@@ -1030,6 +1175,28 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     return EL_OK;
 }
 
+// The mean image of sums[i * stride] over the accepted samples, and their
+// counts, to host arrays (either may be null): divided on the GPU, which writes
+// it to the stage.  A 1920 x 1080 frame takes 1.9 ms, of which a caller's fresh
+// arrays cost 1.6; sums and counts copied to pageable memory and divided by the
+// host took 12.9.
+static hipError_t readMean(el_ctx* c, const float4* sums, uint32_t stride, size_t npx, float* rgba,
+                           uint32_t* samples) {
+    if (hipError_t e = clearPending(c); e != hipSuccess) return e;
+    const size_t nR = rgba ? sizeof(float4) : 0, nS = samples ? sizeof(uint32_t) : 0;
+    // a chunk of n pixels: n float4, then n counts
+    return stageOut(
+        *c->stage, c->stream, npx, nR + nS,
+        [&](size_t first, size_t n, unsigned char* chunk) {
+            return launchResolve(c->stream, sums, stride, c->dCounts.as<uint32_t>(), (uint32_t)first, (uint32_t)n,
+                                 nR ? (float4*)chunk : nullptr, nS ? (uint32_t*)(chunk + n * nR) : nullptr);
+        },
+        [&](size_t first, size_t n, const unsigned char* chunk, size_t i0, size_t i1) {
+            if (nR) std::memcpy(rgba + 4 * (first + i0), chunk + i0 * nR, (i1 - i0) * nR);
+            if (nS) std::memcpy(samples + first + i0, chunk + n * nR + i0 * nS, (i1 - i0) * nS);
+        });
+}
+
 extern "C" {
 
 int el_read_passes(el_ctx* c, float* rgba, uint32_t* samples, uint64_t* rays, uint64_t* vertices) {
@@ -1037,18 +1204,7 @@ int el_read_passes(el_ctx* c, float* rgba, uint32_t* samples, uint64_t* rays, ui
     if (!c->hasScene) return fail(c, EL_ERR_STATE, "no scene uploaded");
     EL_HIP(c, hipSetDevice(c->device));
     size_t npx = (size_t)c->cam.x_res * c->cam.y_res;
-    std::vector<float> acc(npx * 4);
-    std::vector<uint32_t> cnt(npx);
-    EL_HIP(c, hipMemcpyAsync(acc.data(), c->dAccum.p, npx * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    EL_HIP(c, hipMemcpyAsync(cnt.data(), c->dCounts.p, npx * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-    EL_HIP(c, hipStreamSynchronize(c->stream));
-    if (rgba)
-        for (size_t i = 0; i < npx; i++) {
-            float n = (float)cnt[i];
-            for (int k = 0; k < 3; k++) rgba[4 * i + k] = cnt[i] ? acc[4 * i + k] / n : 0.f;
-            rgba[4 * i + 3] = 1.f;
-        }
-    if (samples) std::memcpy(samples, cnt.data(), npx * sizeof(uint32_t));
+    if (rgba || samples) EL_HIP(c, readMean(c, c->dAccum.as<float4>(), 1, npx, rgba, samples));
     if (rays) *rays = c->totalRays;
     if (vertices) *vertices = c->totalVerts;
     return EL_OK;
@@ -1062,16 +1218,7 @@ int el_read_aov(el_ctx* c, int pass, float* rgba) {
     if (!c->dAov.p) return fail(c, EL_ERR_STATE, "no AOV rendered (EL_FLAG_AOV)");
     EL_HIP(c, hipSetDevice(c->device));
     size_t npx = (size_t)c->cam.x_res * c->cam.y_res;
-    std::vector<float> a(npx * 12);
-    std::vector<uint32_t> cnt(npx);
-    EL_HIP(c, hipMemcpyAsync(a.data(), c->dAov.p, npx * 48, hipMemcpyDeviceToHost, c->stream));
-    EL_HIP(c, hipMemcpyAsync(cnt.data(), c->dCounts.p, npx * 4, hipMemcpyDeviceToHost, c->stream));
-    EL_HIP(c, hipStreamSynchronize(c->stream));
-    int k = pass - EL_PASS_NORMAL;
-    for (size_t i = 0; i < npx; i++) {
-        for (int j = 0; j < 3; j++) rgba[4 * i + j] = cnt[i] ? a[12 * i + 4 * k + j] / (float)cnt[i] : 0.f;
-        rgba[4 * i + 3] = 1.f;
-    }
+    EL_HIP(c, readMean(c, c->dAov.as<float4>() + (pass - EL_PASS_NORMAL), 3, npx, rgba, nullptr));
     return EL_OK;
 }
 
@@ -1117,6 +1264,10 @@ int el_set_texture(el_ctx* c, int32_t id, const float* rgb) {
 }  // extern "C"
 
 // ---------------------------------------------------------------- queries --
+// Host queries of up to this many rays (160 KB of rays and answers) leave the
+// copies out: 1000 rays take 47 instead of 95 us.
+constexpr uint32_t kDirectRays = 4096;
+
 static int traceCommon(el_ctx* c, const el_ray* rays, const float* tmax, uint32_t n, int32_t* tri, float* t,
                        float* uv, uint8_t* occ, int devp, bool any, bool count, uint64_t* nodes, uint64_t* tris) {
     if (!c || !rays) return fail(c, EL_ERR_ARG, "null argument");
@@ -1131,51 +1282,83 @@ static int traceCommon(el_ctx* c, const el_ray* rays, const float* tmax, uint32_
     float* dT = t;
     float* dUV = uv;
     uint8_t* dOcc = occ;
-    if (!devp) {
-        EL_HIP(c, upload(c->tRays, rays, (size_t)n * sizeof(el_ray), c->stream));
+    Stage& st = *c->stage;
+    // A short host query (a pick) goes through the stage: the kernel reads the
+    // rays from it and writes the answers to it, without a copy each way.
+    const bool direct = !devp && !count && n <= kDirectRays;
+    const size_t rayBytes = (size_t)n * sizeof(el_ray);
+    if (direct) {
+        EL_HIP(c, st.ensure(kDirectRays * (sizeof(el_ray) + 16)));
+        std::memcpy(st.p, rays, rayBytes);
+        dR = (const float*)st.p;
+        unsigned char* out = st.p + rayBytes;
+        if (any) {
+            std::memcpy(out, tmax, (size_t)n * 4);
+            dTm = (const float*)out;
+            dOcc = out + (size_t)n * 4;
+        } else {
+            dTri = (int32_t*)out;
+            dT = (float*)(out + (size_t)n * 4);
+            if (uv) dUV = (float*)(out + (size_t)n * 8);
+        }
+    } else if (!devp) {
+        EL_HIP(c, upload(c->tRays, rays, rayBytes, c->stream));
         dR = c->tRays.as<float>();
         if (any) {
             EL_HIP(c, upload(c->tTmax, tmax, (size_t)n * 4, c->stream));
             dTm = c->tTmax.as<float>();
             EL_HIP(c, c->tOcc.ensure(n));
             dOcc = c->tOcc.as<uint8_t>();
-        } else {
-            EL_HIP(c, c->tTri.ensure((size_t)n * 4));
-            EL_HIP(c, c->tT.ensure((size_t)n * 4));
-            dTri = c->tTri.as<int32_t>();
-            dT = c->tT.as<float>();
-            if (uv) {
-                EL_HIP(c, c->tUV.ensure((size_t)n * 8));
-                dUV = c->tUV.as<float>();
-            }
+        } else if (uv) {
+            EL_HIP(c, c->tUV.ensure((size_t)n * 8));
+            dUV = c->tUV.as<float>();
         }
-    } else if (count) {
-        EL_HIP(c, c->tTri.ensure((size_t)n * 4));
-        EL_HIP(c, c->tT.ensure((size_t)n * 4));
-        if (!dTri) dTri = c->tTri.as<int32_t>();
-        if (!dT) dT = c->tT.as<float>();
     }
-    if (!devp && count) {
+    if (!any && !direct && (!devp || count)) {
         EL_HIP(c, c->tTri.ensure((size_t)n * 4));
         EL_HIP(c, c->tT.ensure((size_t)n * 4));
-        dTri = c->tTri.as<int32_t>();
-        dT = c->tT.as<float>();
+        if (!devp || !dTri) dTri = c->tTri.as<int32_t>();
+        if (!devp || !dT) dT = c->tT.as<float>();
     }
     unsigned long long* ctr = c->dCounters.as<unsigned long long>();
     EL_HIP(c, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, c->stream));
     EL_HIP(c, launchTrace(cfgOf(c), c->ds, dR, dTm, n, dTri, dT, dUV, dOcc, any, count, ctr));
-    unsigned long long h[kCounterWords];
-    EL_HIP(c, hipMemcpyAsync(h, ctr, sizeof h, hipMemcpyDeviceToHost, c->stream));
-    if (!devp) {
-        if (any) {
-            EL_HIP(c, hipMemcpyAsync(occ, dOcc, n, hipMemcpyDeviceToHost, c->stream));
-        } else if (!count) {
-            EL_HIP(c, hipMemcpyAsync(tri, dTri, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
-            EL_HIP(c, hipMemcpyAsync(t, dT, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
-            if (uv) EL_HIP(c, hipMemcpyAsync(uv, dUV, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
-        }
+    if (!devp && !direct && !count) {
+        // a chunk of n rays: each answer's n values after the other's
+        const std::vector<std::pair<void*, size_t>> host =
+            any ? std::vector<std::pair<void*, size_t>>{{occ, 1}}
+                : std::vector<std::pair<void*, size_t>>{{tri, 4}, {t, 4}, {uv, uv ? 8 : 0}};
+        const unsigned char* const dev[3] = {any ? (unsigned char*)dOcc : (unsigned char*)dTri, (unsigned char*)dT,
+                                             (unsigned char*)dUV};
+        size_t bytes = 0;
+        for (auto& o : host) bytes += o.second;
+        EL_HIP(c, stageOut(
+                      st, c->stream, n, bytes,
+                      [&](size_t first, size_t m, unsigned char* chunk) {
+                          hipError_t e = hipSuccess;
+                          for (size_t k = 0; k < host.size() && e == hipSuccess; k++) {
+                              const size_t w = host[k].second;
+                              if (w) e = hipMemcpyAsync(chunk, dev[k] + first * w, m * w, hipMemcpyDeviceToHost, c->stream);
+                              chunk += m * w;
+                          }
+                          return e;
+                      },
+                      [&](size_t first, size_t m, const unsigned char* chunk, size_t i0, size_t i1) {
+                          for (auto& o : host) {
+                              const size_t w = o.second;
+                              if (w) std::memcpy((unsigned char*)o.first + (first + i0) * w, chunk + i0 * w, (i1 - i0) * w);
+                              chunk += m * w;
+                          }
+                      }));
     }
-    EL_HIP(c, hipStreamSynchronize(c->stream));
+    EL_HIP(c, readTallies(c, ctr));
+    const unsigned long long* const h = st.tallies;
+    if (direct && any) std::memcpy(occ, dOcc, n);
+    if (direct && !any) {
+        std::memcpy(tri, dTri, (size_t)n * 4);
+        std::memcpy(t, dT, (size_t)n * 4);
+        if (uv) std::memcpy(uv, dUV, (size_t)n * 8);
+    }
     if (nodes) *nodes = tally(h, kStatNodes);
     if (tris) *tris = tally(h, kStatTris);
     if (tally(h, kStatOverflow)) return fail(c, EL_ERR_RANGE, "traversal stack overflow (results incomplete)");
@@ -1304,6 +1487,7 @@ struct el_batch {
     std::string graphKey;
     el_stats stats{};
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    std::shared_ptr<Stage> stage = std::make_shared<Stage>();
 };
 
 static int bfail(el_batch* b, int code, const std::string& what) {
@@ -1339,6 +1523,7 @@ int el_batch_create(el_batch** out, int device) {
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (hipEventCreate(&b->e0) != hipSuccess || hipEventCreate(&b->e1) != hipSuccess) return EL_ERR_HIP;
     if (b->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
+    if (b->stage->ensureTallies() != hipSuccess) return EL_ERR_HIP;
     *out = b.release();
     return EL_OK;
 }
@@ -1363,7 +1548,7 @@ int el_batch_add(el_batch* b, const el_scene_view* view, uint32_t spp, uint64_t 
     if (spp == 0) return bfail(b, EL_ERR_ARG, "spp must be positive");
     if (b->scenes.size() >= 65536) return bfail(b, EL_ERR_RANGE, "at most 65536 scenes per batch");
     el_ctx* c = nullptr;
-    int rc = el_create(&c, b->device);
+    int rc = createContext(&c, b->device, b->stage);
     if (rc) return bfail(b, rc, "context creation failed");
     rc = el_upload_scene(c, view);
     if (rc) {
@@ -1540,23 +1725,15 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
     q.segSize = (uint32_t)segSize;
     q.gstack = lc.gstack;
     q.gthreads = lc.maxThreads;
-    // clear the accumulations and tallies (outside any captured graph)
-    for (size_t i = 0; i < S; i++) {
-        el_ctx* c = b->scenes[i];
-        const size_t npx = (size_t)c->cam.x_res * c->cam.y_res;
-        EL_BHIP(b, hipMemsetAsync(c->dAccum.p, 0, npx * sizeof(float4), b->stream));
-        EL_BHIP(b, hipMemsetAsync(c->dCounts.p, 0, npx * sizeof(uint32_t), b->stream));
-    }
     unsigned long long* ctr = b->dCounters.as<unsigned long long>();
-    EL_BHIP(b, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, b->stream));
     const DevScene* dsc = b->dScenes.as<DevScene>();
     const bool apart = (p->flags & EL_BATCH_SERIAL_SHADOWS) != 0;
     auto launchAll = [&]() -> hipError_t {   // the launches of el_render's loop
         hipError_t e;
         for (const BatchGen& g : gens) {
             const BatchSeg* gseg = b->dSegs.as<BatchSeg>() + g.segOffset;
-            if ((e = launchBtCamera(lc, dsc, gseg, g.nseg, g.count, depth, !(p->flags & EL_BATCH_NO_CULL), q)) !=
-                hipSuccess)
+            if ((e = launchBtCamera(lc, dsc, gseg, g.nseg, g.count, depth, !(p->flags & EL_BATCH_NO_CULL), q,
+                                    &g == &gens[0], ctr)) != hipSuccess)
                 return e;
             bool extended = false;
             for (uint32_t bo = 0; bo < depth; bo++) {
@@ -1638,8 +1815,9 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         EL_BHIP(b, launchAll());
         EL_BHIP(b, hipEventRecord(b->e1, b->stream));
     }
-    unsigned long long h[kCounterWords];
-    EL_BHIP(b, hipMemcpyAsync(h, ctr, sizeof h, hipMemcpyDeviceToHost, b->stream));
+    const unsigned long long* const h = b->stage->tallies;
+    EL_BHIP(b, hipMemcpyAsync(b->stage->tallies, ctr, sizeof(unsigned long long) * kCounterWords,
+                              hipMemcpyDeviceToHost, b->stream));
     EL_BHIP(b, hipStreamSynchronize(b->stream));
     float t = 0;
     EL_BHIP(b, hipEventElapsedTime(&t, b->e0, b->e1));
@@ -1649,6 +1827,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         c->sampleBase = sppCap ? std::min(sppCap, b->spp[i]) : b->spp[i];
         c->accSeed = b->seed[i];
         c->accDepth = depth;
+        c->accPending = false;
         c->accMixed = true;   // batch RNG streams carry the scene index: no el_adjoint on them
         c->recValid = false;
     }

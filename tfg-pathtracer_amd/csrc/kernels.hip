@@ -139,6 +139,10 @@ template <bool WIDE>
 __device__ __forceinline__ WorkSource chunkSource(uint32_t* qcounters, int kind, uint32_t n, bool quads) {
     return chunkSource<WIDE>(qcounters, kind, n, quads, gridWave(), gridWaves());
 }
+// The first kernel of a render zeroes the tallies that the others add to.
+__device__ __forceinline__ void zeroTallies(unsigned long long* counters) {
+    if (blockIdx.x == 0 && threadIdx.x < kXcds * kStatSlots) counters[threadIdx.x] = 0;
+}
 // Zeroes the chunk counters of `kind` (threads 0..kChunkShares-1 of block 0).
 __device__ __forceinline__ void resetChunks(uint32_t* qcounters, int kind) {
     if (blockIdx.x == 0 && threadIdx.x < kChunkShares)
@@ -684,7 +688,8 @@ __device__ __forceinline__ uint64_t recordKey(const DevScene& s, const RenderArg
 
 // Camera rays go to queue 0 at index = path slot (no compaction); padding
 // slots get a zero direction, which the extend kernel reports as dead.
-EL_KERNEL(1) void k_wf_camera(DevScene s, RenderArgs a, WfState q) {
+EL_KERNEL(1) void k_wf_camera(DevScene s, RenderArgs a, WfState q, unsigned long long* counters) {
+    if (a.zeroTallies) zeroTallies(counters);
     uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < a.genCount; slot += stride) {
         uint32_t sample, x, y;
@@ -1139,8 +1144,9 @@ EL_KERNEL(1) void k_wf_finalize(DevScene s, RenderArgs a, WfState q, float4* __r
         uint32_t sample, x, y;
         const uint32_t idx = slotPixel(s, a, j, sample, x, y);
         if (idx == 0xFFFFFFFFu) continue;   // padding pixel
-        float4 acc = accum[idx];
-        uint32_t n = counts[idx];
+        const bool fresh = a.fresh && sample == 0;
+        float4 acc = fresh ? make_float4(0.f, 0.f, 0.f, 0.f) : accum[idx];
+        uint32_t n = fresh ? 0u : counts[idx];
         float4 A[3];
         if (aov)
             for (int k = 0; k < 3; k++) A[k] = aov[3 * (uint64_t)idx + k];
@@ -1351,7 +1357,9 @@ __device__ __forceinline__ uint32_t findSeg(const BatchSeg* segs, uint32_t nseg,
 // Camera rays of a batch generation: slot -> (scene, sample, pixel) through
 // the segment table; the scene id rides in the ray's d.w.
 EL_KERNEL(1) void k_bt_camera(ManyScenes sc, const BatchSeg* __restrict__ segs, uint32_t nseg, uint32_t genCount,
-                              uint32_t maxDepth, uint32_t cull, WfState q) {
+                              uint32_t maxDepth, uint32_t cull, WfState q, uint32_t zero,
+                              unsigned long long* counters) {
+    if (zero) zeroTallies(counters);
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < genCount; slot += stride) {
         const BatchSeg g = segs[findSeg(segs, nseg, slot, false)];
@@ -1398,8 +1406,10 @@ EL_KERNEL(1) void k_bt_finalize(ManyScenes sc, const BatchSeg* __restrict__ segs
         // stay in registers (added in sample order) and are stored once
         const uint32_t idx = q.pathPix[first];
         if (idx == 0xFFFFFFFFu) continue;   // padding pixel
-        float4 acc = s.accum[idx];
-        uint32_t n = s.counts[idx];
+        // a batch render starts from an empty accumulation: sample 0 of a pixel, which every pixel has once
+        const bool fresh = q.pathSample[first] == 0;
+        float4 acc = fresh ? make_float4(0.f, 0.f, 0.f, 0.f) : s.accum[idx];
+        uint32_t n = fresh ? 0u : s.counts[idx];
         for (uint32_t slot = first; slot < end; slot += g.npad) {
             const float4 Lf = finishedL(q, slot);
             paths++;
@@ -1454,6 +1464,21 @@ __global__ void __launch_bounds__(256) k_residual_l2(const float4* __restrict__ 
         double b = 0.0;
         for (uint32_t w = 0; w < (blockDim.x >> 6); w++) b += s_part[w];
         atomicAdd(loss, b);
+    }
+}
+
+// Pixels [first, first + n) of a mean image: sums[i * stride] / counts[i] and
+// alpha 1 (0 without samples), and the counts.  The outputs are mapped host
+// memory, so the image crosses the bus as it is divided, once.
+__global__ void __launch_bounds__(256) k_resolve(const float4* __restrict__ sums, uint32_t stride,
+                                                 const uint32_t* __restrict__ counts, uint32_t first, uint32_t n,
+                                                 float4* __restrict__ rgba, uint32_t* __restrict__ samples) {
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const uint32_t i = first + k, c = counts[i];
+        const float fc = (float)c;
+        const float4 a = sums[(uint64_t)i * stride];
+        if (rgba) rgba[k] = c ? make_float4(a.x / fc, a.y / fc, a.z / fc, 1.f) : make_float4(0.f, 0.f, 0.f, 1.f);
+        if (samples) samples[k] = c;
     }
 }
 
@@ -1528,6 +1553,13 @@ hipError_t launchAdjBounce(const LaunchCfg& c, const DevScene& s, const RenderAr
     return hipGetLastError();
 }
 
+hipError_t launchResolve(hipStream_t stream, const float4* sums, uint32_t stride, const uint32_t* counts,
+                         uint32_t first, uint32_t n, float4* rgba, uint32_t* samples) {
+    hipLaunchKernelGGL(k_resolve, dim3(gridFor(n, 256, 2048)), dim3(256), 0, stream, sums, stride, counts, first, n,
+                       rgba, samples);
+    return hipGetLastError();
+}
+
 hipError_t launchResidualL2(hipStream_t stream, const float4* accum, const uint32_t* counts, const float* target,
                             uint32_t npx, float* r, double* loss) {
     const uint32_t grid = gridFor(npx, 256, 4096);
@@ -1541,9 +1573,10 @@ hipError_t launchEnvTable(hipStream_t stream, const DevScene& s, float4* tab) {
     return hipGetLastError();
 }
 
-hipError_t launchWfCamera(const LaunchCfg& c, const DevScene& s, const RenderArgs& a, const WfState& q) {
+hipError_t launchWfCamera(const LaunchCfg& c, const DevScene& s, const RenderArgs& a, const WfState& q,
+                          unsigned long long* counters) {
     uint32_t grid = gridFor(a.genCount, c.shadeBlock, c.maxThreads / c.shadeBlock);
-    hipLaunchKernelGGL(k_wf_camera, dim3(grid), dim3(c.shadeBlock), 0, c.stream, s, a, q);
+    hipLaunchKernelGGL(k_wf_camera, dim3(grid), dim3(c.shadeBlock), 0, c.stream, s, a, q, counters);
     return hipGetLastError();
 }
 
@@ -1622,10 +1655,11 @@ hipError_t launchWfFinalize(const LaunchCfg& c, const DevScene& s, const RenderA
 
 // ---- batch launchers
 hipError_t launchBtCamera(const LaunchCfg& c, const DevScene* scenes, const BatchSeg* segs, uint32_t nseg,
-                          uint32_t genCount, uint32_t maxDepth, bool cull, const WfState& q) {
+                          uint32_t genCount, uint32_t maxDepth, bool cull, const WfState& q, bool zeroTallies,
+                          unsigned long long* counters) {
     uint32_t grid = gridFor(genCount, c.shadeBlock, c.maxThreads / c.shadeBlock);
     hipLaunchKernelGGL(k_bt_camera, dim3(grid), dim3(c.shadeBlock), 0, c.stream, ManyScenes{scenes}, segs, nseg,
-                       genCount, maxDepth, cull ? 1u : 0u, q);
+                       genCount, maxDepth, cull ? 1u : 0u, q, zeroTallies ? 1u : 0u, counters);
     return hipGetLastError();
 }
 

@@ -57,6 +57,9 @@ struct RenderArgs {
     uint32_t genCount;      // wavefront: work items in the generation
     uint32_t npad;          // wavefront: padded pixel count (8x8 tiles)
     uint32_t cull;          // stop zero-throughput paths that cannot turn NaN
+    uint32_t fresh;         // wavefront: the accumulation holds nothing yet and is not cleared: finalize
+                            // starts a pixel's sums from zero at sample 0 (every pixel has that sample once)
+    uint32_t zeroTallies;   // wavefront: the camera launch zeroes the tallies
     float4* rec;            // per (sample, pixel): the path's radiance before the clamp, or null
     // Wavefront renders that record, and adjoints that replay, path vertices
     // (one scene; all null otherwise): the closest hit (tri, t, u, v; tri -1:
@@ -135,6 +138,10 @@ hipError_t launchTrace(const LaunchCfg& c, const dev::DevScene& s, const float* 
                        unsigned long long* counters);
 hipError_t launchPlain(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, float4* accum,
                        uint32_t* counts, float4* aov, unsigned long long* counters);
+// Pixels [first, first + n) of the mean image sums[i * stride] / counts[i] to rgba, and counts to samples (mapped host
+// memory; either may be null).
+hipError_t launchResolve(hipStream_t stream, const float4* sums, uint32_t stride, const uint32_t* counts,
+                         uint32_t first, uint32_t n, float4* rgba, uint32_t* samples);
 // r = 2 (mean image - target) per pixel and channel (FP64 arithmetic, FP32
 // store); *loss += sum (mean image - target)^2 (the caller zeroes it).
 hipError_t launchResidualL2(hipStream_t stream, const float4* accum, const uint32_t* counts, const float* target,
@@ -148,7 +155,8 @@ hipError_t launchAdjBounce(const LaunchCfg& c, const dev::DevScene& s, const Ren
 // Batch (many scenes, scene id per queue entry): scenes = device array of
 // DevScene; segs = the generation's segment table (device).
 hipError_t launchBtCamera(const LaunchCfg& c, const dev::DevScene* scenes, const BatchSeg* segs, uint32_t nseg,
-                          uint32_t genCount, uint32_t maxDepth, bool cull, const WfState& q);
+                          uint32_t genCount, uint32_t maxDepth, bool cull, const WfState& q, bool zeroTallies,
+                          unsigned long long* counters);
 hipError_t launchBtExtend(const LaunchCfg& c, const dev::DevScene* scenes, int width, const WfState& q,
                           const float4* rayIn, const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount,
                           unsigned long long* counters);
@@ -162,7 +170,8 @@ hipError_t launchBtTrace(const LaunchCfg& c, const dev::DevScene* scenes, int wi
                          unsigned long long* counters);
 hipError_t launchBtFinalize(const LaunchCfg& c, const dev::DevScene* scenes, const BatchSeg* segs, uint32_t nseg,
                             uint32_t finTotal, const WfState& q, unsigned long long* counters);
-hipError_t launchWfCamera(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, const WfState& q);
+hipError_t launchWfCamera(const LaunchCfg& c, const dev::DevScene& s, const RenderArgs& a, const WfState& q,
+                          unsigned long long* counters);
 hipError_t launchWfExtend(const LaunchCfg& c, const dev::DevScene& s, const WfState& q, const float4* rayIn,
                           const uint32_t* countIn, uint32_t* resetNext, uint32_t maxCount, bool countTraversal,
                           unsigned long long* counters);
