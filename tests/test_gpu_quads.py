@@ -98,3 +98,20 @@ def test_queues_in_one_launch_equal_launches_of_their_own(gpu_ctx, side, spp, wi
     gpu_ctx.render(1, depth=1, bvh_width=4)   # the context is shared: back to the default tree
     for o in out[1:]:
         assert all(np.array_equal(x, y) for x, y in zip(out[0], o))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [131072, 131073, 262144 - 15, 262144 + 16, 393216 + 1, 917504, (1 << 22) + 65, 10_000_001])
+def test_every_chunk_is_traced_once(gpu_ctx, field, n):
+    """Full and partial turns of a launch's waves (8,192 x 16 rays a turn by quads, 8,192 x 64 and more by lanes): every
+    ray is answered as in a launch of its own part."""
+    print(f"[quads] {n} rays in turns", flush=True)
+    gpu_ctx.upload(field)
+    some = raygen.random_rays(field.vertices(), 1 << 16, seed=21)
+    want = gpu_ctx.trace_closest(some)
+    rays = np.tile(some, ((n + len(some) - 1) // len(some), 1))[:n]
+    got = gpu_ctx.trace_closest(rays)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, np.concatenate([y] * ((n + len(y) - 1) // len(y)))[:n])
+    occ = gpu_ctx.trace_any(rays, np.full(n, np.inf, np.float32))
+    assert np.array_equal(occ, got[0] >= 0)

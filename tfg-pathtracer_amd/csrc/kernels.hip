@@ -95,7 +95,9 @@ __device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n) {
 
 // Waves of the grid and the calling one's index.
 __device__ __forceinline__ uint32_t gridWaves() { return (gridDim.x * blockDim.x) >> 6; }
-__device__ __forceinline__ uint32_t gridWave() { return (blockIdx.x * blockDim.x + threadIdx.x) >> 6; }
+__device__ __forceinline__ uint32_t gridWave() {
+    return __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+}
 
 // Chunks of n items for `waves` waves, the first-th of which calls: kChunkRays,
 // smaller (down to the G rays a wave holds at once: one per lane, or one per
@@ -155,7 +157,7 @@ struct QueueMap {
     __device__ __forceinline__ void load(const uint32_t* cnt) {
         pre[0] = 0;
 #pragma unroll
-        for (int k = 0; k < kXcds; k++) pre[k + 1] = pre[k] + cnt[k];
+        for (int k = 0; k < kXcds; k++) pre[k + 1] = pre[k] + __builtin_amdgcn_readfirstlane(cnt[k]);   // scalar
     }
     __device__ __forceinline__ uint32_t total() const { return pre[kXcds]; }
     __device__ __forceinline__ uint64_t entry(uint32_t i, uint32_t segSize) const {
@@ -1084,6 +1086,9 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_trace(P sc, WfState q, const float4* __restrict
         nH += cntH[k];
         nP += cntP[k];
     }
+    nE = __builtin_amdgcn_readfirstlane(nE);
+    nH = __builtin_amdgcn_readfirstlane(nH);
+    nP = __builtin_amdgcn_readfirstlane(nP);
     const bool quads = useQuads<W>(sc.any(), nE + nH + nP);
     // Every wave works on one queue: a wave for each chunk if they suffice,
     // else in proportion to the rays (at least one), a closest hit counted as
@@ -1093,10 +1098,10 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_trace(P sc, WfState q, const float4* __restrict
     uint32_t wE = (nE + G - 1) / G, wH = (nH + G - 1) / G;
     if (wE + wH + (nP + G - 1) / G > waves) {
         const float e = 0.75f * (float)nE, share = (float)(waves - 3) / (e + (float)nH + (float)nP);
-        wE = nE ? 1u + (uint32_t)(e * share) : 0u;
-        wH = nH ? 1u + (uint32_t)((float)nH * share) : 0u;
+        wE = nE ? __builtin_amdgcn_readfirstlane(1u + (uint32_t)(e * share)) : 0u;
+        wH = nH ? __builtin_amdgcn_readfirstlane(1u + (uint32_t)((float)nH * share)) : 0u;
     }
-    const uint32_t w = __builtin_amdgcn_readfirstlane(gridWave());
+    const uint32_t w = gridWave();
     const int kind = w < wE ? 0 : w < wE + wH ? 1 : 2;
     QueueTally tl;
     QueueMap qm;
