@@ -367,8 +367,9 @@ template bool quantizeNode<8>(const WideNode<8>&, QNode<8>&);
 void packLaneNode(const QNode<4>& n, uint32_t out[16]) {
     for (int j = 0; j < 4; j++) {
         uint32_t* w = out + 4 * j;
-        w[0] = (uint32_t)n.child[j];
-        w[1] = n.plane(0, j) | n.plane(2, j) << 8 | (j < 3 ? ((n.exps >> (8 * j)) & 0xffu) << 23 : 0u);
+        w[0] = (uint32_t)(n.child[j] >= 0 ? 4 * n.child[j] : n.child[j]);
+        w[1] = n.plane(0, j) | n.plane(2, j) << 8 | (j < 3 ? ((n.exps >> (8 * j)) & 0xffu) << 23 : 0u) |
+               (n.child[j] == -1 ? 0x80000000u : 0u);
         w[2] = n.plane(4, j) | n.plane(1, j) << 8 | n.plane(3, j) << 16 | n.plane(5, j) << 24;
         w[3] = 0;
         if (j < 3) std::memcpy(&w[3], &n.p[j], 4);

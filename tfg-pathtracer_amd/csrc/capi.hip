@@ -184,7 +184,7 @@ inline unsigned long long tally(const unsigned long long* h, int slot) {
 // device's address comes from hipGetSymbolAddress, looked up once per device
 // by el_create with that device current.
 constexpr size_t kScratchCounterBytes = 512;                  // >= kCounterWords * 8
-constexpr size_t kScratchSpillInts = size_t(4) << 20;         // 16 MiB of spill slots
+constexpr size_t kScratchSpillInts = (size_t(4) << 20) + 1024;   // 16 MiB of spill slots and a block's visit rows
 constexpr size_t kScratchBytes = kScratchCounterBytes + kScratchSpillInts * sizeof(int);
 static_assert(kScratchCounterBytes >= sizeof(unsigned long long) * kXcds * kStatSlots, "tallies fit");
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -447,7 +447,7 @@ static int uploadBvh(el_ctx* c, int width) {
     const void* nodes = width == 4 ? (const void*)lanes.data() : (const void*)c->wide.nodes.data();
     EL_HIP(c, upload(c->dNodes, nodes, c->wide.nodes.size(), c->stream));
     EL_HIP(c, upload(c->dTris, c->wide.triStream.data(), c->wide.triStream.size() * sizeof(float), c->stream));
-    c->gcap = std::max(1, c->wide.stackBound + 2 - dev::kShortStack);
+    c->gcap = dev::spillRows(c->wide.stackBound);
     EL_HIP(c, c->dGstack.ensure((size_t)c->gcap * c->maxThreads * sizeof(int)));
     c->ds.nodes = c->dNodes.p;
     c->ds.tris = c->dTris.as<float4>();

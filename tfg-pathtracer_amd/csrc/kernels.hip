@@ -215,13 +215,12 @@ __device__ __forceinline__ void blockAlloc3(const bool (&want)[3], uint32_t* con
 __device__ __forceinline__ TravStack makeStack(const DevScene& s, int* gstack, uint32_t gthreads) {
     extern __shared__ int lds[];
     TravStack st;
-    st.lds = lds + threadIdx.x;
-    st.ldsStride = blockDim.x;
+    st.lds = lds + (threadIdx.x >> 6) * (kShortStack * 64) + (threadIdx.x & 63u);
     uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     st.g = gstack + gtid;
     st.gstride = (int)gthreads;
     st.gcap = s.gcap;
-    st.sp = st.lo = 0;
+    st.reset();
     st.overflow = false;
     return st;
 }
