@@ -783,6 +783,7 @@ static int wfPlan(el_ctx* c, const LaunchCfg& lc, uint64_t total, uint64_t npad,
     q.pendP = c->wPend.as<float4>();
     q.counters = c->wCounters.as<uint32_t>();
     q.segSize = (uint32_t)segSize;
+    q.cap = qcap;
     q.gstack = lc.gstack;
     q.gthreads = lc.maxThreads;
     return EL_OK;
@@ -1723,6 +1724,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
     q.pendP = b->wPend.as<float4>();
     q.counters = b->wCounters.as<uint32_t>();
     q.segSize = (uint32_t)segSize;
+    q.cap = qcap;
     q.gstack = lc.gstack;
     q.gthreads = lc.maxThreads;
     unsigned long long* ctr = b->dCounters.as<unsigned long long>();

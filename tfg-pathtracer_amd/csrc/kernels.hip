@@ -160,16 +160,25 @@ struct QueueMap {
         for (int k = 0; k < kXcds; k++) pre[k + 1] = pre[k] + __builtin_amdgcn_readfirstlane(cnt[k]);   // scalar
     }
     __device__ __forceinline__ uint32_t total() const { return pre[kXcds]; }
-    __device__ __forceinline__ uint64_t entry(uint32_t i, uint32_t segSize) const {
+    __device__ __forceinline__ uint32_t entry(uint32_t i, uint32_t segSize) const {
         // selects only: a dynamic index into pre[] would put it in scratch
-        uint32_t s = 0, base = 0;
+        uint32_t off = 0;
+#pragma unroll
+        for (int k = 1; k < kXcds; k++) off = i >= pre[k] ? (uint32_t)k * segSize - pre[k] : off;
+        return off + i;
+    }
+    // The same for the lanes that take consecutive items i, the lowest lane
+    // the first: mostly of one segment, which is then looked up in scalar
+    // registers.
+    __device__ __forceinline__ uint32_t entryOfWave(uint32_t i, uint32_t segSize) const {
+        const uint32_t first = __builtin_amdgcn_readfirstlane(i);
+        uint32_t off = 0, end = pre[1];
 #pragma unroll
         for (int k = 1; k < kXcds; k++) {
-            bool past = i >= pre[k];
-            s = past ? (uint32_t)k : s;
-            base = past ? pre[k] : base;
+            off = first >= pre[k] ? (uint32_t)k * segSize - pre[k] : off;
+            end = first >= pre[k] ? pre[k + 1] : end;
         }
-        return (uint64_t)s * segSize + (i - base);
+        return waveMask(i >= end) == 0 ? off + i : entry(i, segSize);
     }
 };
 
@@ -212,33 +221,34 @@ __device__ __forceinline__ void blockAlloc3(const bool (&want)[3], uint32_t* con
     __syncthreads();   // s_cnt is reused by the next call
 }
 
-__device__ __forceinline__ TravStack makeStack(const DevScene& s, int* gstack, uint32_t gthreads) {
+__device__ __forceinline__ TravStack makeStack(const DevScene& s, int* gstack, uint32_t gthreads,
+                                               unsigned long long* counters) {
     extern __shared__ int lds[];
     TravStack st;
     st.lds = lds + (threadIdx.x >> 6) * (kShortStack * 64) + (threadIdx.x & 63u);
-    uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    st.g = gstack + gtid;
+    st.g = gstack + 64u * gridWave();
     st.gstride = (int)gthreads;
     st.gcap = s.gcap;
+    st.dropped = counters + xcdOf() * kStatSlots + kStatOverflow;
     st.reset();
-    st.overflow = false;
     return st;
 }
 
-// Traces the items of ws, by quads or by lanes.  overflow is set if a lane's stack was too small.
+// Traces the items of ws, by quads or by lanes.  traced: the wave's rays, in its first lane (else 0).
 template <int W, bool ANY, bool COUNT, bool PER_RAY_BVH, class Load, class Store>
 __device__ __forceinline__ void traceQueue(const DevScene& s, int* gstack, uint32_t gthreads, const WorkSource& ws,
                                            bool quads, uint32_t refill, Load&& load, Store&& store,
-                                           TraceCounters& cnt, uint32_t& traced, uint32_t& overflow) {
+                                           unsigned long long* counters, TraceCounters& cnt, uint32_t& traced) {
+    uint32_t rays = 0;
     if (W == 4 && quads) {
         extern __shared__ int lds[];
         QuadStack st{lds + (threadIdx.x >> 6) * (kQuadStack * 16) + ((threadIdx.x >> 2) & 15u), 0};
-        traceQuadRange<ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, traced);
+        traceQuadRange<ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, rays);
     } else {
-        TravStack st = makeStack(s, gstack, gthreads);
-        traceWaveRange<W, ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, traced);
-        overflow |= st.overflow;
+        TravStack st = makeStack(s, gstack, gthreads, counters);
+        traceWaveRange<W, ANY, COUNT, PER_RAY_BVH>(s, st, ws, refill, load, store, cnt, rays);
     }
+    traced = __lane_id() == 0 ? rays : 0u;
 }
 
 // ------------------------------------------------------------------ trace --
@@ -248,11 +258,12 @@ EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, 
                                     float* __restrict__ outUV, uint8_t* __restrict__ outOcc, int* gstack,
                                     uint32_t gthreads, uint32_t refill, unsigned long long* counters) {
     TraceCounters cnt{0, 0};
-    uint32_t traced = 0, overflow = 0;
+    uint32_t traced = 0;
     const bool quads = useQuads<W>(s, n);
     const WorkSource ws = splitWork(n, quads, gridWave(), gridWaves());
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
-                    BvhPtr&) {
+                    BvhPtr&, uint32_t& item) {
+        item = i;
         const float* r = rays + (uint64_t)i * 6;
         ox = r[0];
         oy = r[1];
@@ -275,10 +286,10 @@ EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, 
             }
         }
     };
-    traceQueue<W, ANY, COUNT, false>(s, gstack, gthreads, ws, quads, refill, load, store, cnt, traced, overflow);
-    const int slots[3] = {kStatNodes, kStatTris, kStatOverflow};
-    const uint32_t vals[3] = {cnt.nodes, cnt.tris, overflow};
-    blockFlush<3>(counters, slots, vals);
+    traceQueue<W, ANY, COUNT, false>(s, gstack, gthreads, ws, quads, refill, load, store, counters, cnt, traced);
+    const int slots[2] = {kStatNodes, kStatTris};
+    const uint32_t vals[2] = {cnt.nodes, cnt.tris};
+    blockFlush<2>(counters, slots, vals);
 }
 
 // --------------------------------------------------------- shared shading --
@@ -458,11 +469,11 @@ template <int W>
 EL_KERNEL(EL_WPE_PLAIN) void k_plain(DevScene s, RenderArgs a, float4* __restrict__ accum, uint32_t* __restrict__ counts,
                         float4* __restrict__ aov, int* gstack, uint32_t gthreads,
                         unsigned long long* counters) {
-    TravStack st = makeStack(s, gstack, gthreads);
+    TravStack st = makeStack(s, gstack, gthreads, counters);
     TraceCounters cnt{0, 0};
     const uint32_t W_ = s.cam.xRes, H_ = s.cam.yRes;
     const uint32_t tilesX = (W_ + 15) / 16;
-    uint32_t rays = 0, verts = 0, paths = 0, overflow = 0;
+    uint32_t rays = 0, verts = 0, paths = 0;
     uint32_t stride = gridDim.x * blockDim.x;
     uint32_t total = tilesX * ((H_ + 15) / 16) * 256;
     for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < total; w += stride) {
@@ -478,7 +489,6 @@ EL_KERNEL(EL_WPE_PLAIN) void k_plain(DevScene s, RenderArgs a, float4* __restric
                 surfaceTangents(s, sh, at, ab);
             }
         });
-        overflow |= st.overflow;
         if (a.rec) a.rec[(uint64_t)a.sample * W_ * H_ + idx] = make_float4(L.x, L.y, L.z, 1.f);
         L = clamp3(L);
         if (!anyNan(L)) {
@@ -493,9 +503,9 @@ EL_KERNEL(EL_WPE_PLAIN) void k_plain(DevScene s, RenderArgs a, float4* __restric
             }
         }
     }
-    const int slots[4] = {kStatRays, kStatVerts, kStatPaths, kStatOverflow};
-    const uint32_t vals[4] = {rays, verts, paths, overflow};
-    blockFlush<4>(counters, slots, vals);
+    const int slots[3] = {kStatRays, kStatVerts, kStatPaths};
+    const uint32_t vals[3] = {rays, verts, paths};
+    blockFlush<3>(counters, slots, vals);
 }
 
 // ---------------------------------------------------------------- adjoint --
@@ -713,9 +723,9 @@ EL_KERNEL(1) void k_wf_camera(DevScene s, RenderArgs a, WfState q, unsigned long
         }
         q.pathQuiet[slot] = quiet;
         if (q.pathVis) q.pathVis[slot] = 0u;
-        float4* Q = q.ray[0] + 2 * (uint64_t)slot;
+        float4* Q = q.ray[0] + slot;
         Q[0] = make_float4(o.x, o.y, o.z, __uint_as_float(slot));
-        Q[1] = make_float4(d.x, d.y, d.z, __uint_as_float(a.scene));
+        Q[q.cap] = make_float4(d.x, d.y, d.z, __uint_as_float(a.scene));
     }
     if (blockIdx.x == 0 && threadIdx.x < kXcds) q.counters[kQRay0 + threadIdx.x] = threadIdx.x == 0 ? a.genCount : 0u;
     resetChunks(q.counters, kChunkExt);
@@ -741,7 +751,8 @@ struct ManyScenes {
 
 // Tallies of a launch's traversals.
 struct QueueTally {
-    uint32_t rays = 0, overflow = 0;
+    unsigned long long* counters;
+    uint32_t rays = 0;
     TraceCounters cnt{0, 0};
 };
 
@@ -752,9 +763,9 @@ __device__ __forceinline__ void extendQueue(const P& sc, const WfState& q, const
                                             QueueTally& tl) {
     const uint32_t segSize = q.segSize;
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
-                    BvhPtr& bvh) {
-        const uint64_t e = qm.entry(i, segSize);
-        const float4 A = rayIn[2 * e], B = rayIn[2 * e + 1];
+                    BvhPtr& bvh, uint32_t& item) {
+        item = qm.entryOfWave(i, segSize);
+        const float4 A = rayIn[item], B = rayIn[q.cap + item];
         ox = A.x;
         oy = A.y;
         oz = A.z;
@@ -768,11 +779,11 @@ __device__ __forceinline__ void extendQueue(const P& sc, const WfState& q, const
         }
         return !(B.x == 0.f && B.y == 0.f && B.z == 0.f);   // zero direction: camera-queue padding
     };
-    auto store = [&](uint32_t i, const TraceResult& h, bool) {
-        q.hits[qm.entry(i, segSize)] = make_float4(__int_as_float(h.tri), h.t, h.u, h.v);
+    auto store = [&](uint32_t e, const TraceResult& h, bool) {
+        q.hits[e] = make_float4(__int_as_float(h.tri), h.t, h.u, h.v);
     };
-    traceQueue<W, false, COUNT, P::kMany>(sc.any(), q.gstack, q.gthreads, ws, quads, refill, load, store, tl.cnt,
-                                          tl.rays, tl.overflow);
+    traceQueue<W, false, COUNT, P::kMany>(sc.any(), q.gstack, q.gthreads, ws, quads, refill, load, store, tl.counters,
+                                          tl.cnt, tl.rays);
 }
 
 // Clears the counters the next shade kernel appends to: the next ray queue
@@ -796,11 +807,11 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_extend(P sc, WfState q, const float4* __restric
     const uint32_t n = qm.total();
     resetForShade(q, resetNext, q.parity);
     const bool quads = useQuads<W>(sc.any(), n);
-    QueueTally tl;
+    QueueTally tl{counters};
     extendQueue<W, COUNT>(sc, q, rayIn, qm, chunkSource<P::kMany>(q.counters, kChunkExt, n, quads), quads, refill, tl);
-    const int slots[5] = {kStatRays, kStatOverflow, kStatNodes, kStatTris, kStatExtRays};
-    const uint32_t vals[5] = {tl.rays, tl.overflow, tl.cnt.nodes, tl.cnt.tris, tl.rays};
-    blockFlush<5>(counters, slots, vals);
+    const int slots[4] = {kStatRays, kStatNodes, kStatTris, kStatExtRays};
+    const uint32_t vals[4] = {tl.rays, tl.cnt.nodes, tl.cnt.tris, tl.rays};
+    blockFlush<4>(counters, slots, vals);
 }
 
 // Adds `c` to a path's radiance.  The first bounce writes it (the radiance
@@ -869,7 +880,7 @@ EL_KERNEL(EL_WPE_SHADE) void k_wf_shade(P sc, RenderArgs a, WfState q, const flo
                 e = (uint32_t)qm.entry(i, q.segSize);
                 const int tri = __float_as_int(q.hits[e].x);
                 if (tri == -1) {
-                    const float4 A = rayIn[2 * (uint64_t)e], B = rayIn[2 * (uint64_t)e + 1];
+                    const float4 A = rayIn[e], B = rayIn[q.cap + e];
                     const uint32_t slot = __float_as_uint(A.w);
                     const DevScene& s = sc.get(__float_as_uint(B.w));
                     const float4 Tf = bounce == 0 ? make_float4(1, 1, 1, 0) : q.pathT[slot];
@@ -883,7 +894,7 @@ EL_KERNEL(EL_WPE_SHADE) void k_wf_shade(P sc, RenderArgs a, WfState q, const flo
                     // escape (tri -2: camera-queue padding, no path)
                     if (a.recHits && tri >= -1) {
                         const DevScene& s = sc.get(0);
-                        const uint32_t slot = __float_as_uint(rayIn[2 * (uint64_t)e].w);
+                        const uint32_t slot = __float_as_uint(rayIn[e].w);
                         uint32_t smp, px, py;
                         const uint32_t pix = slotPixel(s, a, slot, smp, px, py);
                         if (pix != 0xFFFFFFFFu)
@@ -915,7 +926,7 @@ EL_KERNEL(EL_WPE_SHADE) void k_wf_shade(P sc, RenderArgs a, WfState q, const flo
         VertexOut vo;
         uint32_t slot = 0, sid = 0;
         if (has) {
-            const float4 A = rayIn[2 * (uint64_t)e], B = rayIn[2 * (uint64_t)e + 1];
+            const float4 A = rayIn[e], B = rayIn[q.cap + e];
             const float4 hr = q.hits[e];
             slot = __float_as_uint(A.w);
             sid = __float_as_uint(B.w);
@@ -976,21 +987,21 @@ EL_KERNEL(EL_WPE_SHADE) void k_wf_shade(P sc, RenderArgs a, WfState q, const flo
         uint64_t at[3];
         blockAlloc3(want, outCnt, q.segSize, at, overflow);   // ends with a barrier: the pool may be refilled
         if (at[0] != ~0ull) {
-            float4* Q = rayOut + 2 * at[0];
+            float4* Q = rayOut + at[0];
             Q[0] = make_float4(vo.nextO.x, vo.nextO.y, vo.nextO.z, __uint_as_float(slot));
-            Q[1] = make_float4(vo.nextD.x, vo.nextD.y, vo.nextD.z, __uint_as_float(sid));
+            Q[q.cap] = make_float4(vo.nextD.x, vo.nextD.y, vo.nextD.z, __uint_as_float(sid));
         }
         if (at[1] != ~0ull) {
-            float4* S = q.shadowH + 3 * at[1];
+            float4* S = q.shadowH + at[1];
             S[0] = make_float4(vo.hOrig.x, vo.hOrig.y, vo.hOrig.z, __uint_as_float(slot));
-            S[1] = make_float4(vo.hDir.x, vo.hDir.y, vo.hDir.z, __int_as_float(0x7f800000));
-            S[2] = make_float4(vo.contribH.x, vo.contribH.y, vo.contribH.z, __uint_as_float(sid));
+            S[q.cap] = make_float4(vo.hDir.x, vo.hDir.y, vo.hDir.z, __int_as_float(0x7f800000));
+            S[2 * q.cap] = make_float4(vo.contribH.x, vo.contribH.y, vo.contribH.z, __uint_as_float(sid));
         }
         if (at[2] != ~0ull) {
-            float4* S = q.shadowP + 3 * at[2];
+            float4* S = q.shadowP + at[2];
             S[0] = make_float4(vo.pOrig.x, vo.pOrig.y, vo.pOrig.z, __uint_as_float(slot));
-            S[1] = make_float4(vo.pDir.x, vo.pDir.y, vo.pDir.z, vo.pTmax);
-            S[2] = make_float4(vo.contribP.x, vo.contribP.y, vo.contribP.z, __uint_as_float(sid));
+            S[q.cap] = make_float4(vo.pDir.x, vo.pDir.y, vo.pDir.z, vo.pTmax);
+            S[2 * q.cap] = make_float4(vo.contribP.x, vo.contribP.y, vo.contribP.z, __uint_as_float(sid));
         }
     }
     const int slots[3] = {kStatRays, kStatVerts, kStatOverflow};
@@ -1012,9 +1023,9 @@ __device__ __forceinline__ void shadowQueue(const P& sc, const WfState& q, const
                                             uint32_t visBit, uint32_t refill, QueueTally& tl) {
     const uint32_t segSize = q.segSize;
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
-                    BvhPtr& bvh) {
-        const uint64_t e = qm.entry(i, segSize);
-        const float4 A = sh[3 * e], B = sh[3 * e + 1];
+                    BvhPtr& bvh, uint32_t& item) {
+        item = qm.entryOfWave(i, segSize);
+        const float4 A = sh[item], B = sh[q.cap + item];
         ox = A.x;
         oy = A.y;
         oz = A.z;
@@ -1023,17 +1034,16 @@ __device__ __forceinline__ void shadowQueue(const P& sc, const WfState& q, const
         dz = B.z;
         tm = B.w;
         if (P::kMany) {
-            const DevScene& sx = sc.get(__float_as_uint(sh[3 * e + 2].w));
+            const DevScene& sx = sc.get(__float_as_uint(sh[2 * q.cap + item].w));
             bvh = BvhPtr{(const uint4*)sx.nodes, sx.tris};
         }
         return true;
     };
-    auto store = [&](uint32_t i, const TraceResult& h, bool) {
+    auto store = [&](uint32_t e, const TraceResult& h, bool) {
         const bool blocked = h.tri >= 0;
         if (blocked && !defer) return;
-        const uint64_t e = qm.entry(i, segSize);
-        const uint32_t slot = __float_as_uint(sh[3 * e].w);
-        const float4 C = sh[3 * e + 2];
+        const uint32_t slot = __float_as_uint(sh[e].w);
+        const float4 C = sh[2 * q.cap + e];
         if (REC && !blocked) atomicOr(&q.pathVis[slot], visBit);
         if (defer) {
             q.pendP[slot] = blocked ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(C.x, C.y, C.z, 0.f);
@@ -1043,8 +1053,8 @@ __device__ __forceinline__ void shadowQueue(const P& sc, const WfState& q, const
         const float4 L = q.pathL[slot];
         q.pathL[slot] = make_float4(L.x + C.x, L.y + C.y, L.z + C.z, L.w);
     };
-    traceQueue<W, true, false, P::kMany>(sc.any(), q.gstack, q.gthreads, ws, quads, refill, load, store, tl.cnt,
-                                         tl.rays, tl.overflow);
+    traceQueue<W, true, false, P::kMany>(sc.any(), q.gstack, q.gthreads, ws, quads, refill, load, store, tl.counters,
+                                          tl.cnt, tl.rays);
 }
 
 // One shadow queue of bounce parity q.parity (light: 0 HDRI, 1 point light).
@@ -1054,13 +1064,10 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_shadow(P sc, WfState q, int light, uint32_t ref
     qm.load(q.counters + qShadow(q.parity, light));
     const uint32_t n = qm.total();
     const bool quads = useQuads<W>(sc.any(), n);
-    QueueTally tl;
+    QueueTally tl{counters};
     shadowQueue<W, P, REC>(sc, q, light ? q.shadowP : q.shadowH, qm,
                            chunkSource<P::kMany>(q.counters, chunkShadow(q.parity, light), n, quads), quads, false,
                            q.visBit << light, refill, tl);
-    const int slots[1] = {kStatOverflow};
-    const uint32_t vals[1] = {tl.overflow};
-    blockFlush<1>(counters, slots, vals);
 }
 
 // What follows a shade in one launch: the next bounce's closest hits (rayIn
@@ -1102,7 +1109,7 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_trace(P sc, WfState q, const float4* __restrict
     }
     const uint32_t w = gridWave();
     const int kind = w < wE ? 0 : w < wE + wH ? 1 : 2;
-    QueueTally tl;
+    QueueTally tl{counters};
     QueueMap qm;
     if (kind == 0) {
         qm.load(countIn);
@@ -1118,9 +1125,9 @@ EL_KERNEL(EL_WPE_TRAV) void k_wf_trace(P sc, WfState q, const float4* __restrict
                                refill, tl);
         tl.rays = 0;
     }
-    const int slots[3] = {kStatRays, kStatOverflow, kStatExtRays};
-    const uint32_t vals[3] = {tl.rays, tl.overflow, tl.rays};
-    blockFlush<3>(counters, slots, vals);
+    const int slots[2] = {kStatRays, kStatExtRays};
+    const uint32_t vals[2] = {tl.rays, tl.rays};
+    blockFlush<2>(counters, slots, vals);
 }
 
 // A path's radiance once every launch is done: the last bounce's deferred
@@ -1235,7 +1242,7 @@ EL_KERNEL(EL_WPE_ADJ) void k_adj_bounce(DevScene s, RenderArgs a, WfState q, Adj
             bool hit = false;
             if (i < n) {
                 e = FIRST ? i : (uint32_t)qm.entry(i, q.segSize);
-                const uint32_t slot = FIRST ? i : __float_as_uint(rayIn[2 * (uint64_t)e].w);
+                const uint32_t slot = FIRST ? i : __float_as_uint(rayIn[e].w);
                 uint32_t smp, px, py;
                 const uint32_t pix = slotPixel(s, a, slot, smp, px, py);
                 if (pix != 0xFFFFFFFFu) {
@@ -1279,8 +1286,8 @@ EL_KERNEL(EL_WPE_ADJ) void k_adj_bounce(DevScene s, RenderArgs a, WfState q, Adj
         if (has) {
             v3 o, d, T = mk(1, 1, 1), L = mk(0, 0, 0);
             if (!FIRST) {
-                const float4 A = rayIn[2 * (uint64_t)e], B = rayIn[2 * (uint64_t)e + 1];
-                const float4 C = stateIn[2 * (uint64_t)e], D = stateIn[2 * (uint64_t)e + 1];
+                const float4 A = rayIn[e], B = rayIn[q.cap + e];
+                const float4 C = stateIn[e], D = stateIn[q.cap + e];
                 slot = __float_as_uint(A.w);
                 o = mk(A.x, A.y, A.z);
                 d = mk(B.x, B.y, B.z);
@@ -1327,12 +1334,12 @@ EL_KERNEL(EL_WPE_ADJ) void k_adj_bounce(DevScene s, RenderArgs a, WfState q, Adj
         uint64_t at[3];
         blockAlloc3(want, outCnt, q.segSize, at, overflow);   // ends with a barrier: the pool may be refilled
         if (at[0] != ~0ull) {
-            float4* Q = rayOut + 2 * at[0];
+            float4* Q = rayOut + at[0];
             Q[0] = make_float4(vo.nextO.x, vo.nextO.y, vo.nextO.z, __uint_as_float(slot));
-            Q[1] = make_float4(vo.nextD.x, vo.nextD.y, vo.nextD.z, 0.f);
-            float4* S = stateOut + 2 * at[0];
+            Q[q.cap] = make_float4(vo.nextD.x, vo.nextD.y, vo.nextD.z, 0.f);
+            float4* S = stateOut + at[0];
             S[0] = make_float4(vo.newT.x, vo.newT.y, vo.newT.z, 0.f);
-            S[1] = make_float4(Ln.x, Ln.y, Ln.z, 0.f);
+            S[q.cap] = make_float4(Ln.x, Ln.y, Ln.z, 0.f);
         }
     }
     __syncthreads();
@@ -1386,9 +1393,9 @@ EL_KERNEL(1) void k_bt_camera(ManyScenes sc, const BatchSeg* __restrict__ segs, 
             if (cull) quiet = nanProneBounces(s, rng, (int)maxDepth);
         }
         q.pathQuiet[slot] = quiet;
-        float4* Q = q.ray[0] + 2 * (uint64_t)slot;
+        float4* Q = q.ray[0] + slot;
         Q[0] = make_float4(o.x, o.y, o.z, __uint_as_float(slot));
-        Q[1] = make_float4(d.x, d.y, d.z, __uint_as_float(g.scene));
+        Q[q.cap] = make_float4(d.x, d.y, d.z, __uint_as_float(g.scene));
     }
     if (blockIdx.x == 0 && threadIdx.x < kXcds) q.counters[kQRay0 + threadIdx.x] = threadIdx.x == 0 ? genCount : 0u;
     resetChunks(q.counters, kChunkExt);

@@ -75,9 +75,12 @@ struct RenderArgs {
 };
 
 struct WfState {
-    float4* ray[2];         // ray queues: (o, slot) (d, -) per entry
+    // Queues of `cap` entries, a float4 of an entry in each plane of cap
+    // float4s, so that the lanes of a wave write and read whole lines.
+    float4* ray[2];         // ray queues: (o, slot) (d, scene)
+    uint64_t cap;
     float4* hits;           // (tri, t, u, v) per entry of the current queue
-    float4* shadowH;        // (o, slot) (d, tmax) (contribution) per entry
+    float4* shadowH;        // (o, slot) (d, tmax) (contribution, scene)
     float4* shadowP;
     float4* pathT;          // throughput per path slot (from the first shade on)
     float4* pathL;          // radiance per path slot (from the first shade on)
