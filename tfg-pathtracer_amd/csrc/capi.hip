@@ -947,6 +947,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
             a.genPixel = (uint32_t)(start % npad);
             a.genSample = (uint32_t)(start / npad);
             a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
+            a.run = a.genPixel == 0 && a.genCount % npad == 0 ? (uint32_t)(a.genCount / npad) : 0u;
             a.fresh = c->accPending ? 1u : 0u;
             a.zeroTallies = start == 0 ? 1u : 0u;
             rc = wfWalk(c, lc, a, q, p->flags, timed, ev, ctr);
@@ -1125,6 +1126,7 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
         a.genPixel = (uint32_t)(start % npad);
         a.genSample = (uint32_t)(start / npad);
         a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
+            a.run = a.genPixel == 0 && a.genCount % npad == 0 ? (uint32_t)(a.genCount / npad) : 0u;
         if (!recorded) {
             std::vector<std::pair<size_t, int>> timed;
             size_t ev = 2;
@@ -1689,6 +1691,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
                 s.npad = (uint32_t)npadv[sc];
                 s.wStart = w - sceneBase;
                 s.finStart = g.finTotal;
+                s.run = s.wStart % s.npad == 0 && s.count % s.npad == 0 ? s.count / s.npad : 0u;
                 g.finTotal += std::min<uint32_t>(s.count, s.npad);
                 segs.push_back(s);
                 g.nseg++;

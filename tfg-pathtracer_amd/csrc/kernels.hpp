@@ -56,6 +56,8 @@ struct RenderArgs {
     uint32_t genSample;     //   and sample offset (item = genSample * npad + genPixel)
     uint32_t genCount;      // wavefront: work items in the generation
     uint32_t npad;          // wavefront: padded pixel count (8x8 tiles)
+    uint32_t run;           // wavefront, generation of whole frames: its samples, those of a tile being
+                            // neighbours (slot = (tile * run + sample) * 64 + pixel of the tile); else 0
     uint32_t cull;          // stop zero-throughput paths that cannot turn NaN
     uint32_t fresh;         // wavefront: the accumulation holds nothing yet and is not cleared: finalize
                             // starts a pixel's sums from zero at sample 0 (every pixel has that sample once)
@@ -116,12 +118,13 @@ struct AdjArgs {
 
 // One scene's share of a batch generation: path slots [slotStart,
 // slotStart + count) hold the scene's work items wStart .. (sample-major:
-// w = sample * npad + padded pixel).  finStart: prefix over the generation's
+// w = sample * npad + padded pixel; with `run` the same items in another order).  finStart: prefix over the generation's
 // segments of min(count, npad), the finalize threads of the segment.
 struct BatchSeg {
     uint32_t slotStart, count, scene, npad;
     uint64_t wStart;
-    uint32_t finStart, pad;
+    uint32_t finStart;
+    uint32_t run;   // samples of a segment of whole frames, slots ordered as with RenderArgs::run; else 0
 };
 
 struct LaunchCfg {
