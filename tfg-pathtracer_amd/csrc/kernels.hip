@@ -79,14 +79,17 @@ __device__ __forceinline__ void blockFlush(unsigned long long* counters, const i
 // Whether a launch over n rays of a BVH4 gives each ray to a quad of lanes
 // (traceQuadRange) instead of a lane (traceWaveRange).  A launch that does
 // not fill the GPU lasts as long as one ray's chain of node visits, which is
-// shorter by quads (a visit is ~70 VALU instructions after one 16-byte load
-// instead of ~146 after four; 16 rays share a wave's leaf rounds instead of
+// shorter by quads (a visit is ~60 VALU instructions after one 16-byte load
+// instead of ~115 after four; 16 rays share a wave's leaf rounds instead of
 // 64), while one that does is bound by instruction issue, where a lane per
 // ray needs fewer in all.  Whole calls, lanes against quads: 16,384 rays of
 // the 64-sphere field 92 -> 57 us, 262,144 119 -> 86, 2^20 178 -> 198
-// (occlusion on a 131,072-triangle terrain 249 -> 209), 2^21 294 -> 357; the
+// (occlusion on a 262,144-triangle terrain 249 -> 209), 2^21 294 -> 357; the
 // 256 x 256 frame of 16 samples, whose first launch holds 2^20 rays, 1479 ->
-// 1351 us, a 1920 x 1080 one of one sample (2^21) 2.6 -> 3.1 ms.
+// 1351 us, a 1920 x 1080 one of one sample (2^21) 2.6 -> 3.1 ms.  (Since a
+// lane's visit got shorter, 2^20 random rays take 150 us by lanes and 176 by
+// quads, but occlusion on the terrain 211 and 198, and the 256 x 256 frame the
+// same either way: the line stays.)
 constexpr uint32_t kQuadRays = 1u << 20;
 template <int W>
 __device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n) {
@@ -688,8 +691,8 @@ __device__ __forceinline__ bool workPixel(const DevScene& s, uint32_t p, uint32_
 // triangles and surface records are in their caches, where frame after frame
 // every tile's had to come back for each sample (rendering, frame after frame
 // against tile after tile: 256 x 256 of 16 samples 0.84 -> 0.74 ms, 128 x 128
-// gradient 0.72 -> 0.53, four 1024 x 1024 views' gradient 45.4 -> 42.5, a batch
-// of 32 scenes 10.6 -> 10.4).  Splitting the tiles among the XCDs, by the chunks
+// gradient 0.72 -> 0.53, four 512 x 512 views' gradient 45.4 -> 42.5, a batch
+// of 12 scenes 10.6 -> 10.4).  Splitting the tiles among the XCDs, by the chunks
 // they draw or the blocks' part of the queue, gave nothing more.
 // genPixel + slot < 2^32: both are below 2^31 (checked on the host).
 __device__ __forceinline__ uint32_t slotPixel(const DevScene& s, const RenderArgs& a, uint32_t slot,

@@ -22,7 +22,7 @@ constexpr uint32_t kDefaultBlock = 64;
 constexpr uint32_t kDefaultRefill = 16;
 
 namespace dev {
-constexpr int kAdjMaxDepthHost = 16;   // deepest path the adjoint records (k_adjoint's kAdjMaxDepth)
+constexpr int kAdjMaxDepthHost = 16;   // deepest path the adjoint records
 }
 
 // Tally slots (per XCD copy): the host sums the kXcds copies.
