@@ -874,7 +874,7 @@ __device__ __forceinline__ int visitWords(const uint4* np, const TRay& ray, floa
     const float Ax = (px - ray.ox) * ray.ix, Ay = (py - ray.oy) * ray.iy, Az = (pz - ray.oz) * ray.iz;
     const float Ex = fabsf(Ax * kSlabEps), Ey = fabsf(Ay * kSlabEps), Ez = fabsf(Az * kSlabEps);
     const float Anx = Ax - Ex, Afx = Ax + Ex, Any = Ay - Ey, Afy = Ay + Ey, Anz = Az - Ez, Afz = Az + Ez;
-    tcull *= ray.scale;
+    tcull = (UNSORTED ? tcull : fabsf(tcull)) * ray.scale;
     if constexpr (W == 4) {
         const float Bx = sx * (ray.ix * kSlabScaleInv), By = sy * (ray.iy * kSlabScaleInv), Bz = sz * (ray.iz * kSlabScaleInv);
         const PlaneSel sel = planeSel(ray.ix, ray.iy, ray.iz);
