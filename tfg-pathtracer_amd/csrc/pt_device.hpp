@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "child_order.hpp"
 #include "hdri_table.hpp"
 
 namespace eleven {
@@ -883,11 +884,11 @@ __device__ __forceinline__ int visitWords(const uint4* np, const TRay& ray, floa
         for (int i = 0; i < 4; i++) {
             const HalfPair n = planePair(np[i], sel.nearXY), f = planePair(np[i], sel.farXY), z = planePair(np[i], sel.z);
             const float tz = __builtin_amdgcn_fmed3f(fmaf((float)z.x, Bz, Anz), 0.0f, 1.0f);
-            const float tn = fmaxf(fmaxf(fmaf((float)n.x, Bx, Anx), fmaf((float)n.y, By, Any)), tz);
+            const float tn = entryDistance(fmaf((float)n.x, Bx, Anx), fmaf((float)n.y, By, Any), tz);
             float tf = fminf(fmaf((float)z.y, Bz, Afz), tcull);
             tf = fminf(fminf(fmaf((float)f.x, Bx, Afx), fmaf((float)f.y, By, Afy)), tf) * (1.0f + kFarEps);
             miss[i] = (uint32_t)((__float_as_int(tf - tn) | (int)np[i].y) >> 31);
-            key[i] = __float_as_uint(tn) | miss[i];
+            key[i] = childKey(__float_as_uint(tn), miss[i]);
         }
         st.room();
         if constexpr (UNSORTED) {
@@ -896,10 +897,8 @@ __device__ __forceinline__ int visitWords(const uint4* np, const TRay& ray, floa
                 if (!miss[i]) st.push((int)np[i].x);
             return st.pop();
         } else {
-            auto nearer = [&](int i, int j) { return (key[i] - key[j]) >> 31; };
-            const uint32_t c01 = nearer(0, 1), c02 = nearer(0, 2), c03 = nearer(0, 3), c12 = nearer(1, 2),
-                           c13 = nearer(1, 3), c23 = nearer(2, 3);
-            const uint32_t above[4] = {c01 + c02 + c03, 1u - c01 + c12 + c13, 2u - c02 - c12 + c23, 3u - c03 - c13 - c23};
+            uint32_t above[4];
+            childRows(key, above);
 #pragma unroll
             for (int i = 0; i < 4; i++) st.at(st.sp + above[i] * kStackRow) = (int)np[i].x;
             st.sp += (4u + miss[0] + miss[1] + miss[2] + miss[3]) * kStackRow;
@@ -1404,10 +1403,10 @@ __device__ __forceinline__ void visitQuad(const uint4* __restrict__ nodes, int c
         at += (uint32_t)__popc(nib >> (j + 1)) * kQuadEntry;   // below the children taken after it
     } else {
         // distances as non-negative integers, so that a difference's sign bit is the comparison
-        const int key = hit ? (int)((__float_as_uint(tn) & ~3u) | j) : 0x7fffffff;
-        const uint32_t nearer = ((uint32_t)((int)quadXor<1>((uint32_t)key) - key) >> 31) +
-                                ((uint32_t)((int)quadXor<2>((uint32_t)key) - key) >> 31) +
-                                ((uint32_t)((int)quadXor<3>((uint32_t)key) - key) >> 31);
+        const int key = childKeyOfLane(__float_as_uint(tn), j, hit);
+        const uint32_t nearer = nearerKey((int)quadXor<1>((uint32_t)key), key) +
+                                nearerKey((int)quadXor<2>((uint32_t)key), key) +
+                                nearerKey((int)quadXor<3>((uint32_t)key), key);
         uint32_t c = hit ? kQuadEntry : 0u;
         c += quadXor<1>(c);
         top = c + quadXor<2>(c);
