@@ -25,6 +25,7 @@
 
 #include "child_order.hpp"
 #include "hdri_table.hpp"
+#include "work_turns.hpp"
 
 namespace eleven {
 namespace dev {
@@ -1144,21 +1145,15 @@ struct WorkSource {
 
 // A wave's place in its items (wave-uniform).
 struct WorkCursor {
-    uint32_t cursor = 0, end = 0, turn = 0, place;   // in turn: `place` among the waves in the turn that starts at `turn`
+    uint32_t cursor = 0, end = 0;
+    WorkTurns turns;
     uint32_t tried = 0;      // narrow source: shares found drawn out
-    __device__ __forceinline__ WorkCursor(const WorkSource& ws) : place(ws.first) {}
+    __device__ __forceinline__ WorkCursor(const WorkSource& ws) : turns(ws.first) {}
     // The next chunk after [cursor, end) is used up; false: no items left.
     // The whole wave must call.
     template <bool WIDE>
     __device__ __forceinline__ bool draw(const WorkSource& ws) {
-        if (ws.waves) {
-            const uint32_t c = turn + place;
-            turn += ws.waves;
-            place += (ws.waves * 5) >> 3;
-            place -= place >= ws.waves ? ws.waves : 0u;
-            if (ws.chunks - turn < ws.waves) place = ws.first;   // the last turn, which the waves that start last miss
-            return take(ws, c);
-        }
+        if (ws.waves) return take(ws, turns.next(ws.waves, ws.chunks, ws.first));
         const uint32_t lane = __lane_id();
         // Wide sources (batches, parts == 64): lane l looks at share
         // (home + l) % 64 at once (one load per lane instead of 64
@@ -1223,7 +1218,7 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
         const unsigned long long idle = waveMask(!live);
         const uint32_t nIdle = (uint32_t)__popcll(idle);
         const bool want = nIdle >= refill || nIdle == 64;
-        if (want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
+        if (more && want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
         if (want && more) {
             if (!live) {
                 uint32_t i = wc.cursor + lanesBelow(idle);
@@ -1477,7 +1472,7 @@ __device__ __forceinline__ void traceQuadRange(const DevScene& s, QuadStack& st,
         const unsigned long long idle = waveMask(!live);
         const uint32_t nIdle = (uint32_t)__popcll(idle);
         const bool want = nIdle >= refill || nIdle == 64;
-        if (want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
+        if (more && want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
         if (want && more) {
             if (!live) {
                 const uint32_t i = wc.cursor + (lanesBelow(idle) >> 2);   // quads are idle as a whole
