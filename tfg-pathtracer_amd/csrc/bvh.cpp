@@ -299,6 +299,9 @@ void packWide(const Bvh2& b, const float pad, WideBvh& out) {
             if (!quantizeNode<W>(wn[i], qn[i])) finite = false;
     });
     if (!finite) throw std::runtime_error("non-finite bounding box (vertex data)");
+    for (const QNode<W>& n : qn)
+        for (int a = 0; a < 3; a++)
+            out.maxStepExponent = std::max(out.maxStepExponent, (int)((n.exps >> (8 * a)) & 0xffu) - 127);
     out.nodes.resize(qn.size() * sizeof(QNode<W>));
     std::memcpy(out.nodes.data(), qn.data(), out.nodes.size());
     out.stackBound = std::max(1, maxStack);

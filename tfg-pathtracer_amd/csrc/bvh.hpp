@@ -90,6 +90,7 @@ struct WideBvh {
     std::vector<int> order;             // leaf order -> original index
     int stackBound = 0;                 // worst-case traversal stack depth
     int depth = 0;                      // wide-tree depth (root = 1)
+    int maxStepExponent = -126;         // of the largest grid step (a power of two) of a node on any axis
     float sceneLo[3] = {0, 0, 0}, sceneHi[3] = {0, 0, 0};
 };
 

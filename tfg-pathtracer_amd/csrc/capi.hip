@@ -454,6 +454,7 @@ static int uploadBvh(el_ctx* c, int width) {
     c->ds.width = width;
     c->ds.gcap = c->gcap;
     c->ds.quads = width == 4 && c->wide.stackBound + 2 <= dev::kQuadStack;
+    c->ds.slabUnit = dev::slabUnitOf(c->wide.maxStepExponent);
     c->stats.bvh_width = (uint32_t)width;
     c->stats.stack_bound = (uint32_t)c->wide.stackBound;
     c->stats.node_bytes = c->wide.nodes.size();
@@ -1633,11 +1634,13 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         }
         b->width = width;
     }
-    // scene records: shared spill capacity, per-scene key and accumulation
+    // scene records: shared spill capacity and slab unit, per-scene key and accumulation
     int gcap = 1, quads = 1;
+    float slabUnit = 1.0f;
     for (auto* c : b->scenes) {
         gcap = std::max(gcap, c->gcap);
         quads &= c->ds.quads;
+        slabUnit = std::min(slabUnit, c->ds.slabUnit);
     }
     std::vector<DevScene> recs(S);
     std::vector<uint64_t> work(S), npadv(S);
@@ -1647,6 +1650,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         recs[i] = c->ds;
         recs[i].gcap = gcap;
         recs[i].quads = quads;
+        recs[i].slabUnit = slabUnit;
         recs[i].seedLo = (uint32_t)b->seed[i];
         recs[i].seedHi = (uint32_t)(b->seed[i] >> 32);
         recs[i].accum = c->dAccum.as<float4>();

@@ -23,6 +23,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "child_order.hpp"
 #include "hdri_table.hpp"
 #include "work_turns.hpp"
@@ -176,6 +179,7 @@ struct DevScene {
     int32_t width;                 // BVH width (4 or 8)
     int32_t gcap;                  // global stack entries per thread (a stack per lane)
     int32_t quads;                 // BVH4 within kQuadStack: short queues give a ray to a quad of lanes
+    float slabUnit;                // factor of the slab distances' scale (slabUnitOf)
     DevCamera cam;
     // batches only: the scene's RNG key and accumulation buffers
     uint32_t seedLo, seedHi;
@@ -801,16 +805,28 @@ __device__ __forceinline__ HalfPair planePair(const uint4& w, uint32_t sel) {
 // step / direction) finite down to components of 1e-30, and near planes below 1,
 // where they may be clamped for nothing (fma's clamp modifier), for distances up to
 // 2^24.  A direction longer than 2^20 takes scale 1 instead, as its distances would
-// become denormal otherwise, and components of 2^24 * 1e-30 count as zero.
+// become denormal otherwise, and components of 2^24 * 1e-30 count as zero.  Either
+// is multiplied by the scene's slabUnit: 1, or less where the grid steps of its
+// nodes are so large (2^28 and more) that 2^24 step / direction overflows all the same.
+// A plane distance may overflow by its node's origin, which misses nothing (an
+// infinity less its widening is no number, and the axis is left out), but
+// not by the step alone: a near plane behind the ray would be infinitely far ahead.
 constexpr float kSlabScale = 1.0f / 16777216.0f, kSlabScaleInv = 16777216.0f;
-__device__ __forceinline__ float slabScale(float dx, float dy, float dz) {
-    return fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz)) > 1048576.0f ? 1.0f : kSlabScale;
+struct SlabScale {
+    float scale, tiny;   // tiny: the smallest direction component told from zero
+};
+__device__ __forceinline__ SlabScale slabScale(float dx, float dy, float dz, float unit) {
+    const bool longer = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz)) > 1048576.0f;
+    return SlabScale{longer ? unit : kSlabScale * unit, longer ? 1e-30f * kSlabScaleInv : 1e-30f};
 }
 // Scaled reciprocal of a direction component for the slab tests (at most 2^-24 * 1e30).
-__device__ __forceinline__ float slabInv(float d, float scale) {
-    const float tiny = 1e-30f * (scale * kSlabScaleInv);
-    return 1.0f / (fabsf(d) > tiny ? d : copysignf(tiny, d)) * scale;
+__device__ __forceinline__ float slabInv(float d, const SlabScale& c) {
+    return 1.0f / (fabsf(d) > c.tiny ? d : copysignf(c.tiny, d)) * c.scale;
 }
+// The slabUnit of a scene whose largest grid step is 2^exponent: 2^24 step * kSlabScale / 1e-30 is then below
+// 2^127.  No less than 2^-82, which keeps the reciprocals of components up to 2^20 normal numbers: with steps
+// of 2^109 a triangle's determinant has long overflown.
+inline float slabUnitOf(int exponent) { return std::ldexp(1.0f, std::max(-82, std::min(0, 27 - exponent))); }
 // Widening of a slab distance A + q B: near planes use A - |A| kSlabEps, far planes A + |A| kSlabEps (see visitWords).
 constexpr float kSlabEps = 1.0f / 524288.0f, kFarEps = 1.0f / 1048576.0f;
 
@@ -819,9 +835,9 @@ struct TRay {
     float ox, oy, oz, dx, dy, dz, ix, iy, iz, scale;
 };
 
-__device__ __forceinline__ TRay makeTRay(float ox, float oy, float oz, float dx, float dy, float dz) {
-    const float c = slabScale(dx, dy, dz);
-    return TRay{ox, oy, oz, dx, dy, dz, slabInv(dx, c), slabInv(dy, c), slabInv(dz, c), c};
+__device__ __forceinline__ TRay makeTRay(float ox, float oy, float oz, float dx, float dy, float dz, float unit) {
+    const SlabScale c = slabScale(dx, dy, dz, unit);
+    return TRay{ox, oy, oz, dx, dy, dz, slabInv(dx, c), slabInv(dy, c), slabInv(dz, c), c.scale};
 }
 
 // Visits an inner node: slab-tests its W children against [0, tcull] and
@@ -1054,7 +1070,7 @@ template <int W, bool ANY, bool COUNT>
 __device__ __forceinline__ TraceResult traceRay(const DevScene& s, float ox, float oy, float oz, float dx, float dy,
                                                 float dz, float tmax, TravStack& st, TraceCounters& cnt) {
     const uint4* __restrict__ nodes = (const uint4*)s.nodes;
-    const TRay ray = makeTRay(ox, oy, oz, dx, dy, dz);
+    const TRay ray = makeTRay(ox, oy, oz, dx, dy, dz, s.slabUnit);
     TraceResult r;
     r.tri = -1;
     r.t = tmax;
@@ -1227,7 +1243,7 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
                     BvhPtr rb = bvh;
                     if (load(i, ox, oy, oz, dx, dy, dz, tmax, rb, item)) {
                         if (PER_RAY_BVH) bvh = rb;
-                        ray = makeTRay(ox, oy, oz, dx, dy, dz);
+                        ray = makeTRay(ox, oy, oz, dx, dy, dz, s.slabUnit);
                         r.tri = -1;
                         r.t = tmax;
                         r.u = r.v = 0.f;
@@ -1364,11 +1380,12 @@ struct QuadRay {
     PlaneSel sel;
 };
 __device__ __forceinline__ QuadRay makeQuadRay(float ox, float oy, float oz, float dx, float dy, float dz,
-                                               uint32_t j) {
+                                               float unit, uint32_t j) {
     QuadRay r{ox, oy, oz, dx, dy, dz};
     r.oa = j == 0 ? ox : j == 1 ? oy : oz;
-    r.scale = slabScale(dx, dy, dz);
-    r.ia = slabInv(j == 0 ? dx : j == 1 ? dy : dz, r.scale);
+    const SlabScale c = slabScale(dx, dy, dz, unit);
+    r.scale = c.scale;
+    r.ia = slabInv(j == 0 ? dx : j == 1 ? dy : dz, c);
     r.sel = planeSel(quadLane<0>(r.ia), quadLane<1>(r.ia), quadLane<2>(r.ia));
     return r;
 }
@@ -1481,7 +1498,7 @@ __device__ __forceinline__ void traceQuadRange(const DevScene& s, QuadStack& st,
                     BvhPtr rb = bvh;
                     if (load(i, ox, oy, oz, dx, dy, dz, tmax, rb, item)) {
                         if (PER_RAY_BVH) bvh = rb;
-                        ray = makeQuadRay(ox, oy, oz, dx, dy, dz, j);
+                        ray = makeQuadRay(ox, oy, oz, dx, dy, dz, s.slabUnit, j);
                         r.tri = -1;
                         r.t = tmax;
                         r.u = r.v = 0.f;
