@@ -22,6 +22,7 @@
 
 #include "../../include/eleven.h"
 #include "bvh.hpp"
+#include "dev_buf.hpp"
 #include "hdri_table.hpp"
 #include "host_parallel.hpp"
 #include "kernels.hpp"
@@ -32,32 +33,6 @@ using namespace eleven;
 using eleven::dev::DevScene;
 
 namespace {
-
-struct DevBuf {
-    void* p = nullptr;
-    size_t n = 0;
-    DevBuf() = default;
-    DevBuf(const DevBuf&) = delete;
-    DevBuf& operator=(const DevBuf&) = delete;
-    ~DevBuf() { release(); }
-    void release() {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        n = 0;
-    }
-    hipError_t ensure(size_t bytes) {
-        if (bytes <= n && p) return hipSuccess;
-        release();
-        if (bytes == 0) bytes = 16;
-        hipError_t e = hipMalloc(&p, bytes);
-        if (e == hipSuccess) n = bytes;
-        return e;
-    }
-    template <class T>
-    T* as() const {
-        return (T*)p;
-    }
-};
 
 constexpr int kCounterWords = kXcds * kStatSlots;   // per-XCD copies of the tallies (kernels.hpp)
 
@@ -1794,8 +1769,9 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
                           std::to_string(p->flags & ~EL_BATCH_GRAPH) + "/" + std::to_string(plan) + "/" +
                           std::to_string(lc.block) + "/" + std::to_string(lc.refill) + "/" + std::to_string(Q) +
                           "/" + std::to_string(sppCap) + "/" + std::to_string(total) + "/" +
-                          std::to_string((uintptr_t)b->dSegs.p) + "/" + std::to_string((uintptr_t)b->wRay0.p) +
-                          "/" + std::to_string((uintptr_t)b->dScenes.p) + "/" + std::to_string((uintptr_t)b->dGstack.p);
+                          std::to_string(allocationsOf(b->dScenes, b->dSegs, b->dGstack, b->dCounters, b->wRay0, b->wRay1,
+                                                       b->wHits, b->wShH, b->wShP, b->wT, b->wL, b->wPix, b->wSample,
+                                                       b->wQuiet, b->wPend, b->wCounters));
         if (!b->graph || key != b->graphKey) {
             if (b->graph) {
                 EL_BHIP(b, hipGraphExecDestroy(b->graph));
