@@ -28,6 +28,7 @@
 #include "kernels.hpp"
 #include "pt_device.hpp"
 #include "scene.hpp"
+#include "wf_buffers.hpp"
 
 using namespace eleven;
 using eleven::dev::DevScene;
@@ -207,8 +208,7 @@ struct el_ctx {
 
     DevBuf dNodes, dTris, dShade, dMats, dTexs, dTexels, dLights, dEnvCdf, dEnvGuide, dEnvMap, dEnvBad, dEnvTab, dTexels8, dTexLut, dTangents;
     DevBuf dGstack, dAccum, dCounts, dAov, dCounters;
-    DevBuf wRay0, wRay1, wHits, wShH, wShP, wT, wL, wPix, wSample, wQuiet, wAov, wCounters, wPend;
-    size_t wfCap = 0, wfQcap = 0;
+    WfBuffers wf;
 
     DevBuf tRays, tTmax, tTri, tT, tUV, tOcc;   // scratch for host-pointer ray queries
 
@@ -685,31 +685,6 @@ static hipEvent_t poolEvent(el_ctx* c, size_t i) {
     return c->evPool[i];
 }
 
-// Path slots: `cap`; queue entries: max(cap, kXcds * segSize) (the camera
-// queue is indexed by slot, the compacted queues by XCD segment).  Every
-// buffer keeps the largest size asked of it (DevBuf::ensure); the per-path
-// AOV buffer is sized by this call's capacity whatever the others hold, since
-// renders without AOV may have grown them past its size.
-static int ensureWf(el_ctx* c, size_t cap, size_t qcap, bool aov) {
-    if (aov) EL_HIP(c, c->wAov.ensure(cap * 48));
-    if (cap <= c->wfCap && qcap <= c->wfQcap) return EL_OK;
-    EL_HIP(c, c->wRay0.ensure(qcap * 32));
-    EL_HIP(c, c->wRay1.ensure(qcap * 32));
-    EL_HIP(c, c->wHits.ensure(qcap * 16));
-    EL_HIP(c, c->wShH.ensure(qcap * 48));
-    EL_HIP(c, c->wShP.ensure(qcap * 48));
-    EL_HIP(c, c->wT.ensure(cap * 16));
-    EL_HIP(c, c->wL.ensure(cap * 16));
-    EL_HIP(c, c->wPix.ensure(cap * 4));
-    EL_HIP(c, c->wSample.ensure(cap * 4));
-    EL_HIP(c, c->wQuiet.ensure(cap * 8));
-    EL_HIP(c, c->wPend.ensure(cap * 16));
-    EL_HIP(c, c->wCounters.ensure(kQCounters * sizeof(uint32_t)));
-    c->wfCap = std::max(c->wfCap, cap);
-    c->wfQcap = std::max(c->wfQcap, qcap);
-    return EL_OK;
-}
-
 // Generation size and wavefront state for `total` work items of a frame
 // with `npad` padded pixels: Q paths per generation (queueCap, or by default
 // as many as a quarter of the free device memory holds), rounded to whole
@@ -720,7 +695,7 @@ static int wfPlan(el_ctx* c, const LaunchCfg& lc, uint64_t total, uint64_t npad,
     // memory holds (~216 B of queue and path state per path), so a
     // 1080p x 64 spp frame runs as a single generation.
     Q = queueCap;
-    if (!Q && total <= c->wfCap && (!aov || c->wAov.n >= total * 48)) Q = total;   // held already
+    if (!Q && total <= c->wf.cap && (!aov || c->wf.aov.n >= total * 48)) Q = total;   // held already
     if (!Q) {
         size_t freeB = 0, totalB = 0;
         EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
@@ -738,26 +713,22 @@ static int wfPlan(el_ctx* c, const LaunchCfg& lc, uint64_t total, uint64_t npad,
     // block <= kMaxBlock).
     const uint64_t segSize = (Q + kXcds - 1) / kXcds + lc.maxThreads / kXcds + kMaxBlock;
     const uint64_t qcap = std::max<uint64_t>(Q, kXcds * segSize);
-    int rc = ensureWf(c, Q, qcap, aov);
-    if (rc) return rc;
-    // the launches index Q path slots and qcap queue entries in every buffer
-    if (c->wRay0.n < qcap * 32 || c->wRay1.n < qcap * 32 || c->wHits.n < qcap * 16 || c->wShH.n < qcap * 48 ||
-        c->wShP.n < qcap * 48 || c->wT.n < Q * 16 || c->wL.n < Q * 16 || c->wPix.n < Q * 4 || c->wSample.n < Q * 4 ||
-        c->wQuiet.n < Q * 8 || c->wPend.n < Q * 16 || (aov && c->wAov.n < Q * 48))
+    EL_HIP(c, c->wf.ensure(Q, qcap, aov, kQCounters * sizeof(uint32_t)));
+    if (!c->wf.holds(Q, qcap, aov))
         return fail(c, EL_ERR_STATE, "wavefront buffers smaller than the generation (internal error)");
-    q.ray[0] = c->wRay0.as<float4>();
-    q.ray[1] = c->wRay1.as<float4>();
-    q.hits = c->wHits.as<float4>();
-    q.shadowH = c->wShH.as<float4>();
-    q.shadowP = c->wShP.as<float4>();
-    q.pathT = c->wT.as<float4>();
-    q.pathL = c->wL.as<float4>();
-    q.pathPix = c->wPix.as<uint32_t>();
-    q.pathSample = c->wSample.as<uint32_t>();
-    q.pathQuiet = c->wQuiet.as<uint64_t>();
-    q.pathAov = aov ? c->wAov.as<float4>() : nullptr;
-    q.pendP = c->wPend.as<float4>();
-    q.counters = c->wCounters.as<uint32_t>();
+    q.ray[0] = c->wf.ray0.as<float4>();
+    q.ray[1] = c->wf.ray1.as<float4>();
+    q.hits = c->wf.hits.as<float4>();
+    q.shadowH = c->wf.shadowH.as<float4>();
+    q.shadowP = c->wf.shadowP.as<float4>();
+    q.pathT = c->wf.pathT.as<float4>();
+    q.pathL = c->wf.pathL.as<float4>();
+    q.pathPix = c->wf.pix.as<uint32_t>();
+    q.pathSample = c->wf.sample.as<uint32_t>();
+    q.pathQuiet = c->wf.quiet.as<uint64_t>();
+    q.pathAov = aov ? c->wf.aov.as<float4>() : nullptr;
+    q.pendP = c->wf.pend.as<float4>();
+    q.counters = c->wf.counters.as<uint32_t>();
     q.segSize = (uint32_t)segSize;
     q.cap = qcap;
     q.gstack = lc.gstack;
@@ -1070,10 +1041,10 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     WfState q{};
     const uint64_t perPath = 6 * 32 + 60 + (recorded ? 0 : 16 * depth + 4);
     uint64_t budget = kAdjointBytes;
-    if (c->wfCap < std::min(total, budget / perPath)) {   // buffers will grow: by a quarter of what is free, as a render's
+    if (c->wf.cap < std::min(total, budget / perPath)) {   // buffers will grow: by a quarter of what is free, as a render's
         size_t freeB = 0, totalB = 0;
         EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
-        budget = std::min<uint64_t>(budget, std::max<uint64_t>(freeB / 4, c->wfCap * perPath));
+        budget = std::min<uint64_t>(budget, std::max<uint64_t>(freeB / 4, c->wf.cap * perPath));
     }
     const uint64_t cap = std::max<uint64_t>(1u << 16, budget / perPath);
     int rc = wfPlan(c, lc, total, npad, cap, false, q, Q);
@@ -1460,8 +1431,7 @@ struct el_batch {
     std::vector<uint64_t> seed;
     int width = 4;
     DevBuf dScenes, dSegs, dGstack, dCounters;
-    DevBuf wRay0, wRay1, wHits, wShH, wShP, wT, wL, wPix, wSample, wQuiet, wPend, wCounters;
-    size_t wfCap = 0, wfQcap = 0;
+    WfBuffers wf;
     hipGraphExec_t graph = nullptr;
     std::string graphKey;
     el_stats stats{};
@@ -1570,25 +1540,6 @@ int el_batch_stats(el_batch* b, el_stats* out) {
 
 }  // extern "C"
 
-static int batchEnsureWf(el_batch* b, size_t cap, size_t qcap) {
-    if (cap <= b->wfCap && qcap <= b->wfQcap) return EL_OK;
-    EL_BHIP(b, b->wRay0.ensure(qcap * 32));
-    EL_BHIP(b, b->wRay1.ensure(qcap * 32));
-    EL_BHIP(b, b->wHits.ensure(qcap * 16));
-    EL_BHIP(b, b->wShH.ensure(qcap * 48));
-    EL_BHIP(b, b->wShP.ensure(qcap * 48));
-    EL_BHIP(b, b->wT.ensure(cap * 16));
-    EL_BHIP(b, b->wL.ensure(cap * 16));
-    EL_BHIP(b, b->wPix.ensure(cap * 4));
-    EL_BHIP(b, b->wSample.ensure(cap * 4));
-    EL_BHIP(b, b->wQuiet.ensure(cap * 8));
-    EL_BHIP(b, b->wPend.ensure(cap * 16));
-    EL_BHIP(b, b->wCounters.ensure(kQCounters * sizeof(uint32_t)));
-    b->wfCap = std::max(b->wfCap, cap);
-    b->wfQcap = std::max(b->wfQcap, qcap);
-    return EL_OK;
-}
-
 // Renders every scene of the batch from a cleared accumulation with spp[i]
 // (capped at sppCap if nonzero).  Returns the device time in *ms.
 static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, double* ms) {
@@ -1689,22 +1640,23 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
     lc.gstack = b->dGstack.as<int>();
     const uint64_t segSize = (Q + kXcds - 1) / kXcds + lc.maxThreads / kXcds + kMaxBlock;
     const uint64_t qcap = std::max<uint64_t>(Q, kXcds * segSize);
-    int rc = batchEnsureWf(b, Q, qcap);
-    if (rc) return rc;
+    EL_BHIP(b, b->wf.ensure(Q, qcap, false, kQCounters * sizeof(uint32_t)));
+    if (!b->wf.holds(Q, qcap, false))
+        return bfail(b, EL_ERR_STATE, "wavefront buffers smaller than the generation (internal error)");
     WfState q{};
-    q.ray[0] = b->wRay0.as<float4>();
-    q.ray[1] = b->wRay1.as<float4>();
-    q.hits = b->wHits.as<float4>();
-    q.shadowH = b->wShH.as<float4>();
-    q.shadowP = b->wShP.as<float4>();
-    q.pathT = b->wT.as<float4>();
-    q.pathL = b->wL.as<float4>();
-    q.pathPix = b->wPix.as<uint32_t>();
-    q.pathSample = b->wSample.as<uint32_t>();
-    q.pathQuiet = b->wQuiet.as<uint64_t>();
+    q.ray[0] = b->wf.ray0.as<float4>();
+    q.ray[1] = b->wf.ray1.as<float4>();
+    q.hits = b->wf.hits.as<float4>();
+    q.shadowH = b->wf.shadowH.as<float4>();
+    q.shadowP = b->wf.shadowP.as<float4>();
+    q.pathT = b->wf.pathT.as<float4>();
+    q.pathL = b->wf.pathL.as<float4>();
+    q.pathPix = b->wf.pix.as<uint32_t>();
+    q.pathSample = b->wf.sample.as<uint32_t>();
+    q.pathQuiet = b->wf.quiet.as<uint64_t>();
     q.pathAov = nullptr;
-    q.pendP = b->wPend.as<float4>();
-    q.counters = b->wCounters.as<uint32_t>();
+    q.pendP = b->wf.pend.as<float4>();
+    q.counters = b->wf.counters.as<uint32_t>();
     q.segSize = (uint32_t)segSize;
     q.cap = qcap;
     q.gstack = lc.gstack;
@@ -1769,9 +1721,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
                           std::to_string(p->flags & ~EL_BATCH_GRAPH) + "/" + std::to_string(plan) + "/" +
                           std::to_string(lc.block) + "/" + std::to_string(lc.refill) + "/" + std::to_string(Q) +
                           "/" + std::to_string(sppCap) + "/" + std::to_string(total) + "/" +
-                          std::to_string(allocationsOf(b->dScenes, b->dSegs, b->dGstack, b->dCounters, b->wRay0, b->wRay1,
-                                                       b->wHits, b->wShH, b->wShP, b->wT, b->wL, b->wPix, b->wSample,
-                                                       b->wQuiet, b->wPend, b->wCounters));
+                          std::to_string(allocationsOf(b->dScenes, b->dSegs, b->dGstack, b->dCounters) + b->wf.allocations());
         if (!b->graph || key != b->graphKey) {
             if (b->graph) {
                 EL_BHIP(b, hipGraphExecDestroy(b->graph));
