@@ -28,6 +28,7 @@
 #include "kernels.hpp"
 #include "pt_device.hpp"
 #include "scene.hpp"
+#include "stage.hpp"
 #include "wf_buffers.hpp"
 
 using namespace eleven;
@@ -37,111 +38,7 @@ namespace {
 
 constexpr int kCounterWords = kXcds * kStatSlots;   // per-XCD copies of the tallies (kernels.hpp)
 
-// Host memory that the GPU writes results to on their way to the caller's
-// arrays, which are pageable: two chunks in turn, one filled by the GPU while
-// the other is copied out.
-struct Stage {
-    static constexpr size_t kChunk = 4u << 20;
-    unsigned char* p = nullptr;
-    size_t n = 0;   // bytes of a chunk
-    bool two = false;
-    hipEvent_t filled[2] = {nullptr, nullptr};
-    unsigned long long* tallies = nullptr;   // kCounterWords
-    Stage() = default;
-    Stage(const Stage&) = delete;
-    Stage& operator=(const Stage&) = delete;
-    ~Stage() {
-        if (p) (void)hipHostFree(p);
-        if (tallies) (void)hipHostFree(tallies);
-        for (auto e : filled)
-            if (e) (void)hipEventDestroy(e);
-    }
-    hipError_t ensureTallies() {
-        if (tallies) return hipSuccess;
-        return hipHostMalloc((void**)&tallies, sizeof(unsigned long long) * kCounterWords, hipHostMallocDefault);
-    }
-    hipError_t ensure(size_t bytes) {
-        const size_t want = std::min(kChunk, std::max<size_t>(64u << 10, bytes));
-        const bool both = bytes > kChunk;
-        for (auto& e : filled)
-            if (!e)
-                if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming); r != hipSuccess) return r;
-        if (p && want <= n && both <= two) return hipSuccess;
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
-        n = 0;
-        const hipError_t r = hipHostMalloc((void**)&p, want * (both ? 2 : 1), hipHostMallocDefault);
-        if (r != hipSuccess) return r;
-        n = want;
-        two = both;
-        return hipSuccess;
-    }
-};
-
-// Takes `items` items of `itemBytes` through the stage: fill(first, n, chunk)
-// enqueues on `stream` what writes the items [first, first + n) to a chunk,
-// copy(first, n, chunk, i0, i1) copies the chunk's items [i0, i1) out, on up
-// to 8 host threads (a thread per MB: a frame's copy is bound by the page
-// faults of the caller's fresh arrays, which one thread takes one at a time).
-template <class Fill, class Copy>
-hipError_t stageOut(Stage& st, hipStream_t stream, size_t items, size_t itemBytes, Fill&& fill, Copy&& copy) {
-    if (!items) return hipSuccess;
-    hipError_t e = st.ensure(items * itemBytes);
-    if (e != hipSuccess) return e;
-    const size_t per = st.n / itemBytes, chunks = (items + per - 1) / per;
-    auto count = [&](size_t k) { return std::min(per, items - k * per); };
-    auto chunk = [&](size_t k) { return st.p + (k & 1) * st.n; };
-    auto issue = [&](size_t k) -> hipError_t {
-        hipError_t r = fill(k * per, count(k), chunk(k));
-        return r == hipSuccess ? hipEventRecord(st.filled[k & 1], stream) : r;
-    };
-    std::atomic<size_t> ready{0}, done{0};   // chunks filled; thread-chunks copied
-    std::atomic<bool> failed{false};         // no further chunk gets ready
-    std::atomic<size_t> team{0};             // threads that share a chunk, once known
-    auto part = [&](size_t k, size_t t) {
-        const size_t n = count(k), T = team.load(std::memory_order_relaxed);
-        copy(k * per, n, chunk(k), n * t / T, n * (t + 1) / T);
-    };
-    auto work = [&](size_t t) {
-        while (!team.load(std::memory_order_acquire)) std::this_thread::yield();
-        for (size_t k = 0; k < chunks; k++) {
-            while (ready.load(std::memory_order_acquire) <= k) {
-                if (failed.load(std::memory_order_acquire)) return;
-                std::this_thread::yield();
-            }
-            part(k, t);
-            done.fetch_add(1, std::memory_order_release);
-        }
-    };
-    const size_t wantThreads = std::min<size_t>({(size_t)hostThreads(), 8, items * itemBytes >> 20});
-    std::vector<std::thread> threads;
-    for (size_t k = 0; k < std::min<size_t>(chunks, 2) && e == hipSuccess; k++) e = issue(k);
-    if (e == hipSuccess) {
-        try {
-            threads.reserve(wantThreads);
-            for (size_t t = 1; t < wantThreads; t++) threads.emplace_back(work, t);
-        } catch (...) {   // fewer threads share the work
-        }
-    }
-    const size_t T = threads.size() + 1;
-    team.store(T, std::memory_order_release);
-    for (size_t k = 0; k < chunks && e == hipSuccess; k++) {
-        e = hipEventSynchronize(st.filled[k & 1]);
-        if (e != hipSuccess) break;
-        ready.store(k + 1, std::memory_order_release);
-        part(k, 0);
-        if (k + 2 < chunks) {   // the chunk is filled again once every thread has copied its share
-            while (done.load(std::memory_order_acquire) < (k + 1) * (T - 1)) std::this_thread::yield();
-            e = issue(k + 2);
-        }
-    }
-    if (e != hipSuccess) failed.store(true, std::memory_order_release);
-    for (auto& t : threads) t.join();
-    // an error leaves nothing in flight that writes the stage
-    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
-    return e;
-}
-
+static_assert(kCounterWords <= (int)Stage::kTallyWords, "the stage holds the tallies");
 
 // Sum of the per-XCD copies of tally `slot`.
 inline unsigned long long tally(const unsigned long long* h, int slot) {
@@ -230,7 +127,6 @@ struct el_ctx {
     size_t residualPx = 0;         // aImage holds el_residual_l2's residual for this many pixels (0: none)
     el_stats stats{};
     bool aovOn = false;
-    std::shared_ptr<Stage> stage;   // one for all scenes of a batch
 
     std::vector<hipEvent_t> evPool;
 };
@@ -256,11 +152,14 @@ static hipError_t upload(DevBuf& b, const void* src, size_t bytes, hipStream_t s
     return e;
 }
 
-// The tallies to c->stage->tallies; waits for the stream.
-static hipError_t readTallies(el_ctx* c, const unsigned long long* ctr) {
-    const hipError_t e = hipMemcpyAsync(c->stage->tallies, ctr, sizeof(unsigned long long) * kCounterWords,
-                                        hipMemcpyDeviceToHost, c->stream);
-    return e == hipSuccess ? hipStreamSynchronize(c->stream) : e;
+// The tallies to the stage; waits for the stream.
+static hipError_t readTallies(StageLease& stage, const unsigned long long* ctr) {
+    stage.inFlight(true);
+    hipError_t e = hipMemcpyAsync(stage->tallies, ctr, sizeof(unsigned long long) * kCounterWords, hipMemcpyDeviceToHost,
+                                  stage.stream());
+    if (e == hipSuccess) e = hipStreamSynchronize(stage.stream());
+    if (e == hipSuccess) stage.inFlight(false);
+    return e;
 }
 
 static LaunchCfg cfgOf(el_ctx* c) {
@@ -274,7 +173,18 @@ static LaunchCfg cfgOf(el_ctx* c) {
     return l;
 }
 
-static int createContext(el_ctx** out, int device, std::shared_ptr<Stage> stage) {
+extern "C" {
+
+int el_device_count(int* out) {
+    if (!out) return EL_ERR_ARG;
+    int n = 0;
+    hipError_t e = hipGetDeviceCount(&n);
+    if (e != hipSuccess) n = 0;
+    *out = n;
+    return EL_OK;
+}
+
+int el_create(el_ctx** out, int device) {
     if (!out) return EL_ERR_ARG;
     *out = nullptr;
     std::unique_ptr<el_ctx> c(new el_ctx());
@@ -291,24 +201,9 @@ static int createContext(el_ctx** out, int device, std::shared_ptr<Stage> stage)
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (c->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
     if (scratchAddress(device, &c->scratch) != hipSuccess) return EL_ERR_HIP;
-    if (stage->ensureTallies() != hipSuccess) return EL_ERR_HIP;
-    c->stage = std::move(stage);
     *out = c.release();
     return EL_OK;
 }
-
-extern "C" {
-
-int el_device_count(int* out) {
-    if (!out) return EL_ERR_ARG;
-    int n = 0;
-    hipError_t e = hipGetDeviceCount(&n);
-    if (e != hipSuccess) n = 0;
-    *out = n;
-    return EL_OK;
-}
-
-int el_create(el_ctx** out, int device) { return createContext(out, device, std::make_shared<Stage>()); }
 
 void el_destroy(el_ctx* c) {
     if (!c) return;
@@ -797,6 +692,8 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     if (depth > 64) return fail(c, EL_ERR_RANGE, "max_depth above 64");
     EL_HIP(c, hipSetDevice(c->device));
     if (p->spp == 0) return EL_OK;
+    StageLease stage(c->device, c->stream);
+    EL_HIP(c, stage.take());
     if (p->bvh_width && (int)p->bvh_width != c->width) {
         int rc = uploadBvh(c, (int)p->bvh_width);
         if (rc) return rc;
@@ -867,7 +764,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     double extendMs = 0, shadeMs = 0, shadowMs = 0;
     uint64_t extendLaunches = 0;
     EL_HIP(c, hipEventRecord(e0, c->stream));
-    unsigned long long* const h = c->stage->tallies;   // the launches' tallies, read back with the last sync
+    const unsigned long long* const h = stage->tallies;   // the launches' tallies, read back with the last sync
 
     if (p->mode == EL_MODE_PLAIN) {
         for (uint32_t s = 0; s < p->spp; s++) {
@@ -905,7 +802,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
         }
         c->accPending = false;
         EL_HIP(c, hipEventRecord(e1, c->stream));
-        EL_HIP(c, readTallies(c, ctr));   // the tallies and every event
+        EL_HIP(c, readTallies(stage, ctr));   // the tallies and every event
         for (auto& t : timed) {
             float ms = 0;
             EL_HIP(c, hipEventElapsedTime(&ms, c->evPool[t.first], c->evPool[t.first + 1]));
@@ -914,7 +811,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     }
     if (p->mode == EL_MODE_PLAIN) {
         EL_HIP(c, hipEventRecord(e1, c->stream));
-        EL_HIP(c, readTallies(c, ctr));
+        EL_HIP(c, readTallies(stage, ctr));
     }
     float totalMs = 0;
     EL_HIP(c, hipEventElapsedTime(&totalMs, e0, e1));
@@ -989,6 +886,8 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     if (accumulate && (!c->adjSumValid || c->adjSumTex != gtex))
         return fail(c, EL_ERR_STATE, "EL_ADJ_ACCUMULATE without a previous el_adjoint with the same grad_texture");
     EL_HIP(c, hipSetDevice(c->device));
+    StageLease stage(c->device, c->stream);
+    EL_HIP(c, stage.take());
     const size_t npx = (size_t)c->cam.x_res * c->cam.y_res;
     const size_t M = c->mats.size();
     const size_t ntex = gtex >= 0 ? (size_t)c->texs[gtex].w * c->texs[gtex].h * 3 : 0;
@@ -1092,12 +991,12 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     EL_HIP(c, hipEventRecord(e1, c->stream));
     std::vector<double> hm(M * 6);
     EL_HIP(c, hipMemcpyAsync(hm.data(), c->aMat.p, M * 6 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    const unsigned long long* const h = c->stage->tallies;
+    const unsigned long long* const h = stage->tallies;
     if (ntex && dtex && devp)
         EL_HIP(c, hipMemcpyAsync(dtex, c->aTex.p, ntex * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
     if (ntex && dtex && !devp)
         EL_HIP(c, stageOut(
-                      *c->stage, c->stream, ntex, sizeof(float),
+                      stage, ntex, sizeof(float),
                       [&](size_t first, size_t n, unsigned char* chunk) {
                           return hipMemcpyAsync(chunk, c->aTex.as<float>() + first, n * sizeof(float),
                                                 hipMemcpyDeviceToHost, c->stream);
@@ -1105,7 +1004,7 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
                       [&](size_t first, size_t, const unsigned char* chunk, size_t i0, size_t i1) {
                           std::memcpy(dtex + first + i0, (const float*)chunk + i0, (i1 - i0) * sizeof(float));
                       }));
-    EL_HIP(c, readTallies(c, ctr));
+    EL_HIP(c, readTallies(stage, ctr));
     float ms = 0;
     EL_HIP(c, hipEventElapsedTime(&ms, e0, e1));
     std::vector<float> fm(M * 6);
@@ -1133,10 +1032,12 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
 static hipError_t readMean(el_ctx* c, const float4* sums, uint32_t stride, size_t npx, float* rgba,
                            uint32_t* samples) {
     if (hipError_t e = clearPending(c); e != hipSuccess) return e;
+    StageLease stage(c->device, c->stream);
+    if (hipError_t e = stage.take(); e != hipSuccess) return e;
     const size_t nR = rgba ? sizeof(float4) : 0, nS = samples ? sizeof(uint32_t) : 0;
     // a chunk of n pixels: n float4, then n counts
     return stageOut(
-        *c->stage, c->stream, npx, nR + nS,
+        stage, npx, nR + nS,
         [&](size_t first, size_t n, unsigned char* chunk) {
             return launchResolve(c->stream, sums, stride, c->dCounts.as<uint32_t>(), (uint32_t)first, (uint32_t)n,
                                  nR ? (float4*)chunk : nullptr, nS ? (uint32_t*)(chunk + n * nR) : nullptr);
@@ -1232,7 +1133,9 @@ static int traceCommon(el_ctx* c, const el_ray* rays, const float* tmax, uint32_
     float* dT = t;
     float* dUV = uv;
     uint8_t* dOcc = occ;
-    Stage& st = *c->stage;
+    StageLease stage(c->device, c->stream);
+    EL_HIP(c, stage.take());
+    Stage& st = *stage;
     // A short host query (a pick) goes through the stage: the kernel reads the
     // rays from it and writes the answers to it, without a copy each way.
     const bool direct = !devp && !count && n <= kDirectRays;
@@ -1272,6 +1175,7 @@ static int traceCommon(el_ctx* c, const el_ray* rays, const float* tmax, uint32_
     }
     unsigned long long* ctr = c->dCounters.as<unsigned long long>();
     EL_HIP(c, hipMemsetAsync(ctr, 0, sizeof(unsigned long long) * kCounterWords, c->stream));
+    stage.inFlight(direct);
     EL_HIP(c, launchTrace(cfgOf(c), c->ds, dR, dTm, n, dTri, dT, dUV, dOcc, any, count, ctr));
     if (!devp && !direct && !count) {
         // a chunk of n rays: each answer's n values after the other's
@@ -1283,7 +1187,7 @@ static int traceCommon(el_ctx* c, const el_ray* rays, const float* tmax, uint32_
         size_t bytes = 0;
         for (auto& o : host) bytes += o.second;
         EL_HIP(c, stageOut(
-                      st, c->stream, n, bytes,
+                      stage, n, bytes,
                       [&](size_t first, size_t m, unsigned char* chunk) {
                           hipError_t e = hipSuccess;
                           for (size_t k = 0; k < host.size() && e == hipSuccess; k++) {
@@ -1301,7 +1205,7 @@ static int traceCommon(el_ctx* c, const el_ray* rays, const float* tmax, uint32_
                           }
                       }));
     }
-    EL_HIP(c, readTallies(c, ctr));
+    EL_HIP(c, readTallies(stage, ctr));
     const unsigned long long* const h = st.tallies;
     if (direct && any) std::memcpy(occ, dOcc, n);
     if (direct && !any) {
@@ -1436,7 +1340,6 @@ struct el_batch {
     std::string graphKey;
     el_stats stats{};
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    std::shared_ptr<Stage> stage = std::make_shared<Stage>();
 };
 
 static int bfail(el_batch* b, int code, const std::string& what) {
@@ -1472,7 +1375,6 @@ int el_batch_create(el_batch** out, int device) {
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (hipEventCreate(&b->e0) != hipSuccess || hipEventCreate(&b->e1) != hipSuccess) return EL_ERR_HIP;
     if (b->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
-    if (b->stage->ensureTallies() != hipSuccess) return EL_ERR_HIP;
     *out = b.release();
     return EL_OK;
 }
@@ -1497,7 +1399,7 @@ int el_batch_add(el_batch* b, const el_scene_view* view, uint32_t spp, uint64_t 
     if (spp == 0) return bfail(b, EL_ERR_ARG, "spp must be positive");
     if (b->scenes.size() >= 65536) return bfail(b, EL_ERR_RANGE, "at most 65536 scenes per batch");
     el_ctx* c = nullptr;
-    int rc = createContext(&c, b->device, b->stage);
+    int rc = el_create(&c, b->device);
     if (rc) return bfail(b, rc, "context creation failed");
     rc = el_upload_scene(c, view);
     if (rc) {
@@ -1552,6 +1454,8 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         return bfail(b, EL_ERR_ARG, "block must be a multiple of 64, at most 256");
     if (p->refill > 64) return bfail(b, EL_ERR_ARG, "refill must be 0..64");
     EL_BHIP(b, hipSetDevice(b->device));
+    StageLease stage(b->device, b->stream);
+    EL_BHIP(b, stage.take());
     const int width = p->bvh_width ? (int)p->bvh_width : b->width;
     if (width != b->width) {
         for (auto* c : b->scenes) {
@@ -1750,10 +1654,8 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
         EL_BHIP(b, launchAll());
         EL_BHIP(b, hipEventRecord(b->e1, b->stream));
     }
-    const unsigned long long* const h = b->stage->tallies;
-    EL_BHIP(b, hipMemcpyAsync(b->stage->tallies, ctr, sizeof(unsigned long long) * kCounterWords,
-                              hipMemcpyDeviceToHost, b->stream));
-    EL_BHIP(b, hipStreamSynchronize(b->stream));
+    const unsigned long long* const h = stage->tallies;
+    EL_BHIP(b, readTallies(stage, ctr));
     float t = 0;
     EL_BHIP(b, hipEventElapsedTime(&t, b->e0, b->e1));
     *ms = t;
