@@ -1,16 +1,19 @@
 // The pool of pinned stages and the copy through them, over a stand-in for the runtime: who gets which memory, what is
-// pinned and given back, what an error leaves, and what the host threads do meanwhile.  Modes: pool, copy.
+// pinned and given back, what an error leaves, and what the host threads do meanwhile.  Modes: pool, copy, wait.
 #include "stage.hpp"
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <ctime>
 #include <string>
 
 using namespace eleven;
 
 static std::atomic<int> pins{0}, frees{0}, syncs{0};
 static std::atomic<int> failSync{-1};   // which event wait fails
+static std::atomic<int> busyMs{0};      // how long the GPU works before the next event
 extern "C" {
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     pins++;
@@ -28,7 +31,10 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
 }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return failSync-- == 0 ? hipErrorUnknown : hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) {
+    std::this_thread::sleep_for(std::chrono::milliseconds(busyMs.exchange(0)));
+    return failSync-- == 0 ? hipErrorUnknown : hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) {
     syncs++;
     return hipSuccess;
@@ -126,10 +132,33 @@ static void copy() {
     }
 }
 
+// Host threads' time while the GPU works for 400 ms before the first chunk is there.
+static void wait() {
+    StagePool pool;
+    for (int fails : {-1, 0}) {
+        StageLease a(0, nullptr, pool);
+        check(a.take() == hipSuccess, "a stage");
+        busyMs = 400;
+        failSync = fails;
+        std::vector<unsigned char> out(12 << 20);
+        const std::clock_t from = std::clock();
+        const hipError_t e = stageOut(
+            a, out.size(), 1, [](size_t, size_t, unsigned char*) { return hipSuccess; },
+            [&](size_t first, size_t, const unsigned char* chunk, size_t i0, size_t i1) {
+                std::memcpy(&out[first + i0], chunk + i0, i1 - i0);
+            });
+        const double ms = 1e3 * (double)(std::clock() - from) / CLOCKS_PER_SEC;
+        check(e == (fails ? hipSuccess : hipErrorUnknown), "the wait's result");
+        printf("processor time %.0f ms\n", ms);
+        check(ms < 200, "the helpers sleep while the GPU works");
+    }
+}
+
 int main(int, char** argv) {
     const std::string mode = argv[1];
     if (mode == "pool") pool();
     if (mode == "copy") copy();
+    if (mode == "wait") wait();
     printf("bad=%d\n", bad);
     return bad != 0;
 }

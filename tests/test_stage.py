@@ -79,3 +79,8 @@ def test_contexts_in_several_threads():
         for k, (a, b) in enumerate(zip(x, y)):
             # the material gradients (every sixth) are sums of atomics
             assert np.allclose(a, b, rtol=1e-5, atol=1e-6) if k % 6 == 5 else np.array_equal(a, b)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None or not HIP.exists(), reason="needs g++ and the HIP headers")
+def test_helpers_sleep_while_the_gpu_works(tmp_path):
+    test_stages_on_the_host(tmp_path, "wait")

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -156,6 +157,8 @@ private:
 // copy(first, n, chunk, i0, i1) copies the chunk's items [i0, i1) out, on up
 // to 8 host threads (a thread per MB: a frame's copy is bound by the page
 // faults of the caller's fresh arrays, which one thread takes one at a time).
+// They sleep until the first chunk is there, for which the GPU may have a whole
+// render to finish, and look for each other's progress from then on.
 template <class Fill, class Copy>
 hipError_t stageOut(StageLease& lease, size_t items, size_t itemBytes, Fill&& fill, Copy&& copy) {
     if (!items) return hipSuccess;
@@ -173,13 +176,18 @@ hipError_t stageOut(StageLease& lease, size_t items, size_t itemBytes, Fill&& fi
     };
     std::atomic<size_t> ready{0}, done{0};   // chunks filled; thread-chunks copied
     std::atomic<bool> failed{false};         // no further chunk gets ready
-    std::atomic<size_t> team{0};             // threads that share a chunk, once known
+    std::mutex mu;
+    std::condition_variable begun;
+    size_t team = 0;                         // threads that share a chunk: known, under mu, with the first one ready
     auto part = [&](size_t k, size_t t) {
-        const size_t n = count(k), T = team.load(std::memory_order_relaxed);
+        const size_t n = count(k), T = team;
         copy(k * per, n, chunk(k), n * t / T, n * (t + 1) / T);
     };
     auto work = [&](size_t t) {
-        while (!team.load(std::memory_order_acquire)) std::this_thread::yield();
+        {
+            std::unique_lock<std::mutex> lock(mu);
+            begun.wait(lock, [&] { return team != 0; });
+        }
         for (size_t k = 0; k < chunks; k++) {
             while (ready.load(std::memory_order_acquire) <= k) {
                 if (failed.load(std::memory_order_acquire)) return;
@@ -200,18 +208,28 @@ hipError_t stageOut(StageLease& lease, size_t items, size_t itemBytes, Fill&& fi
         }
     }
     const size_t T = threads.size() + 1;
-    team.store(T, std::memory_order_release);
+    auto begin = [&] {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            team = T;
+        }
+        begun.notify_all();
+    };
     for (size_t k = 0; k < chunks && e == hipSuccess; k++) {
         e = hipEventSynchronize(st.filled[k & 1]);
         if (e != hipSuccess) break;
         ready.store(k + 1, std::memory_order_release);
+        if (k == 0) begin();
         part(k, 0);
         if (k + 2 < chunks) {   // the chunk is filled again once every thread has copied its share
             while (done.load(std::memory_order_acquire) < (k + 1) * (T - 1)) std::this_thread::yield();
             e = issue(k + 2);
         }
     }
-    if (e != hipSuccess) failed.store(true, std::memory_order_release);
+    if (e != hipSuccess) {
+        failed.store(true, std::memory_order_release);
+        begin();
+    }
     for (auto& t : threads) t.join();
     if (e == hipSuccess) lease.inFlight(false);   // every chunk was waited for
     return e;
