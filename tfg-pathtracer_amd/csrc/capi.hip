@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/eleven.h"
+#include "adjoint_plan.hpp"
 #include "bvh.hpp"
 #include "dev_buf.hpp"
 #include "hdri_table.hpp"
@@ -865,11 +866,6 @@ extern "C" int el_residual_l2(el_ctx* c, const float* target, double* loss) {
     return EL_OK;
 }
 
-// el_adjoint: device memory for a generation of paths (queues, path state and
-// records), so that its memory does not grow with the pixels and samples:
-// 4.4 M paths at depth 6, enough to fill the GPU.
-constexpr uint64_t kAdjointBytes = 2ull << 30;
-
 extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* dimage, float* dmat, float* dtex,
                           int devp) {
     const bool accumulate = (p && (p->flags & EL_ADJ_ACCUMULATE) != 0);
@@ -938,14 +934,16 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     if (npad >= (1ull << 31)) return fail(c, EL_ERR_RANGE, "frame too large for the adjoint");
     uint64_t Q = 0;
     WfState q{};
-    const uint64_t perPath = 6 * 32 + 60 + (recorded ? 0 : 16 * depth + 4);
-    uint64_t budget = kAdjointBytes;
-    if (c->wf.cap < std::min(total, budget / perPath)) {   // buffers will grow: by a quarter of what is free, as a render's
+    const AdjointMemory memory{WfBuffers::kEntryBytes, WfBuffers::kSlotBytes,
+                               lc.maxThreads + (uint64_t)kXcds * (kMaxBlock + 1), recorded ? 0 : 16ull * depth + 4,
+                               c->wf.cap, c->wf.qcap, c->aHits.n + c->aVis.n};
+    hipError_t asked = hipSuccess;
+    const uint64_t cap = adjointPaths(memory, total, [&]() -> uint64_t {
         size_t freeB = 0, totalB = 0;
-        EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
-        budget = std::min<uint64_t>(budget, std::max<uint64_t>(freeB / 4, c->wf.cap * perPath));
-    }
-    const uint64_t cap = std::max<uint64_t>(1u << 16, budget / perPath);
+        asked = hipMemGetInfo(&freeB, &totalB);
+        return freeB;
+    });
+    EL_HIP(c, asked);
     int rc = wfPlan(c, lc, total, npad, cap, false, q, Q);
     if (rc) return rc;
     if (recorded) {
@@ -972,7 +970,7 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
         a.genPixel = (uint32_t)(start % npad);
         a.genSample = (uint32_t)(start / npad);
         a.genCount = (uint32_t)std::min<uint64_t>(Q, total - start);
-            a.run = a.genPixel == 0 && a.genCount % npad == 0 ? (uint32_t)(a.genCount / npad) : 0u;
+        a.run = a.genPixel == 0 && a.genCount % npad == 0 ? (uint32_t)(a.genCount / npad) : 0u;
         if (!recorded) {
             std::vector<std::pair<size_t, int>> timed;
             size_t ev = 2;

@@ -8,6 +8,7 @@
 namespace eleven {
 
 struct WfBuffers {
+    static constexpr size_t kEntryBytes = 176, kSlotBytes = 64;   // of a queue entry and a path slot (aov apart)
     DevBuf ray0, ray1, hits, shadowH, shadowP;              // per queue entry
     DevBuf pathT, pathL, pix, sample, quiet, pend, aov;     // per path slot
     DevBuf counters;
