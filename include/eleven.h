@@ -52,18 +52,18 @@ extern "C" {
 #define EL_FLAG_COUNT_TRAVERSAL 2u /* wavefront: tally node fetches and
                                       triangle tests of the closest-hit stage */
 #define EL_FLAG_RECORD_PATHS 8u /* opt-in, O(pixels x spp x depth) memory:
-                                   keep each path's radiance (16 B per path,
-                                   when that fits half of the free device
-                                   memory); needs a cleared accumulation (the
-                                   record covers this one render and ends with
-                                   el_clear and el_set_camera; its buffers go
-                                   back at the next render that does not
-                                   record).  Wavefront renders with max_depth
-                                   <= 16 also keep every vertex's hit and
-                                   shadow answers (16 B per vertex + 4 B per
-                                   path, when that fits a quarter of the free
-                                   device memory): el_adjoint then traces no
-                                   ray.  The image is the same either way.   */
+                                   wavefront renders with max_depth <= 16 keep
+                                   every vertex's hit and shadow answers and
+                                   each path's radiance (16 B per vertex +
+                                   20 B per path, when the vertices fit a
+                                   quarter of the free device memory):
+                                   el_adjoint then traces no ray.  Other
+                                   renders keep nothing.  Needs a cleared
+                                   accumulation (the record covers this one
+                                   render and ends with el_clear and
+                                   el_set_camera; its buffers go back at the
+                                   next render that does not record).  The
+                                   image is the same either way.             */
 
 #define EL_FLAG_SERIAL_SHADOWS 16u /* wavefront: every closest-hit and shadow
                                      queue in a launch of its own, one after
@@ -189,8 +189,8 @@ typedef struct {
                                   the scene, the accumulation and the render's
                                   queues: a generation's hits and shadow
                                   answers, adjoint image, gradients          */
-    uint64_t record_bytes;     /* device memory held by the last recording
-                                  render (EL_FLAG_RECORD_PATHS), 0 if none   */
+    uint64_t record_bytes;     /* device memory held by the last render's record
+                                  (EL_FLAG_RECORD_PATHS), 0 if it kept none  */
 } el_stats;
 
 /* Adjoint of the accumulated image (no counterpart in the reference, which

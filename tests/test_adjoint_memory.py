@@ -5,6 +5,7 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 import eleven
 from eleven import scenegen
@@ -24,7 +25,6 @@ def test_generations_within_their_memory(tmp_path):
 @pytest.mark.gpu
 def test_an_adjoint_takes_two_gibibytes_at_most():
     """512 x 512 x 16 paths of depth 16, after a plain render: no queues are there yet."""
-    import torch
     print("[adjoint memory] depth 16", flush=True)
     ctx = eleven.Context(0)
     ctx.upload(scenegen.sphere_field_arrays(n_spheres=4, res=(512, 512), seed=1))

@@ -116,11 +116,10 @@ struct el_ctx {
     bool accPending = false;       // the accumulation is empty, but its buffers are not cleared
     bool accMixed = false;         // renders since el_clear used different seeds or depths
     DevBuf dRec;                   // per (sample, pixel) path radiance of a recorded render
-    DevBuf dRecHits, dRecVis, wVis;  // its vertices (wavefront recordings: RenderArgs::recHits / recVis)
-    bool recHits = false;          // with recValid: dRecHits / dRecVis hold the recorded render's vertices
+    DevBuf dRecHits, dRecVis, wVis;  // its vertices (RenderArgs::recHits / recVis)
     bool adjSumValid = false;      // aMat / aTex hold the sums of the el_adjoint calls so far
     int32_t adjSumTex = -1;        // their grad_texture
-    bool recValid = false;         // dRec covers the whole accumulation
+    bool recValid = false;         // the record covers the whole accumulation
     uint64_t totalRays = 0, totalVerts = 0, totalPaths = 0;
     DevBuf aImage, aMat, aTex;     // adjoint image, FP64 material and FP32 texel gradients
     DevBuf aHits, aVis, aQueue;    // el_adjoint: a generation's hits and shadow answers, the replay's queue counts
@@ -355,7 +354,6 @@ static int clearAccum(el_ctx* c) {
     c->sampleBase = 0;
     c->accMixed = false;
     c->recValid = false;
-    c->recHits = false;
     c->totalRays = c->totalVerts = c->totalPaths = 0;
     return EL_OK;
 }
@@ -724,39 +722,35 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     a.sample = c->sampleBase;
     a.cull = (p->flags & EL_FLAG_NO_CULL) ? 0u : 1u;
     bool record = (p->flags & EL_FLAG_RECORD_PATHS) != 0;
-    bool recordHits = false;
-    if (!record && c->dRec.p) releaseRecord(c);
+    if (record && c->sampleBase != 0) return fail(c, EL_ERR_STATE, "EL_FLAG_RECORD_PATHS needs a cleared accumulation");
+    // Wavefront renders record every vertex's hit and shadow answers (16 B per
+    // vertex + 4 B per path) and the paths' radiance (16 B), from which el_adjoint
+    // replays without tracing, when the radiance fits half of the free device
+    // memory and the vertices a quarter of the rest.  Without the vertices the
+    // adjoint walks the paths again, and has no use for their radiance.
+    record = record && p->mode != EL_MODE_PLAIN && depth <= (uint32_t)dev::kAdjMaxDepthHost;
     if (record) {
-        if (c->sampleBase != 0) return fail(c, EL_ERR_STATE, "EL_FLAG_RECORD_PATHS needs a cleared accumulation");
-        // the radiance record (16 B per path) is kept only when it fits half
-        // of the free device memory; otherwise el_adjoint replays without it.
-        // Wavefront renders also keep every vertex's hit and shadow answers
-        // (16 B per vertex + 4 B per path) when they fit a quarter of the
-        // free memory, so that el_adjoint replays without tracing.
         const size_t recBytes = (size_t)p->spp * npx * sizeof(float4), hitBytes = recBytes * depth;
-        const bool wantHits = p->mode != EL_MODE_PLAIN && depth <= (uint32_t)dev::kAdjMaxDepthHost;
         auto holds = [](const DevBuf& b, size_t n) { return b.p && n <= b.n && n >= b.n / 4; };
         // buffers of another size go back first: the rules are about the memory without them
-        if (!holds(c->dRec, recBytes) || (wantHits && !holds(c->dRecHits, hitBytes))) {
+        if (!holds(c->dRec, recBytes) || !holds(c->dRecHits, hitBytes)) {
             releaseRecord(c);
             size_t freeB = 0, totalB = 0;
             EL_HIP(c, hipMemGetInfo(&freeB, &totalB));
-            record = recBytes <= freeB / 2;
-            recordHits = record && wantHits && hitBytes <= (freeB - recBytes) / 4;
-        } else {
-            recordHits = wantHits;
+            record = recBytes <= freeB / 2 && hitBytes <= (freeB - recBytes) / 4;
         }
-        if (record) {
-            EL_HIP(c, c->dRec.ensure(recBytes));
-            a.rec = c->dRec.as<float4>();
-        }
-        if (recordHits) {
-            EL_HIP(c, c->dRecHits.ensure(hitBytes));
-            EL_HIP(c, c->dRecVis.ensure((size_t)p->spp * npx * sizeof(uint32_t)));
-            a.recHits = c->dRecHits.as<float4>();
-            a.recVis = c->dRecVis.as<uint32_t>();
-            a.recStride = (uint64_t)p->spp * npx;
-        }
+    }
+    if (record) {
+        const size_t paths = (size_t)p->spp * npx;
+        EL_HIP(c, c->dRec.ensure(paths * sizeof(float4)));
+        EL_HIP(c, c->dRecHits.ensure(paths * depth * sizeof(float4)));
+        EL_HIP(c, c->dRecVis.ensure(paths * sizeof(uint32_t)));
+        a.rec = c->dRec.as<float4>();
+        a.recHits = c->dRecHits.as<float4>();
+        a.recVis = c->dRecVis.as<uint32_t>();
+        a.recStride = paths;
+    } else if (c->dRec.p) {
+        releaseRecord(c);
     }
     c->recValid = false;
 
@@ -781,7 +775,7 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
         WfState q{};
         int rc = wfPlan(c, lc, total, npad, p->queue_cap, aov, q, Q);
         if (rc) return rc;
-        if (recordHits) {
+        if (record) {
             EL_HIP(c, c->wVis.ensure(Q * sizeof(uint32_t)));
             q.pathVis = c->wVis.as<uint32_t>();
         }
@@ -825,7 +819,6 @@ extern "C" int el_render(el_ctx* c, const el_render_params* p) {
     }
     c->sampleBase += p->spp;
     c->recValid = record;
-    c->recHits = recordHits;
     c->stats.record_bytes = record ? c->dRec.n + c->dRecHits.n + c->dRecVis.n + c->wVis.n : 0;
     c->totalRays += tally(h, kStatRays);
     c->totalVerts += tally(h, kStatVerts);
@@ -928,7 +921,7 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
     // wavefront EL_FLAG_RECORD_PATHS render) are traced no more: the
     // recording stopped no earlier than the replay does.  Others are walked
     // again here, recording the generation's hits and shadow answers.
-    const bool recorded = c->recValid && c->recHits;
+    const bool recorded = c->recValid;
     const uint64_t npad = (uint64_t)((c->cam.x_res + 7) / 8) * ((c->cam.y_res + 7) / 8) * 64;
     const uint64_t total = (uint64_t)c->sampleBase * npad;
     if (npad >= (1ull << 31)) return fail(c, EL_ERR_RANGE, "frame too large for the adjoint");

@@ -492,7 +492,6 @@ EL_KERNEL(EL_WPE_PLAIN) void k_plain(DevScene s, RenderArgs a, float4* __restric
                 surfaceTangents(s, sh, at, ab);
             }
         });
-        if (a.rec) a.rec[(uint64_t)a.sample * W_ * H_ + idx] = make_float4(L.x, L.y, L.z, 1.f);
         L = clamp3(L);
         if (!anyNan(L)) {
             float4 acc = accum[idx];

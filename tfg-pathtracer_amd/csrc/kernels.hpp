@@ -62,7 +62,7 @@ struct RenderArgs {
     uint32_t fresh;         // wavefront: the accumulation holds nothing yet and is not cleared: finalize
                             // starts a pixel's sums from zero at sample 0 (every pixel has that sample once)
     uint32_t zeroTallies;   // wavefront: the camera launch zeroes the tallies
-    float4* rec;            // per (sample, pixel): the path's radiance before the clamp, or null
+    float4* rec;            // wavefront: per (sample, pixel) the path's radiance before the clamp, or null
     // Wavefront renders that record, and adjoints that replay, path vertices
     // (one scene; all null otherwise): the closest hit (tri, t, u, v; tri -1:
     // escaped) of vertex b of a path at recHits[b * recStride + key], and per

@@ -16,9 +16,9 @@ numbers: finite differences of the loss are differences of the same paths.
 Memory: by default nothing of a path is kept between the forward and the
 backward; the adjoint recomputes the paths from their RNG counters (path
 replay), a bounded number of them at a time, so the device memory of a
-gradient is O(pixels) plus at most 2 GiB.  record=True keeps each path's
-radiance and, in wavefront mode, every vertex (16 B per path + 16 B per
-vertex: O(pixels x spp x depth)), which lets the adjoint replay the paths
+gradient is O(pixels) plus at most 2 GiB.  record=True keeps, in wavefront
+mode, every vertex and each path's radiance (16 B per vertex + 20 B per
+path: O(pixels x spp x depth)), which lets the adjoint replay the paths
 without tracing.
 """
 from __future__ import annotations
@@ -88,8 +88,8 @@ class Renderer:
         if texture is not None:
             self.ctx.set_texture(self.grad_texture, np.ascontiguousarray(texture, np.float32))
         self.ctx.clear()
-        # record: the paths' radiance (wavefront: also every vertex) let the
-        # backward replay each path once, without tracing in wavefront mode
+        # record: the paths' vertices (wavefront mode) let the backward replay
+        # them without tracing
         self.ctx.render(self.spp, depth=self.depth, seed=self.seed, mode=self.mode,
                         flags=FLAG_RECORD_PATHS if self.record else 0)
         return self.ctx.read()[0][..., :3].copy() if read else None

@@ -21,7 +21,7 @@ ranges after every Adam update.
 Memory: by default the adjoint replays each path from its RNG counters
 (O(pixels) device memory per view and at most 2 GiB for the paths in
 flight); record=True keeps the replayed render's
-paths instead (EL_FLAG_RECORD_PATHS: O(pixels x spp x depth)).
+paths instead (EL_FLAG_RECORD_PATHS, wavefront mode: O(pixels x spp x depth)).
 """
 from __future__ import annotations
 
@@ -98,8 +98,8 @@ class MultiView:
 
     def render_view(self, v: int, seed: int, spp: int | None = None, record: bool = False, read: bool = True):
         """Mean image of view v (None with read=False); with `record`, the
-        render keeps its paths for a following el_adjoint (which then walks
-        each path once, from the recorded vertices in wavefront mode)."""
+        render keeps its paths (wavefront mode) for a following el_adjoint,
+        which then replays them without tracing."""
         self.ctx.set_camera(self.cameras[v])
         self.ctx.render(spp or self.spp, depth=self.depth, seed=seed, mode=self.mode,
                         flags=FLAG_RECORD_PATHS if record else 0)
