@@ -168,7 +168,7 @@ static LaunchCfg cfgOf(el_ctx* c) {
     l.block = c->block;
     l.shadeBlock = 256;
     l.refill = c->refill;
-    l.maxThreads = c->maxThreads;
+    l.maxThreads = l.quadThreads = c->maxThreads;
     l.gstack = c->dGstack.as<int>();
     return l;
 }
@@ -1232,7 +1232,7 @@ int el_trace_closest_noalloc(el_ctx* c, const el_ray* d_rays, uint32_t n, int32_
     if (!c->scratch) return fail(c, EL_ERR_STATE, "no device scratch");
     if (n == 0) return EL_OK;
     EL_HIP(c, hipSetDevice(c->device));
-    // as many resident threads as the spill area holds at the scene's depth
+    // as many resident threads as the spill area holds at the scene's depth (by quads, which spill nothing, all)
     LaunchCfg lc = cfgOf(c);
     const uint64_t fit = kScratchSpillInts / (uint64_t)c->gcap;
     uint32_t threads = (uint32_t)std::min<uint64_t>(c->maxThreads, fit);
@@ -1530,7 +1530,7 @@ static int batchRender(el_batch* b, const el_batch_params* p, uint32_t sppCap, d
     lc.stream = b->stream;
     lc.block = p->block ? p->block : kDefaultBlock;
     lc.shadeBlock = 256;
-    lc.maxThreads = b->maxThreads;
+    lc.maxThreads = lc.quadThreads = b->maxThreads;
     lc.refill = p->refill ? p->refill : kDefaultRefill;
     lc.gstack = b->dGstack.as<int>();
     const uint64_t segSize = (Q + kXcds - 1) / kXcds + lc.maxThreads / kXcds + kMaxBlock;

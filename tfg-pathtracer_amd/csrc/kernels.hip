@@ -90,7 +90,6 @@ __device__ __forceinline__ void blockFlush(unsigned long long* counters, const i
 // lane's visit got shorter, 2^20 random rays take 150 us by lanes and 176 by
 // quads, but occlusion on the terrain 211 and 198, and the 256 x 256 frame the
 // same either way: the line stays.)
-constexpr uint32_t kQuadRays = 1u << 20;
 template <int W>
 __device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n) {
     return W == 4 && s.quads && n <= kQuadRays;
@@ -1541,7 +1540,9 @@ static uint32_t queueGrid(const LaunchCfg& c, int width, uint64_t n) {
 hipError_t launchTrace(const LaunchCfg& c, const DevScene& s, const float* rays, const float* tmax, uint32_t n,
                        int32_t* tri, float* t, float* uv, uint8_t* occ, bool any, bool count,
                        unsigned long long* counters) {
-    uint32_t grid = queueGrid(c, s.width, n);
+    // by quads (useQuads): a spill area smaller than the GPU's threads need not hold them back
+    const bool quads = s.width == 4 && s.quads && n <= kQuadRays;
+    uint32_t grid = quads ? gridFor((uint64_t)n * 4, c.block, c.quadThreads / c.block) : queueGrid(c, s.width, n);
     size_t lds = sizeof(int) * kShortStack * c.block;
 #define EL_TRACE(WW, A, C)                                                                                   \
     hipLaunchKernelGGL((k_trace<WW, A, C>), dim3(grid), dim3(c.block), lds, c.stream, s, rays, tmax, n, tri, t, \

@@ -102,6 +102,9 @@ struct WfState {
     uint32_t gthreads;
 };
 
+// Rays up to which a BVH4 launch may give each to a quad of lanes (useQuads, kernels.hip).
+constexpr uint32_t kQuadRays = 1u << 20;
+
 // Materials whose gradient sums k_adj_bounce keeps in LDS (24 KB of FP64: two blocks of it still fit a CU).
 constexpr uint32_t kAdjLdsMats = 512;
 
@@ -132,6 +135,7 @@ struct LaunchCfg {
     uint32_t block;         // traversal kernels (trace, extend, shadow) and the plain megakernel
     uint32_t shadeBlock;    // camera, shade, finalize
     uint32_t maxThreads;    // grid * block upper bound (size of the spill area)
+    uint32_t quadThreads;   // the same for a trace by quads, which spills nothing
     uint32_t refill;        // persistent traversal: idle lanes that trigger a refill
     int* gstack;
 };
