@@ -82,17 +82,20 @@ __device__ __forceinline__ void blockFlush(unsigned long long* counters, const i
 // shorter by quads (a visit is ~60 VALU instructions after one 16-byte load
 // instead of ~115 after four; 16 rays share a wave's leaf rounds instead of
 // 64), while one that does is bound by instruction issue, where a lane per
-// ray needs fewer in all.  Whole calls, lanes against quads: 16,384 rays of
-// the 64-sphere field 92 -> 57 us, 262,144 119 -> 86, 2^20 178 -> 198
-// (occlusion on a 262,144-triangle terrain 249 -> 209), 2^21 294 -> 357; the
-// 256 x 256 frame of 16 samples, whose first launch holds 2^20 rays, 1479 ->
-// 1351 us, a 1920 x 1080 one of one sample (2^21) 2.6 -> 3.1 ms.  (Since a
-// lane's visit got shorter, 2^20 random rays take 150 us by lanes and 176 by
-// quads, but occlusion on the terrain 211 and 198, and the 256 x 256 frame the
-// same either way: the line stays.)
+// ray needs fewer in all.
+//
+// Queries: over seven scenes (sphere fields of 962 to 245,762 triangles,
+// terrains of 4,096 to 1,048,576), whole calls by lanes take 1.03 to 1.39 times
+// what they take by quads at 131,072 and 200,000 rays, 0.93 to 1.20 at 393,217
+// (half of the closest hits and half of the occlusion queries on either side), 0.77
+// to 1.05 at 2^19 and 0.67 to 0.92 at 2^20.
+// Renders: the 256 x 256 frame of 16 samples over 64 spheres, whose first
+// launch holds 2^20 rays and the others what is left of them, takes 1479 us with
+// quads up to 2^19 and 1351 up to 2^20; a 1920 x 1080 one of one sample (2^21) 2.6
+// ms by lanes and 3.1 by quads.
 template <int W>
-__device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n) {
-    return W == 4 && s.quads && n <= kQuadRays;
+__device__ __forceinline__ bool useQuads(const DevScene& s, uint32_t n, uint32_t most = kQuadRays) {
+    return W == 4 && s.quads && n <= most;
 }
 
 // Waves of the grid and the calling one's index.
@@ -261,7 +264,7 @@ EL_KERNEL(EL_WPE_TRAV) void k_trace(DevScene s, const float* __restrict__ rays, 
                                     uint32_t gthreads, uint32_t refill, unsigned long long* counters) {
     TraceCounters cnt{0, 0};
     uint32_t traced = 0;
-    const bool quads = useQuads<W>(s, n);
+    const bool quads = useQuads<W>(s, n, kQuadQueryRays);
     const WorkSource ws = splitWork(n, quads, gridWave(), gridWaves());
     auto load = [&](uint32_t i, float& ox, float& oy, float& oz, float& dx, float& dy, float& dz, float& tm,
                     BvhPtr&, uint32_t& item) {
@@ -1541,7 +1544,7 @@ hipError_t launchTrace(const LaunchCfg& c, const DevScene& s, const float* rays,
                        int32_t* tri, float* t, float* uv, uint8_t* occ, bool any, bool count,
                        unsigned long long* counters) {
     // by quads (useQuads): a spill area smaller than the GPU's threads need not hold them back
-    const bool quads = s.width == 4 && s.quads && n <= kQuadRays;
+    const bool quads = s.width == 4 && s.quads && n <= kQuadQueryRays;
     uint32_t grid = quads ? gridFor((uint64_t)n * 4, c.block, c.quadThreads / c.block) : queueGrid(c, s.width, n);
     size_t lds = sizeof(int) * kShortStack * c.block;
 #define EL_TRACE(WW, A, C)                                                                                   \

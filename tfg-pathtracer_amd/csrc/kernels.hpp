@@ -102,8 +102,10 @@ struct WfState {
     uint32_t gthreads;
 };
 
-// Rays up to which a BVH4 launch may give each to a quad of lanes (useQuads, kernels.hip).
+// Rays up to which a BVH4 launch gives each to a quad of lanes (useQuads,
+// kernels.hip): the launches of a render, and those of the ray queries.
 constexpr uint32_t kQuadRays = 1u << 20;
+constexpr uint32_t kQuadQueryRays = 3u << 17;
 
 // Materials whose gradient sums k_adj_bounce keeps in LDS (24 KB of FP64: two blocks of it still fit a CU).
 constexpr uint32_t kAdjLdsMats = 512;
