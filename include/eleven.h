@@ -61,9 +61,10 @@ extern "C" {
                                    renders keep nothing.  Needs a cleared
                                    accumulation (the record covers this one
                                    render and ends with el_clear and
-                                   el_set_camera; its buffers go back at the
-                                   next render that does not record).  The
-                                   image is the same either way.             */
+                                   el_set_camera; its buffers go back then if
+                                   they take more than 2 GiB, else at the next
+                                   render that does not record).  The image
+                                   is the same either way.                   */
 
 #define EL_FLAG_SERIAL_SHADOWS 16u /* wavefront: every closest-hit and shadow
                                      queue in a launch of its own, one after

@@ -337,7 +337,10 @@ static int uploadBvh(el_ctx* c, int width) {
 
 // Gives back the buffers of a recording render (EL_FLAG_RECORD_PATHS), which
 // cover only the accumulation they were recorded into: at the next render that
-// does not record (recording steps in a row keep them) and with the scene.
+// does not record, with the scene, and with the accumulation if they
+// are larger than kKeptRecord (recording steps in a row keep smaller ones, whose
+// allocation takes as long as the step's rays).
+constexpr size_t kKeptRecord = size_t(2) << 30;
 static void releaseRecord(el_ctx* c) {
     c->dRec.release();
     c->dRecHits.release();
@@ -354,6 +357,7 @@ static int clearAccum(el_ctx* c) {
     c->sampleBase = 0;
     c->accMixed = false;
     c->recValid = false;
+    if (c->dRec.n + c->dRecHits.n + c->dRecVis.n + c->wVis.n > kKeptRecord) releaseRecord(c);
     c->totalRays = c->totalVerts = c->totalPaths = 0;
     return EL_OK;
 }
