@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <memory>
 #include <mutex>
@@ -157,8 +158,10 @@ private:
 // copy(first, n, chunk, i0, i1) copies the chunk's items [i0, i1) out, on up
 // to 8 host threads (a thread per MB: a frame's copy is bound by the page
 // faults of the caller's fresh arrays, which one thread takes one at a time).
-// They sleep until the first chunk is there, for which the GPU may have a whole
-// render to finish, and look for each other's progress from then on.
+// They look for the first chunk for kSpin, which a read-back of a finished image
+// takes, then sleep until it is there: the GPU may have a whole adjoint to
+// finish first.  (Asleep at once, a wake-up of ~40 us each came on top of a
+// read-back of 1 MB and more: twelve images 1.79 -> 1.89 ms.)
 template <class Fill, class Copy>
 hipError_t stageOut(StageLease& lease, size_t items, size_t itemBytes, Fill&& fill, Copy&& copy) {
     if (!items) return hipSuccess;
@@ -178,15 +181,19 @@ hipError_t stageOut(StageLease& lease, size_t items, size_t itemBytes, Fill&& fi
     std::atomic<bool> failed{false};         // no further chunk gets ready
     std::mutex mu;
     std::condition_variable begun;
-    size_t team = 0;                         // threads that share a chunk: known, under mu, with the first one ready
+    std::atomic<size_t> team{0};             // threads that share a chunk: known with the first one ready
+    constexpr auto kSpin = std::chrono::microseconds(200);
     auto part = [&](size_t k, size_t t) {
-        const size_t n = count(k), T = team;
+        const size_t n = count(k), T = team.load(std::memory_order_relaxed);
         copy(k * per, n, chunk(k), n * t / T, n * (t + 1) / T);
     };
     auto work = [&](size_t t) {
-        {
+        auto known = [&] { return team.load(std::memory_order_acquire) != 0; };
+        for (const auto from = std::chrono::steady_clock::now(); !known();) {
+            std::this_thread::yield();
+            if (std::chrono::steady_clock::now() - from < kSpin) continue;
             std::unique_lock<std::mutex> lock(mu);
-            begun.wait(lock, [&] { return team != 0; });
+            begun.wait(lock, known);
         }
         for (size_t k = 0; k < chunks; k++) {
             while (ready.load(std::memory_order_acquire) <= k) {
@@ -211,7 +218,7 @@ hipError_t stageOut(StageLease& lease, size_t items, size_t itemBytes, Fill&& fi
     auto begin = [&] {
         {
             std::lock_guard<std::mutex> lock(mu);
-            team = T;
+            team.store(T, std::memory_order_release);
         }
         begun.notify_all();
     };
