@@ -1165,7 +1165,10 @@ struct WorkCursor {
     WorkTurns turns;
     uint32_t tried = 0;      // narrow source: shares found drawn out
     __device__ __forceinline__ WorkCursor(const WorkSource& ws) : turns(ws.first) {}
-    // The next chunk after [cursor, end) is used up; false: no items left.
+    // The next chunk after [cursor, end) is used up; false: no items left,
+    // and none will come.  One-scene launches do not ask again then; batches
+    // do, with a load a time, since the test costs their kernels more in
+    // registers (a batch of 12 scenes 8.67 and 8.75 ms of GPU).
     // The whole wave must call.
     template <bool WIDE>
     __device__ __forceinline__ bool draw(const WorkSource& ws) {
@@ -1234,7 +1237,7 @@ __device__ __forceinline__ void traceWaveRange(const DevScene& s, TravStack& st,
         const unsigned long long idle = waveMask(!live);
         const uint32_t nIdle = (uint32_t)__popcll(idle);
         const bool want = nIdle >= refill || nIdle == 64;
-        if (more && want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
+        if ((PER_RAY_BVH || more) && want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
         if (want && more) {
             if (!live) {
                 uint32_t i = wc.cursor + lanesBelow(idle);
@@ -1489,7 +1492,7 @@ __device__ __forceinline__ void traceQuadRange(const DevScene& s, QuadStack& st,
         const unsigned long long idle = waveMask(!live);
         const uint32_t nIdle = (uint32_t)__popcll(idle);
         const bool want = nIdle >= refill || nIdle == 64;
-        if (more && want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
+        if ((PER_RAY_BVH || more) && want && wc.cursor >= wc.end) more = wc.draw<PER_RAY_BVH>(ws);
         if (want && more) {
             if (!live) {
                 const uint32_t i = wc.cursor + (lanesBelow(idle) >> 2);   // quads are idle as a whole
