@@ -1,5 +1,5 @@
 // The pool of pinned stages and the copy through them, over a stand-in for the runtime: who gets which memory, what is
-// pinned and given back, what an error leaves, and what the host threads do meanwhile.  Modes: pool, copy, wait.
+// pinned and given back, what an error leaves, and what the host threads do meanwhile.  Modes: pool, copy, wait, contexts.
 #include "stage.hpp"
 
 #include <chrono>
@@ -132,6 +132,23 @@ static void copy() {
     }
 }
 
+// A thread for each of eight contexts: their calls at the same time pin once each, and what the contexts leave is freed.
+static void contexts() {
+    StagePool pool;
+    for (int k = 0; k < 8; k++) pool.contexts(1, 1);
+    for (int round = 0; round < 3; round++) {
+        std::vector<std::unique_ptr<StageLease>> at;
+        for (int k = 0; k < 8; k++) {
+            at.push_back(std::make_unique<StageLease>(1, nullptr, pool));
+            check(at.back()->take() == hipSuccess && (*at.back())->ensure(100000) == hipSuccess, "a stage");
+        }
+    }
+    check(pins == 16, "eight stages, and the memory of each pinned once");
+    check(pool.idleCount() == 8, "one stays for each context");
+    for (int k = 0; k < 8; k++) pool.contexts(1, -1);
+    check(pool.idleCount() == StagePool::kIdle && frees == 12, "what the contexts leave is given back");
+}
+
 // Host threads' time while the GPU works for 400 ms before the first chunk is there.
 static void wait() {
     StagePool pool;
@@ -159,6 +176,7 @@ int main(int, char** argv) {
     if (mode == "pool") pool();
     if (mode == "copy") copy();
     if (mode == "wait") wait();
+    if (mode == "contexts") contexts();
     printf("bad=%d\n", bad);
     return bad != 0;
 }

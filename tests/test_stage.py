@@ -84,3 +84,8 @@ def test_contexts_in_several_threads():
 @pytest.mark.skipif(shutil.which("g++") is None or not HIP.exists(), reason="needs g++ and the HIP headers")
 def test_helpers_sleep_while_the_gpu_works(tmp_path):
     test_stages_on_the_host(tmp_path, "wait")
+
+
+@pytest.mark.skipif(shutil.which("g++") is None or not HIP.exists(), reason="needs g++ and the HIP headers")
+def test_a_stage_for_each_context(tmp_path):
+    test_stages_on_the_host(tmp_path, "contexts")

@@ -201,6 +201,7 @@ int el_create(el_ctx** out, int device) {
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return EL_ERR_HIP;
     if (c->dCounters.ensure(sizeof(unsigned long long) * kCounterWords) != hipSuccess) return EL_ERR_HIP;
     if (scratchAddress(device, &c->scratch) != hipSuccess) return EL_ERR_HIP;
+    stagePool().contexts(device, 1);
     *out = c.release();
     return EL_OK;
 }
@@ -211,6 +212,7 @@ void el_destroy(el_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (auto e : c->evPool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    stagePool().contexts(c->device, -1);
     delete c;
 }
 

@@ -65,9 +65,10 @@ struct Stage {
 // time take 0.3 to 0.8 ms, which a stage for each context put into every
 // context's first call (1000 rays on a new context took 556 us, 200 by
 // pageable copies, and take 115 with a pooled stage; the first adjoint of a 128 x
-// 128 frame with 256 x 256 texels 1822, 1610 and 1074).  At most kIdle stages a device
-// (of 8 MiB, the largest) stay pinned for the next call, until the process ends;
-// the others are given back at once.
+// 128 frame with 256 x 256 texels 1822, 1610 and 1074).  As many stages of a
+// device (of 8 MiB at most, the largest) stay pinned for the next call as it
+// has contexts, so that a thread for each finds one, and kIdle where there are
+// fewer, until the process ends; the others are given back at once.
 class StagePool {
 public:
     static constexpr size_t kIdle = 2;
@@ -89,21 +90,22 @@ public:
         return std::unique_ptr<Stage>(new (std::nothrow) Stage());
     }
     void give(int device, std::unique_ptr<Stage> s) noexcept {
-        std::unique_ptr<Stage> surplus;   // freed after the lock
+        std::vector<std::unique_ptr<Stage>> surplus;   // freed after the lock
         std::lock_guard<std::mutex> lock(mu);
-        size_t held = 0, least = idle.size();
-        for (size_t i = 0; i < idle.size(); i++) {
-            if (idle[i].first != device) continue;
-            held++;
-            if (least == idle.size() || idle[i].second->bytes() < idle[least].second->bytes()) least = i;
-        }
-        if (held >= kIdle) {
-            if (idle[least].second->bytes() < s->bytes()) std::swap(idle[least].second, s);
-            surplus = std::move(s);
-            return;
-        }
         try {
             idle.emplace_back(device, std::move(s));
+            trim(device, surplus);
+        } catch (...) {
+        }
+    }
+    // A context of the device was made (1) or is gone (-1).
+    void contexts(int device, int change) noexcept {
+        std::vector<std::unique_ptr<Stage>> surplus;
+        std::lock_guard<std::mutex> lock(mu);
+        try {
+            if (users.size() <= (size_t)device) users.resize(device + 1, 0);
+            users[device] += change;
+            trim(device, surplus);
         } catch (...) {
         }
     }
@@ -113,8 +115,25 @@ public:
     }
 
 private:
+    // Moves the smallest of the device's idle stages to `surplus` until it has no more than it may.
+    void trim(int device, std::vector<std::unique_ptr<Stage>>& surplus) {
+        const size_t most = std::max(kIdle, (size_t)device < users.size() ? (size_t)std::max(0, users[device]) : 0);
+        for (;;) {
+            size_t held = 0, least = idle.size();
+            for (size_t i = 0; i < idle.size(); i++) {
+                if (idle[i].first != device) continue;
+                held++;
+                if (least == idle.size() || idle[i].second->bytes() < idle[least].second->bytes()) least = i;
+            }
+            if (held <= most) return;
+            surplus.push_back(std::move(idle[least].second));
+            idle[least] = std::move(idle.back());
+            idle.pop_back();
+        }
+    }
     std::mutex mu;
     std::vector<std::pair<int, std::unique_ptr<Stage>>> idle;
+    std::vector<int> users;   // contexts by device
 };
 
 // The process's pool, made by the first call that takes a stage (the runtime
