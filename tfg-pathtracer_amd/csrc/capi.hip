@@ -301,23 +301,23 @@ static void setMaterialValues(dev::DevMaterial& d, const el_material& m) {
 static int uploadBvh(el_ctx* c, int width) {
     try {
         c->wide = collapseWide(c->bvh2, c->verts.data(), (int)c->ntri, width);
+        if (width == 4)   // the nodes as the device reads them, in the place of the others
+            parallelFor(c->wide.nodeCount, [&](size_t i0, size_t i1) {
+                for (size_t i = i0; i < i1; i++) {
+                    unsigned char* const at = c->wide.nodes.data() + i * sizeof(QNode<4>);
+                    QNode<4> n;
+                    uint32_t words[16];
+                    static_assert(sizeof words == sizeof n, "a node keeps its size");
+                    std::memcpy(&n, at, sizeof n);
+                    packLaneNode(n, words);
+                    std::memcpy(at, words, sizeof words);
+                }
+            });
     } catch (const std::exception& ex) {
         return fail(c, EL_ERR_RANGE, ex.what());
     }
     c->width = width;
-    std::vector<uint32_t> lanes;   // the BVH4 nodes as the quads read them
-    if (width == 4) {
-        lanes.resize(c->wide.nodeCount * 16);
-        parallelFor(c->wide.nodeCount, [&](size_t i0, size_t i1) {
-            for (size_t i = i0; i < i1; i++) {
-                QNode<4> n;
-                std::memcpy(&n, c->wide.nodes.data() + i * sizeof n, sizeof n);
-                packLaneNode(n, &lanes[i * 16]);
-            }
-        });
-    }
-    const void* nodes = width == 4 ? (const void*)lanes.data() : (const void*)c->wide.nodes.data();
-    EL_HIP(c, upload(c->dNodes, nodes, c->wide.nodes.size(), c->stream));
+    EL_HIP(c, upload(c->dNodes, c->wide.nodes.data(), c->wide.nodes.size(), c->stream));
     EL_HIP(c, upload(c->dTris, c->wide.triStream.data(), c->wide.triStream.size() * sizeof(float), c->stream));
     c->gcap = dev::spillRows(c->wide.stackBound);
     EL_HIP(c, c->dGstack.ensure((size_t)c->gcap * c->maxThreads * sizeof(int)));
