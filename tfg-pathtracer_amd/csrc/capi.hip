@@ -865,6 +865,9 @@ extern "C" int el_residual_l2(el_ctx* c, const float* target, double* loss) {
     return EL_OK;
 }
 
+// Bytes of an output of el_adjoint up to which it is copied with the tallies.
+constexpr size_t kOneWait = 1u << 20;
+
 extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* dimage, float* dmat, float* dtex,
                           int devp) {
     const bool accumulate = (p && (p->flags & EL_ADJ_ACCUMULATE) != 0);
@@ -986,12 +989,36 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
         }
     }
     EL_HIP(c, hipEventRecord(e1, c->stream));
-    std::vector<double> hm(M * 6);
-    EL_HIP(c, hipMemcpyAsync(hm.data(), c->aMat.p, M * 6 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     const unsigned long long* const h = stage->tallies;
+    // The material sums and the texels come with the tallies, in one wait, up to
+    // kOneWait each: a copy to pageable memory is a wait of its own, and so is a
+    // chunk of stageOut, which takes larger textures once the GPU is done.
+    const size_t matBytes = dmat ? M * 6 * sizeof(double) : 0, texBytes = ntex && dtex && !devp ? ntex * sizeof(float) : 0;
+    const size_t matStaged = matBytes <= kOneWait ? matBytes : 0, texStaged = texBytes <= kOneWait ? texBytes : 0;
     if (ntex && dtex && devp)
         EL_HIP(c, hipMemcpyAsync(dtex, c->aTex.p, ntex * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-    if (ntex && dtex && !devp)
+    std::vector<double> large(matBytes > matStaged ? M * 6 : 0);
+    if (!large.empty()) EL_HIP(c, hipMemcpyAsync(large.data(), c->aMat.p, matBytes, hipMemcpyDeviceToHost, c->stream));
+    if (matStaged + texStaged) {
+        EL_HIP(c, stage->ensure(matStaged + texStaged));
+        stage.inFlight(true);
+    }
+    if (matStaged) EL_HIP(c, hipMemcpyAsync(stage->p, c->aMat.p, matStaged, hipMemcpyDeviceToHost, c->stream));
+    if (texStaged) EL_HIP(c, hipMemcpyAsync(stage->p + matStaged, c->aTex.p, texStaged, hipMemcpyDeviceToHost, c->stream));
+    EL_HIP(c, readTallies(stage, ctr));
+    float ms = 0;
+    EL_HIP(c, hipEventElapsedTime(&ms, e0, e1));
+    if (dmat) {
+        const double* const hm = matStaged ? (const double*)stage->p : large.data();
+        std::vector<float> fm(M * 6);
+        for (size_t i = 0; i < M * 6; i++) fm[i] = (float)hm[i];
+        if (devp)
+            EL_HIP(c, hipMemcpy(dmat, fm.data(), fm.size() * sizeof(float), hipMemcpyHostToDevice));
+        else
+            std::memcpy(dmat, fm.data(), fm.size() * sizeof(float));
+    }
+    if (texStaged) std::memcpy(dtex, stage->p + matStaged, texStaged);
+    if (texBytes > texStaged)
         EL_HIP(c, stageOut(
                       stage, ntex, sizeof(float),
                       [&](size_t first, size_t n, unsigned char* chunk) {
@@ -1001,17 +1028,6 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
                       [&](size_t first, size_t, const unsigned char* chunk, size_t i0, size_t i1) {
                           std::memcpy(dtex + first + i0, (const float*)chunk + i0, (i1 - i0) * sizeof(float));
                       }));
-    EL_HIP(c, readTallies(stage, ctr));
-    float ms = 0;
-    EL_HIP(c, hipEventElapsedTime(&ms, e0, e1));
-    std::vector<float> fm(M * 6);
-    for (size_t i = 0; i < M * 6; i++) fm[i] = (float)hm[i];
-    if (dmat) {
-        if (devp)
-            EL_HIP(c, hipMemcpy(dmat, fm.data(), fm.size() * sizeof(float), hipMemcpyHostToDevice));
-        else
-            std::memcpy(dmat, fm.data(), fm.size() * sizeof(float));
-    }
     c->adjSumValid = true;
     c->adjSumTex = gtex;
     c->stats.adjoint_ms = ms;
