@@ -1586,7 +1586,9 @@ hipError_t launchPlain(const LaunchCfg& c, const DevScene& s, const RenderArgs& 
 hipError_t launchAdjBounce(const LaunchCfg& c, const DevScene& s, const RenderArgs& a, const WfState& q,
                            const AdjArgs& g, const float4* rayIn, const float4* stateIn, float4* rayOut,
                            float4* stateOut, unsigned long long* counters) {
-    const uint32_t grid = gridFor(a.genCount, c.shadeBlock, c.maxThreads / c.shadeBlock);
+    // no more blocks than are resident (EL_WPE_ADJ waves of 8 a SIMD): each clears the material sums at its start and adds
+    // them up at its end, of up to kAdjLdsMats materials
+    const uint32_t grid = gridFor(a.genCount, c.shadeBlock, c.maxThreads / 8 * EL_WPE_ADJ / c.shadeBlock);
     const size_t lds = 6 * sizeof(double) * g.ldsMats;
     if (a.bounce == 0)
         hipLaunchKernelGGL(k_adj_bounce<true>, dim3(grid), dim3(c.shadeBlock), lds, c.stream, s, a, q, g, rayIn,
