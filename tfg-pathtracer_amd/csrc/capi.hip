@@ -1003,8 +1003,8 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
         EL_HIP(c, stage->ensure(matStaged + texStaged));
         stage.inFlight(true);
     }
-    if (matStaged) EL_HIP(c, hipMemcpyAsync(stage->p, c->aMat.p, matStaged, hipMemcpyDeviceToHost, c->stream));
-    if (texStaged) EL_HIP(c, hipMemcpyAsync(stage->p + matStaged, c->aTex.p, texStaged, hipMemcpyDeviceToHost, c->stream));
+    if (matStaged) EL_HIP(c, launchCopyOut(c->stream, c->aMat.p, stage->p, matStaged / 4));
+    if (texStaged) EL_HIP(c, launchCopyOut(c->stream, c->aTex.p, stage->p + matStaged, texStaged / 4));
     EL_HIP(c, readTallies(stage, ctr));
     float ms = 0;
     EL_HIP(c, hipEventElapsedTime(&ms, e0, e1));
@@ -1022,8 +1022,7 @@ extern "C" int el_adjoint(el_ctx* c, const el_adjoint_params* p, const float* di
         EL_HIP(c, stageOut(
                       stage, ntex, sizeof(float),
                       [&](size_t first, size_t n, unsigned char* chunk) {
-                          return hipMemcpyAsync(chunk, c->aTex.as<float>() + first, n * sizeof(float),
-                                                hipMemcpyDeviceToHost, c->stream);
+                          return launchCopyOut(c->stream, c->aTex.as<float>() + first, chunk, n);
                       },
                       [&](size_t first, size_t, const unsigned char* chunk, size_t i0, size_t i1) {
                           std::memcpy(dtex + first + i0, (const float*)chunk + i0, (i1 - i0) * sizeof(float));

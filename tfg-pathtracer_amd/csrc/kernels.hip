@@ -1524,6 +1524,15 @@ __global__ void __launch_bounds__(256) k_resolve(const float4* __restrict__ sums
     }
 }
 
+// n 32-bit words to mapped host memory, both 16-byte aligned.  By stores of a
+// kernel, not by a copy engine: the runtime makes an engine's queue when it
+// first takes that engine, in 5 to 6 ms of some call's copy.
+__global__ void __launch_bounds__(256) k_copy_out(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, uint64_t n) {
+    const uint64_t quads = n >> 2, step = (uint64_t)gridDim.x * blockDim.x, i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint64_t i = i0; i < quads; i += step) ((uint4*)dst)[i] = ((const uint4*)src)[i];
+    for (uint64_t i = 4 * quads + i0; i < n; i += step) dst[i] = src[i];
+}
+
 }  // namespace dev
 
 // ------------------------------------------------------------ host launch --
@@ -1603,6 +1612,13 @@ hipError_t launchResolve(hipStream_t stream, const float4* sums, uint32_t stride
                          uint32_t first, uint32_t n, float4* rgba, uint32_t* samples) {
     hipLaunchKernelGGL(k_resolve, dim3(gridFor(n, 256, 2048)), dim3(256), 0, stream, sums, stride, counts, first, n,
                        rgba, samples);
+    return hipGetLastError();
+}
+
+hipError_t launchCopyOut(hipStream_t stream, const void* src, void* dst, uint64_t words) {
+    if (((uintptr_t)src | (uintptr_t)dst) & 15) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_copy_out, dim3(gridFor(words / 4 + 1, 256, 1024)), dim3(256), 0, stream, (const uint32_t*)src,
+                       (uint32_t*)dst, words);
     return hipGetLastError();
 }
 

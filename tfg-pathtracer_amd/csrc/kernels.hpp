@@ -154,6 +154,8 @@ hipError_t launchPlain(const LaunchCfg& c, const dev::DevScene& s, const RenderA
 // memory; either may be null).
 hipError_t launchResolve(hipStream_t stream, const float4* sums, uint32_t stride, const uint32_t* counts,
                          uint32_t first, uint32_t n, float4* rgba, uint32_t* samples);
+// `words` 32-bit words of device memory to mapped host memory (both 16-byte aligned).
+hipError_t launchCopyOut(hipStream_t stream, const void* src, void* dst, uint64_t words);
 // r = 2 (mean image - target) per pixel and channel (FP64 arithmetic, FP32
 // store); *loss += sum (mean image - target)^2 (the caller zeroes it).
 hipError_t launchResidualL2(hipStream_t stream, const float4* accum, const uint32_t* counts, const float* target,
