@@ -42,19 +42,21 @@ struct Stage {
         if (tallies) return hipSuccess;
         return hipHostMalloc((void**)&tallies, sizeof(unsigned long long) * kTallyWords, hipHostMallocDefault);
     }
+    // Memory for an output of `bytes`, taken chunk by chunk: one chunk, or two.
+    // Whole chunks at once: pinning takes as long for 64 KB (0.05 to 0.4 ms), pages
+    // cost when they are touched, and a larger output finds it pinned.
     hipError_t ensure(size_t bytes) {
-        const size_t want = std::min(kChunk, std::max<size_t>(64u << 10, bytes));
         const bool both = bytes > kChunk;
         for (auto& e : filled)
             if (!e)
                 if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming); r != hipSuccess) return r;
-        if (p && want <= n && both <= two) return hipSuccess;
+        if (p && both <= two) return hipSuccess;
         if (p) (void)hipHostFree(p);
         p = nullptr;
         n = 0;
-        const hipError_t r = hipHostMalloc((void**)&p, want * (both ? 2 : 1), hipHostMallocDefault);
+        const hipError_t r = hipHostMalloc((void**)&p, kChunk * (both ? 2 : 1), hipHostMallocDefault);
         if (r != hipSuccess) return r;
-        n = want;
+        n = kChunk;
         two = both;
         return hipSuccess;
     }
