@@ -8,9 +8,15 @@
  *
  * Threading: one el_ctx per host thread; a context owns one HIP stream on
  * one device.  No host thread it starts outlives a call: el_upload_scene
- * builds on up to the hardware's thread count, capped by OMP_NUM_THREADS
- * when that is set.  Calls are synchronous on return unless stated
- * otherwise.
+ * builds on up to the hardware's thread count, and calls that return more than
+ * 2 MB to host memory (el_read_passes, el_read_aov, el_batch_read, el_adjoint,
+ * el_trace_closest, el_trace_any) copy on up to 8 threads, a thread a MB, both
+ * capped by OMP_NUM_THREADS when that is set.  Calls are synchronous on return
+ * unless stated otherwise.
+ *
+ * Host memory: such calls go through pinned memory of the process, at most
+ * 8 MiB for each context of a device (for two where there are fewer), which
+ * stays pinned for the next call until its context or the process ends.
  *
  * Reference interfaces replaced (paths relative to src/tfg-pathtracer/):
  *   renderSetup(Scene*)                       kernel.h:80,  kernel.cu:566-661
@@ -171,8 +177,10 @@ typedef struct {
                                   likewise)                                  */
     double   shadow_ms;        /* summed shadow kernel time (wavefront)      */
     double   shade_ms;         /* summed shading kernel time (wavefront)     */
-    uint64_t extend_launches;  /* number of closest-hit launches timed       */
-    uint64_t extend_rays;      /* rays processed by those launches           */
+    uint64_t extend_launches;  /* closest-hit queues traced (bounces x
+                                  generations; a launch each, and timed, with
+                                  EL_FLAG_KERNEL_TIMES)                      */
+    uint64_t extend_rays;      /* rays of those queues                       */
     uint64_t node_fetches;     /* closest-hit node fetches (COUNT_TRAVERSAL) */
     uint64_t tri_tests;        /* closest-hit triangle tests (COUNT_TRAVERSAL) */
     uint64_t node_bytes;       /* size of the device BVH node array          */
@@ -276,11 +284,11 @@ int  el_set_camera(el_ctx* ctx, const el_camera* camera);
  * number at a time; a material whose albedo comes from a texture gets no
  * albedo gradient (its texels do, if selected).  Without a recording render
  * the paths of a generation are traced again first, which needs at most
- * 2 GiB whatever the pixel and sample counts; the vertices that a wavefront
+ * 2 GiB whatever the pixel and sample counts, and no more than a quarter of the
+ * free memory unless even 65,536 paths need that; the vertices that a wavefront
  * EL_FLAG_RECORD_PATHS render kept are replayed without tracing.  A context
  * whose wavefront queues are larger already (they are shared) allocates only
- * the rest.  With `device_ptrs` != 0 the three
- * arrays are device pointers.  d_materials and d_texture may be NULL:
+ * the rest.  With `device_ptrs` != 0 the three arrays are device pointers.  d_materials and d_texture may be NULL:
  * nothing is copied out, and the sums stay in the context for following
  * EL_ADJ_ACCUMULATE calls. */
 int  el_adjoint(el_ctx* ctx, const el_adjoint_params* params, const float* d_image,
@@ -309,12 +317,13 @@ int  el_trace_closest(el_ctx* ctx, const el_ray* rays, uint32_t n,
  * allocate device memory (tight serving loops, harnesses that forbid
  * hipMalloc).  The traversal's scratch -- its tallies and the per-thread
  * spill area of its stack -- is a static device array of the library,
- * 16 MiB + 512 B on each GPU the library runs on, held until the process
+ * 16 MiB + 4.5 KiB on each GPU the library runs on, held until the process
  * ends; the call allocates nothing, waits for its stream before returning
  * (so it cannot be captured into a graph), and its results equal
  * el_trace_closest's with device_ptrs = 1 (uv may be NULL).  The array
  * bounds the resident threads to 16 MiB / (4 B x the scene's spill slots per
- * thread), so large scenes trace with fewer threads than el_trace_closest.
+ * thread) for more than 393,216 rays (fewer go by quads of lanes, which spill
+ * nothing), so large scenes trace them with fewer threads than el_trace_closest.
  * Every call on one GPU shares that array: calls that overlap on one GPU
  * (two contexts on two host threads) race.  Fails with EL_ERR_RANGE when the
  * scene's stack needs more spill slots per thread than the array holds for

@@ -1110,11 +1110,12 @@ __device__ __forceinline__ uint32_t lanesBelow(unsigned long long m) {
 // registers).  A new ray starts at the root like any other visit: a visit of
 // its own at the refill would run with only the lanes refilled (a 1080p frame of 64
 // samples over 1,048,576 triangles 86.3 instead of 84.6 ms, 2 M closest hits 220 instead of 213 us).  The
-// lane's state has to fit 64 registers, what is the same for a wave is kept
+// lane's state should fit 64 registers, what is the same for a wave is kept
 // once (the count of rays, the spill area's address, the count of dropped
-// entries in memory) and a queue's entry is looked up once a ray: without the
-// 10 to 27 registers that were spilled before, a batch of 12 scenes takes 10.65
-// instead of 11.1 ms, 2 M closest hits 205 instead of 210 us.  The
+// entries in memory) and a queue's entry is looked up once a ray: with 0 to 5
+// registers spilled in launches over one BVH and 6 to 19 in batches, 10 to 27
+// before, a batch of 12 scenes takes 10.65 instead of 11.1 ms, 2 M closest hits
+// 205 instead of 210 us.  The
 // closest hit is order-independent (t, then lower index), so results are
 // identical to traceRay.
 //
